@@ -32,14 +32,16 @@ VALU_PEAK_TOPS = 256 * 4 * 16 * 2.4e9 / 1e12  # lane-ops/s: 256 CU x 4 SIMD x 16
 B_RAY, B_OUT, B_BOX, B_REF, B_TRI = 24, 8, 28, 4, 36
 OPS_RAY, OPS_BOX, OPS_TRI = 6, 24, 155
 # Work of the kernel's traversal per ray (counted by dr_cast_stats on the same rays): a group
-# expansion reads 196 B (8 child boxes + the non-empty mask) and pops read 8 B (link, count); a leaf
-# reads its 24-B box; a plane test reads the 4-B record index of the leaf entry and 32 B of the
-# record, an inside test 32 B more.
-# ops: 6 (1/d) + 12 per octant test (the children of an expanded group with a non-empty leaf below)
-#      + 24 per slab test (those not behind the origin) + 25 per plane test
+# expansion reads 80 B (grid, head and 8 child boxes) and a leaf pop 8 B (its first entry and the
+# next leaf's); a leaf whose hit is tested for acceptance reads a 32-B node record (counted for
+# every leaf); a plane test reads the 4-B record index of the leaf entry and 32 B of the record,
+# an inside test 32 B more.
+# ops: 30 per ray (3 reciprocals, 3 slacks, the root's box) + 27 per group (grid planes and their
+#      near / far order) + 17 per box test (the children of an expanded group with a non-empty
+#      leaf below: 6 conversions, 6 fused products, 5 to combine) + 25 per plane test
 #      + 140 per inside test (6 edge vectors, 3 dots, 3 square roots, 3 divisions).
-K_RAY, K_OUT, K_GROUP, K_POP, K_LEAF, K_PLANE, K_INSIDE = 24, 8, 196, 8, 24, 36, 32
-KOPS_RAY, KOPS_OCTANT, KOPS_SLAB, KOPS_PLANE, KOPS_INSIDE = 6, 12, 24, 25, 140
+K_RAY, K_OUT, K_GROUP, K_POP, K_LEAF, K_PLANE, K_INSIDE = 24, 8, 80, 8, 32, 36, 32
+KOPS_RAY, KOPS_GROUP, KOPS_CHILD, KOPS_PLANE, KOPS_INSIDE = 30, 27, 17, 25, 140
 
 
 # host threads of the CPU legs: the cores this process may run on (the lease's share of the host)
@@ -170,16 +172,14 @@ def _device_scene(D, tris, split=16, depth=12):
 
 def render_roofline(cnt, ms, pixels):
     """Roofline of a render from the work its kernel counted (dr_render_stats): the traversal
-    lane-ops of every cast (as for the cast kernel, plus 6 ops of ray setup per cast) against
-    the VALU peak, and the bytes those casts read (groups, leaf boxes and links, 32-B halves of
+    lane-ops of every cast (as for the cast kernel) against the VALU peak, and the bytes those casts read (groups, leaf boxes and links, 32-B halves of
     triangle records; leaf-ordered records, so no record index) plus the 16-B framebuffer store
     of every pixel, against HBM.  Shading arithmetic (BSDF sampling, light sampling, Philox) is
     not counted, so the VALU fraction understates the kernel's instruction use."""
     seg, ge, lv, pl, ins = (cnt[k] for k in ("segments", "group_expansions", "leaves", "plane_tests", "inside_tests"))
-    ops = (KOPS_RAY * seg + KOPS_OCTANT * cnt["live_children"] + KOPS_SLAB * cnt["slab_tests"] + KOPS_PLANE * pl
+    ops = (KOPS_RAY * seg + KOPS_GROUP * ge + KOPS_CHILD * cnt["live_children"] + KOPS_PLANE * pl
            + KOPS_INSIDE * ins)
-    pops = max(ge - seg, 0) + lv
-    byts = K_GROUP * ge + K_POP * pops + K_LEAF * lv + (K_PLANE - 4) * pl + K_INSIDE * ins + 16 * pixels
+    byts = K_GROUP * ge + (K_POP + K_LEAF) * lv + (K_PLANE - 4) * pl + K_INSIDE * ins + 16 * pixels
     t = ms / 1e3
     return {"bound": "valu", "achieved": round(ops / t / 1e12, 3), "peak": round(VALU_PEAK_TOPS, 2),
             "unit": "T lane-ops/s", "frac": round(ops / t / 1e12 / VALU_PEAK_TOPS, 4),
@@ -498,9 +498,9 @@ def main():
     ge, lv, pl, ins, live, slab = (float(x) for x in cnt)
     kernel_work = {"group_expansions": ge, "leaves": lv, "plane_tests": pl, "inside_tests": ins,
                    "live_children": live, "slab_tests": slab,
-                   "bytes": K_RAY + K_OUT + K_GROUP * ge + K_POP * (ge - 1 + lv) + K_LEAF * lv + K_PLANE * pl
+                   "bytes": K_RAY + K_OUT + K_GROUP * ge + (K_POP + K_LEAF) * lv + K_PLANE * pl
                    + K_INSIDE * ins,
-                   "ops": KOPS_RAY + KOPS_OCTANT * live + KOPS_SLAB * slab + KOPS_PLANE * pl + KOPS_INSIDE * ins}
+                   "ops": KOPS_RAY + KOPS_GROUP * ge + KOPS_CHILD * live + KOPS_PLANE * pl + KOPS_INSIDE * ins}
     log(f"kernel work per ray: {kernel_work}")
     kA_ms, wallA, outA = timed(rA, args.steps)
     log(f"batch A: {kA_ms:.3f} ms/launch ({len(coherent) / kA_ms / 1e3:.1f} Mrays/s)")

@@ -69,6 +69,7 @@ void scene_retain(dr_scene s) { s->refs.fetch_add(1); }
 void scene_release(dr_scene s) {
   if (s->refs.fetch_sub(1) != 1) return;
   dev_free(s->groups);
+  dev_free(s->nodes);
   dev_free(s->recs);
   dev_free(s->urecs);
   dev_free(s->lref);
@@ -190,6 +191,7 @@ int dr_scene_create(dr_octree t, dr_scene *out) {
   if (!s) return dr::fail(DR_ERR_ALLOC, "dr_scene_create: out of host memory");
   (void)hipGetDevice(&s->device);
   int rc = dr::dev_upload(s->groups, flat.groups.data(), flat.groups.size() * sizeof(float));
+  if (rc == DR_OK) rc = dr::dev_upload(s->nodes, flat.nodes.data(), flat.nodes.size() * sizeof(float));
   if (rc == DR_OK) rc = dr::dev_upload(s->recs, flat.recs.data(), flat.recs.size() * sizeof(float));
   if (rc == DR_OK) rc = dr::dev_upload(s->urecs, flat.urecs.data(), flat.urecs.size() * sizeof(float));
   if (rc == DR_OK) rc = dr::dev_upload(s->lref, flat.lref.data(), flat.lref.size() * sizeof(int32_t));
@@ -202,6 +204,7 @@ int dr_scene_create(dr_octree t, dr_scene *out) {
   if (rc != DR_OK) { dr_scene_destroy(s); return rc; }
   dr::DevTree &T = s->tree;
   T.groups = (const float4 *)s->groups.p;
+  T.nodes = (const float4 *)s->nodes.p;
   T.recs = (const float4 *)s->recs.p;
   T.urecs = (const float4 *)s->urecs.p;
   T.lref = (const int *)s->lref.p;
@@ -210,7 +213,7 @@ int dr_scene_create(dr_octree t, dr_scene *out) {
   T.root_is_leaf = flat.root_is_leaf;
   T.root_start = flat.root_start;
   T.root_count = flat.root_count;
-  T.margin = flat.prune_margin;
+  T.reach = flat.reach;
   s->max_depth = flat.max_depth;
   s->ntris = (int)t->host.tris.size();
   s->shade_host.resize(s->ntris);

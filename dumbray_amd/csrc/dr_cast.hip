@@ -163,7 +163,7 @@ __global__ __launch_bounds__(kCastBlock, 4) void k_cast(DevTree T, const float *
           r = slot;
           const float2 *R = (const float2 *)(rays + 6 * (size_t)r);
           const float2 q0 = R[0], q1 = R[1], q2 = R[2];
-          walk_begin(T, w, v3(q0.x, q0.y, q1.x), v3(q1.y, q2.x, q2.y), exclude ? exclude[r] : -1, stk, S, cc);
+          walk_begin(T, w, v3(q0.x, q0.y, q1.x), v3(q1.y, q2.x, q2.y), exclude ? exclude[r] : -1);
           if (w.state == kWalkDone) finish();
         } else {
           exhausted = true;

@@ -40,7 +40,7 @@ struct dr_scene_s {
   // batch request; the scene's memory is freed with the last one
   std::atomic<int> refs{1};
   int device = 0;
-  dr::DevBuf groups, recs, urecs, lref, shade;
+  dr::DevBuf groups, nodes, recs, urecs, lref, shade;
   dr::DevBuf faces;                        // per triangle: vertices a, b, c, then their normals (18 floats)
   std::vector<float> faces_host;
   dr::DevTree tree;
@@ -64,7 +64,7 @@ struct dr_scene_s {
   };
   std::mutex scratch_mu;
   std::vector<StreamScratch> scratch;
-  int64_t bytes() const { return (int64_t)(groups.bytes + recs.bytes + urecs.bytes + lref.bytes + shade.bytes + faces.bytes + work.bytes); }
+  int64_t bytes() const { return (int64_t)(groups.bytes + nodes.bytes + recs.bytes + urecs.bytes + lref.bytes + shade.bytes + faces.bytes + work.bytes); }
 };
 
 // One renderer's shading tables of a scene (dr_shading_create).

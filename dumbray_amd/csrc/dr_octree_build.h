@@ -22,26 +22,28 @@ struct OctreeHost {
 int build_octree(const float *tris9, int ntris, int split_threshold, int max_depth, int nthreads, OctreeHost &out);
 
 // ---------------------------------------------------------------- device layout
-// A "group" is the 8 contiguous children of one interior node, stored as 72
-// 32-bit words (288 B):
-//   [0..47]  reference boxes: min.x[8] min.y[8] min.z[8] max.x[8] max.y[8] max.z[8]
-//   [48]     bits 0-7: child k has a non-empty leaf at or below it;
-//            bits 8-15: child k is interior
-//   [49]     group of the first interior child.  Interior children get consecutive
-//            groups (breadth-first order), so interior child k's group is this
-//            plus the number of interior children before k.
-//   [50..55] unused
-//   [56..63] link: interior -> child group index; leaf -> first triangle record
-//   [64..71] count: -1 interior, 0 empty leaf (or only degenerate triangles), >0 records
+// A "group" is the 8 contiguous children of one interior node: 32 words, one 128-B line.
+//   [0..2]   origin of the group's grid          [3]  head (below)
+//   [4..6]   cell size of the grid per axis      [7]  group of the first interior child
+//   [8..19]  child boxes in grid cells, one byte each: min.x[8] min.y[8] min.z[8] max.x[8]
+//            max.y[8] max.z[8]
+//   [20..28] first leaf entry of child k, and the end of child 7's (child k holds the entries
+//            [20 + k] .. [21 + k]; none if it is interior or empty)
+//   head: bits 0-7: child k has a non-empty leaf at or below it; bits 8-15: child k is interior
+// Interior children get consecutive groups (breadth-first order), so interior child k's group is
+// word 7 plus the number of interior children before k.
 // Child k uses the reference's numbering (bit0 = z-high, bit1 = y-high, bit2 = x-high).
-// Traversal drops a child whose box, widened by the tree's prune margin, lies
-// outside the ray's forward octant: a leaf accepts a hit only if the hit point
-// o + d*t (t >= 0) is inside its box, that point never leaves the closed octant
-// of o that d points into, and every non-empty leaf box lies inside each of its
-// ancestors' boxes widened by the margin (computed exactly when flattening).
-constexpr int kGroupWords = 72;
+// A child's grid box holds every non-empty leaf box at or below it (rounded outwards, checked in
+// double when flattening), so it decides only which subtrees can be skipped.  The reference's own
+// decisions, the slab tests of the leaf and of its ancestors, are taken from the node records
+// when a hit is about to be accepted.
+constexpr int kGroupWords = 32;
 constexpr int kGroupF4 = kGroupWords / 4;
-constexpr int kGroupMask = 48, kGroupBase = 49, kGroupLink = 56, kGroupCount = 64;
+constexpr int kGroupHead = 3, kGroupBase = 7, kGroupBoxes = 8, kGroupEntry = 20;
+// A node record, 8 words: min.x min.y min.z max.x | max.y max.z parent nested.  Node 8 * g + k is
+// child k of group g; parent is the parent's node, -1 under the root; nested is 1 if the box lies
+// inside the box of every ancestor, the root included.
+constexpr int kNodeWords = 8, kNodeF4 = kNodeWords / 4;
 // A triangle record is 16 words (64 B):
 //   a.x a.y a.z n.x | n.y n.z b.x b.y | b.z c.x c.y c.z | thr0 thr1 thr2 id
 // n = (b-a) x (c-a) and thr* = the ray-independent right-hand sides of the
@@ -54,6 +56,7 @@ constexpr int kRecWords = 16;
 
 struct OctreeFlat {
   std::vector<float> groups;               // ngroups * kGroupWords words (ints stored bitwise)
+  std::vector<float> nodes;                // 8 * ngroups * kNodeWords words
   std::vector<float> recs;                 // nrec * 16 words, one per leaf entry (leaf order)
   std::vector<float> urecs;                // the same records once per distinct triangle
   std::vector<int32_t> lref;               // leaf entry -> its record in urecs
@@ -61,7 +64,7 @@ struct OctreeFlat {
   int root_is_leaf = 0, root_start = 0, root_count = 0;
   int ngroups = 0, nrec = 0;
   int max_depth = 0;                       // depth of the deepest node (root: 0), not the build limit
-  float prune_margin = 0.0f;               // see the group layout above
+  float reach = 0.0f;                      // largest magnitude of a box coordinate, inf if one is not finite
 };
 int flatten_octree(const OctreeHost &t, OctreeFlat &out);
 

@@ -503,6 +503,40 @@ static void put_rec(std::vector<float> &recs, const Tri &t, int32_t id) {
   recs.insert(recs.end(), w, w + kRecWords);
 }
 
+// The grid and the child boxes of a group: box[k] for the children in `mask`, an inverted box for
+// the others.  A cell size and every cell are rounded so that the grid box holds the child's.
+static void quantize_group(const Box *box, uint32_t mask, float *G) {
+  unsigned char *cells = (unsigned char *)(G + kGroupBoxes);
+  for (int axis = 0; axis < 3; axis++) {
+    double lo = 0.0, hi = 0.0;
+    bool any = false;
+    for (int k = 0; k < 8; k++) {
+      if (!((mask >> k) & 1u)) continue;
+      const double s = axis_of(box[k].s, axis), e = axis_of(box[k].e, axis);
+      lo = any ? std::min(lo, s) : s;
+      hi = any ? std::max(hi, e) : e;
+      any = true;
+    }
+    float cell = (float)((hi - lo) / 255.0);
+    while (lo + 255.0 * (double)cell < hi) cell = std::nextafter(cell, __builtin_inff());
+    if (!std::isfinite(cell) || !std::isfinite(lo)) { lo = 0.0; cell = 0.0f; }   // see OctreeFlat::reach
+    G[axis] = (float)lo;                                   // lo is a box coordinate: exact
+    G[4 + axis] = cell;
+    for (int k = 0; k < 8; k++) {
+      int a = 255, b = 0;
+      if ((mask >> k) & 1u) {
+        const double s = axis_of(box[k].s, axis), e = axis_of(box[k].e, axis);
+        a = cell > 0.0f ? (int)std::floor(std::min(255.0, std::max(0.0, (s - lo) / (double)cell))) : 0;
+        b = cell > 0.0f ? (int)std::ceil(std::min(255.0, std::max(0.0, (e - lo) / (double)cell))) : 0;
+        while (a > 0 && lo + a * (double)cell > s) a--;
+        while (b < 255 && lo + b * (double)cell < e) b++;
+      }
+      cells[8 * axis + k] = (unsigned char)a;
+      cells[24 + 8 * axis + k] = (unsigned char)b;
+    }
+  }
+}
+
 int flatten_octree(const OctreeHost &t, OctreeFlat &out) {
   out = OctreeFlat();
   const int nn = (int)t.bounds.size();
@@ -567,47 +601,60 @@ int flatten_octree(const OctreeHost &t, OctreeFlat &out) {
     }
     slb[i] = b;
   }
-  // prune margin: how far any non-empty leaf box reaches beyond the box of any of its
-  // ancestors (evaluated in double), plus a guard of 4 ulps of the largest coordinate so
-  // that the fp32 sum box + margin is never below the leaf's face.
-  double poke = 0.0, maxabs = 0.0;
-  for (int i = 1; i < nn; i++) {
-    const Box &b = t.bounds[i], &l = slb[i];
-    if (!(l.s.x <= l.e.x)) continue;                   // no non-empty leaf below
-    const double d[6] = {(double)l.e.x - b.e.x, (double)l.e.y - b.e.y, (double)l.e.z - b.e.z,
-                         (double)b.s.x - l.s.x, (double)b.s.y - l.s.y, (double)b.s.z - l.s.z};
-    for (double v : d) poke = std::max(poke, v);
-    const double c[6] = {b.s.x, b.s.y, b.s.z, b.e.x, b.e.y, b.e.z};
-    for (double v : c) maxabs = std::max(maxabs, std::fabs(v));
+  // the part of a node's box that lies in all its ancestors' boxes too
+  std::vector<Box> common(nn);
+  std::vector<int32_t> parent(nn, -1);
+  common[0] = t.bounds[0];
+  float reach = 0.0f;
+  for (int i = 0; i < nn; i++) {
+    const Box &b = t.bounds[i];
+    for (float v : {b.s.x, b.s.y, b.s.z, b.e.x, b.e.y, b.e.z})
+      reach = std::isfinite(v) ? std::max(reach, std::fabs(v)) : __builtin_inff();
+    if (t.children[i] < 0) continue;
+    for (int c = t.children[i]; c < t.children[i] + 8; c++) {
+      const Box &q = t.bounds[c], &p = common[i];
+      parent[c] = i;
+      common[c].s = v3(std::max(q.s.x, p.s.x), std::max(q.s.y, p.s.y), std::max(q.s.z, p.s.z));
+      common[c].e = v3(std::min(q.e.x, p.e.x), std::min(q.e.y, p.e.y), std::min(q.e.z, p.e.z));
+    }
   }
-  out.prune_margin = (float)(poke + 4.0 * maxabs * 1.1920928955078125e-07 + 1e-30);
+  out.reach = reach;
+  out.nodes.assign((size_t)out.ngroups * 8 * kNodeWords, 0.0f);
   out.groups.assign((size_t)out.ngroups * kGroupWords, 0.0f);
   for (int g = 0; g < out.ngroups; g++) {
     float *G = &out.groups[(size_t)g * kGroupWords];
+    const int first = 1 + 8 * g;
     uint32_t nonempty = 0, interior = 0;
     int32_t first_child = 0;
     for (int k = 0; k < 8; k++) {
-      const int node = 1 + 8 * g + k;
-      const Box &b = t.bounds[node];
-      G[0 + k] = b.s.x; G[8 + k] = b.s.y; G[16 + k] = b.s.z;
-      G[24 + k] = b.e.x; G[32 + k] = b.e.y; G[40 + k] = b.e.z;
+      const int node = first + k;
+      const Box &b = t.bounds[node], &cm = common[node];
       if (slb[node].s.x <= slb[node].e.x) nonempty |= 1u << k;
-      int32_t link, count;
+      int32_t link, count = 0;
       if (t.children[node] >= 0) {
         link = (t.children[node] - 1) / 8;
-        count = -1;
         const int rank = __builtin_popcount(interior);
         if (rank == 0) first_child = link;
         else if (link != first_child + rank) return -1;   // not breadth-first
         interior |= 1u << k;
+        link = (int32_t)(out.recs.size() / kRecWords);
       } else {
         leaf_records(node, link, count);
       }
-      memcpy(&G[kGroupLink + k], &link, 4);
-      memcpy(&G[kGroupCount + k], &count, 4);
+      memcpy(&G[kGroupEntry + k], &link, 4);
+      link += count;
+      if (k == 7) memcpy(&G[kGroupEntry + 8], &link, 4);
+      float *N = &out.nodes[(size_t)(node - 1) * kNodeWords];
+      const float w[6] = {b.s.x, b.s.y, b.s.z, b.e.x, b.e.y, b.e.z};
+      memcpy(N, w, sizeof(w));
+      const int32_t up = parent[node] - 1;                 // -1: the root
+      const int32_t nested = eq(cm.s, b.s) && eq(cm.e, b.e) ? 1 : 0;
+      memcpy(&N[6], &up, 4);
+      memcpy(&N[7], &nested, 4);
     }
+    quantize_group(&slb[first], nonempty, G);
     const uint32_t head = nonempty | (interior << 8);
-    memcpy(&G[kGroupMask], &head, 4);
+    memcpy(&G[kGroupHead], &head, 4);
     memcpy(&G[kGroupBase], &first_child, 4);
   }
   out.nrec = (int)(out.recs.size() / kRecWords);

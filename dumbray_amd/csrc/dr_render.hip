@@ -154,7 +154,6 @@ struct Tables {
 
 // Path updates of the benchmark plugins (DR_PLUGINS_BENCHMARK).
 struct BenchPath {
-  static constexpr bool kFastSlab = true;
   // k_render_stream: a job outside the image is written at once, and the job's block is read
   // back from the block ring when its pixel is written (29.5 ms at 1080p 16 spp, against
   // 30.8 ms with the other choices, which suit RefPath)
@@ -195,7 +194,7 @@ struct BenchPath {
     bool photons = false;
     if (st.phase == 0) {
       if (!w.hit) return true;
-      setup_vertex(P, K, tb.shade, w.h, w.ray.d, st);
+      setup_vertex(P, K, tb.shade, w.h, w.d, st);
       photons = st.kind == DR_LAMBERT;
     } else {
       const V3 e = w.h.p - st.p;
@@ -220,9 +219,6 @@ struct BenchPath {
 // sample are computed again where they are used; both are functions of the vertex and
 // of counter-based random numbers, so the order of evaluation does not change them.
 struct RefPath {
-  // waves holding an axis-parallel photon (a directional light along an axis) take the
-  // NaN-handling form; the example scene's soft lights do not (15.0 -> 14.1 ms at 1080p)
-  static constexpr bool kFastSlab = true;
   // k_render_stream: a job outside the image goes through the path-update phase, and the
   // job's block stays in a register (example scene 8.5 ms, against 9.4-9.9 ms otherwise:
   // fewer spilled registers)
@@ -342,7 +338,7 @@ struct RefPath {
       if (!w.hit) return true;                        // the layer ray missed (:418-421)
       h = w.h.id;
       hp = w.h.p;
-      din = w.ray.d;
+      din = w.d;
       mid = __float_as_int(tb.shade[h].w);
       const int kind = P.materials[mid].kind;
       light = (kind == DR_MIRROR || kind == DR_METAL) ? P.nlights : -1;   // delta BSDFs take no direct light
@@ -421,8 +417,8 @@ enum : int {
   kRcPlane,             // triangle plane tests
   kRcInside,            // triangle inside tests
   kRcPaths,             // path jobs (pixel samples) started
-  kRcLive,              // children of expanded groups with a non-empty leaf below (octant tests)
-  kRcSlab,              // children whose slab test ran
+  kRcLive,              // children of expanded groups with a non-empty leaf below (box tests)
+  kRcSlab,              // children that the box test kept
   kRcCount
 };
 struct RenderCounters {
@@ -516,7 +512,7 @@ __device__ __forceinline__ void render_block(const DevTree &T, const Tables &tb,
               const float zero[3] = {0.0f, 0.0f, 0.0f};
               finish(zero);
             } else {
-              walk_begin(T, w, ps.ray_o(), ps.ray_d(), ps.ray_excl(), lds.stk, kRB, nullptr);
+              walk_begin(T, w, ps.ray_o(), ps.ray_d(), ps.ray_excl());
               if (kStats) { rc->paths++; rc->segments++; }
             }
           } else {
@@ -529,7 +525,7 @@ __device__ __forceinline__ void render_block(const DevTree &T, const Tables &tb,
         continue;
       }
       // ---- one traversal step of every ray in flight
-      if (job >= 0 && w.state == kWalkTrace) walk_step<PathT::kFastSlab>(T, w, lds.stk, kRB, cc);
+      if (job >= 0 && w.state == kWalkTrace) walk_step(T, w, lds.stk, kRB, cc);
       // ---- leaf tests, batched
       const bool pend = job >= 0 && w.state == kWalkLeaf;
       const uint64_t pm = __ballot(pend);
@@ -542,7 +538,7 @@ __device__ __forceinline__ void render_block(const DevTree &T, const Tables &tb,
           if (ps.shade(P, K, tb, w)) {
             finish(ps.color());
           } else {
-            walk_begin(T, w, ps.ray_o(), ps.ray_d(), ps.ray_excl(), lds.stk, kRB, nullptr);
+            walk_begin(T, w, ps.ray_o(), ps.ray_d(), ps.ray_excl());
             if (kStats) { rc->segments++; rc->photons += ps.photon() ? 1 : 0; }
           }
         }
@@ -732,7 +728,7 @@ __global__ __launch_bounds__(kRB, kRenderWaves) void k_render_stream(DevTree T, 
             if (PathT::kStreamBlackInUpdate) w.state = kWalkDone;
             else finish(0.0f, 0.0f, 0.0f);
           } else {
-            walk_begin(T, w, ps.ray_o(), ps.ray_d(), ps.ray_excl(), stk, kRB, nullptr);
+            walk_begin(T, w, ps.ray_o(), ps.ray_d(), ps.ray_excl());
             if (kStats) { rc.paths++; rc.segments++; }
           }
         }
@@ -744,7 +740,7 @@ __global__ __launch_bounds__(kRB, kRenderWaves) void k_render_stream(DevTree T, 
       continue;
     }
     // ---- one traversal step of every ray in flight
-    if (live && w.state == kWalkTrace) walk_step<PathT::kFastSlab>(T, w, stk, kRB, cc);
+    if (live && w.state == kWalkTrace) walk_step(T, w, stk, kRB, cc);
     // ---- leaf tests, batched
     const bool pend = live && w.state == kWalkLeaf;
     const uint64_t pm = __ballot(pend);
@@ -766,7 +762,7 @@ __global__ __launch_bounds__(kRB, kRenderWaves) void k_render_stream(DevTree T, 
           const bool black = PathT::kStreamBlackInUpdate && nopath;
           finish(black ? 0.0f : c0, black ? 0.0f : c1, black ? 0.0f : c2);
         } else {
-          walk_begin(T, w, ps.ray_o(), ps.ray_d(), ps.ray_excl(), stk, kRB, nullptr);
+          walk_begin(T, w, ps.ray_o(), ps.ray_d(), ps.ray_excl());
           if (kStats) { rc.segments++; rc.photons += ps.photon() ? 1 : 0; }
         }
       }
@@ -945,7 +941,7 @@ __global__ __launch_bounds__(kRB, kRenderWaves) void k_backward(DevTree T, const
               // SphericalSegmentLense::getPixelColor scales the sample colour by its filter
               for (int c = 0; c < 3; c++)
                 wdl[c] = spw * g[c] * (P.lens == DR_SPHERICAL_SEGMENT_LENS ? P.lens_p[4 + c] : 1.0f);
-              walk_begin(T, w, st.o, st.d, st.restrict_tri, stk, kRB, nullptr);
+              walk_begin(T, w, st.o, st.d, st.restrict_tri);
             }
           } else {
             exhausted = true;
@@ -971,7 +967,7 @@ __global__ __launch_bounds__(kRB, kRenderWaves) void k_backward(DevTree T, const
           if (st.phase == 0) {
             if (!w.hit) fin = true;
             else {
-              setup_vertex(P, FK, shade, w.h, w.ray.d, st);
+              setup_vertex(P, FK, shade, w.h, w.d, st);
               V_(K, 0) = __int_as_float(st.mid);
               for (int c = 0; c < 4; c++) V_(K, 4 + c) = 0.0f;
               K++;
@@ -993,7 +989,7 @@ __global__ __launch_bounds__(kRB, kRenderWaves) void k_backward(DevTree T, const
             photons = true;
           }
           if (photons && !next_photon(P, st)) advance();
-          if (!fin) walk_begin(T, w, st.o, st.d, st.restrict_tri, stk, kRB, nullptr);
+          if (!fin) walk_begin(T, w, st.o, st.d, st.restrict_tri);
         }
         // dL/demission of this update's lit photons
         wave_add3(gacc, lit, lkey, ev);

@@ -5,26 +5,36 @@
 // Order of work is the reference's: children of an expanded node are visited
 // in the order canonical ^ i (i = 0..7), a leaf that accepts a hit ends the
 // cast, and inside a leaf the first triangle with the strictly smallest t wins.
-// The box tests of all 8 children are evaluated together when a node is
-// expanded (they are pure, so this only changes when, not whether, they run).
-// Children whose subtree leaves all lie outside the ray's forward octant are
-// dropped: no hit point o + d*t with t >= 0 can be inside their boxes, so the
-// reference would visit them and reject every hit.
+// Which subtrees are skipped is decided by a conservative test on compact child
+// boxes (dr_group.h): it never skips one that holds a leaf able to accept a hit.
+// Whether the reference would have reached the leaf at all (its slab tests on the
+// leaf's box and on those of its ancestors) is decided exactly when a hit is about to
+// be accepted, so the walk visits a superset of the reference's leaves in the
+// reference's order and accepts the same first hit.
 #pragma once
 #include "dr_geom.h"
+#include "dr_group.h"
 #include "dr_octree_build.h"
 
 namespace dr {
 
 struct DevTree {
   const float4 *__restrict__ groups;   // kGroupF4 float4 per group
+  const float4 *__restrict__ nodes;    // kNodeF4 float4 per node below the root
   const float4 *__restrict__ recs;     // 4 float4 per triangle record, one per leaf entry
   const float4 *__restrict__ urecs;    // the same records once per distinct triangle
   const int *__restrict__ lref;        // leaf entry -> record in urecs
   float rsx, rsy, rsz, rex, rey, rez;  // root box
   int root_is_leaf, root_start, root_count;
-  float margin;                        // prune margin of the octant test (see the group layout)
+  float reach;                         // largest magnitude of a box coordinate
 };
+
+__device__ __forceinline__ Box root_box(const DevTree &T) {
+  Box b;
+  b.s = v3(T.rsx, T.rsy, T.rsz);
+  b.e = v3(T.rex, T.rey, T.rez);
+  return b;
+}
 
 struct Hit {
   int id;        // -1 miss
@@ -34,48 +44,13 @@ struct Hit {
 
 // Work counters of one cast (measurement launches only; nullptr elsewhere).
 struct CastCounters {
-  int expand;    // groups expanded (196-B reads: 8 boxes + non-empty mask)
-  int leaves;    // leaves whose triangles were tested (+ leaf box and link/count reads)
+  int expand;    // groups expanded (80-B reads: grid, head and 8 child boxes)
+  int leaves;    // leaves whose triangles were tested (+ the 8-B read of their entries)
   int plane;     // triangle records whose plane test ran (first 32 B)
   int inside;    // records that reached the inside test (second 32 B)
-  int live;      // children of expanded groups with a non-empty leaf below (octant tests run)
-  int slab;      // children whose slab test ran (live and not behind the ray's origin)
+  int live;      // children of expanded groups with a non-empty leaf below
+  int slab;      // children that the box test kept
 };
-
-// A ray prepared for traversal.
-struct TRay {
-  V3 o, d, inv;
-  int canon;     // canonicalOrder (Octree.impl.cuh:181-183)
-  V3 hi, lo;     // prune thresholds: a child is behind if max.k < hi.k or min.k > lo.k (see set_prune)
-};
-__device__ __forceinline__ TRay make_tray(V3 o, V3 d) {
-  TRay r;
-  r.o = o;
-  r.d = d;
-  r.inv = v3(1.0f / d.x, 1.0f / d.y, 1.0f / d.z);
-  int c = (d.z < 0) ? 1 : 0;
-  if (d.y < 0) c += 2;
-  if (d.x < 0) c += 4;
-  r.canon = c;
-  return r;
-}
-
-// v rounded down (up) by at least one ulp of v: below (above) every real number that
-// rounds to v.
-__device__ __forceinline__ float below(float v) { return v - (__builtin_fabsf(v) * 2.4e-7f + 1e-37f); }
-__device__ __forceinline__ float above(float v) { return v + (__builtin_fabsf(v) * 2.4e-7f + 1e-37f); }
-// Prune thresholds of the forward-octant test for margin M.  On an axis with d.k >= 0
-// a child whose box max satisfies max.k < hi.k = below(o.k - M) has max.k + M < o.k in
-// exact arithmetic, so every non-empty leaf below it (within the box widened by M) lies
-// behind o along k; symmetrically lo.k = above(o.k + M) for d.k <= 0.  Axes that do not
-// apply get -inf / +inf.
-__device__ __forceinline__ void set_prune(TRay &r, float M) {
-  const float inf = __builtin_inff();
-  r.hi = v3(r.d.x >= 0 ? below(r.o.x - M) : -inf, r.d.y >= 0 ? below(r.o.y - M) : -inf,
-            r.d.z >= 0 ? below(r.o.z - M) : -inf);
-  r.lo = v3(r.d.x <= 0 ? above(r.o.x + M) : inf, r.d.y <= 0 ? above(r.o.y + M) : inf,
-            r.d.z <= 0 ? above(r.o.z + M) : inf);
-}
 
 // One edge of Triangle::containsVertex (Triangle.impl.h:299-301): fl(fl(D / fl(sqrt(S))) + tol) >= thr
 // with D = dot(edge, p - vertex), S = dot(p - vertex, p - vertex), correctly rounded division
@@ -114,112 +89,69 @@ __device__ __forceinline__ bool inside(V3 p, V3 a, V3 b, V3 c, float thr0, float
          (e2 == 1 || edge_exact(D2, S2, thr2));
 }
 
-// Box of child k of group g (the leaf-acceptance box).
-__device__ __forceinline__ Box child_box(const float4 *__restrict__ G, int g, int k) {
-  const float *f = (const float *)(G + kGroupF4 * (size_t)g);
-  Box b;
-  b.s = v3(f[k], f[8 + k], f[16 + k]);
-  b.e = v3(f[24 + k], f[32 + k], f[40 + k]);
-  return b;
-}
-
 // Traversal stack.  A level holds two words, [2*level][lane] and [2*level+1][lane]:
 //   lo = group << 8 | mask of children still to visit (bit i = child canon ^ i)
 //   hi = first interior child's group << 8 | interior mask (bit k = child k)
 // so popping an interior child needs no memory read.
 constexpr int kStackWordsPerLevel = 2;
 
-// 8 child tests of group g -> stack entry.  A child is kept if it has a non-empty
-// leaf below it, its box widened by the prune margin meets the forward octant of
-// the ray (the thresholds of set_prune), and the reference slab test on its box passes.
-template <bool kFinite>
-__device__ __forceinline__ void group_entry(const float4 *__restrict__ G, int g, const TRay &r, uint32_t &lo,
+// The children of group g to visit -> stack entry: those with a non-empty leaf below them that
+// the box test keeps, in visiting order.
+__device__ __forceinline__ void group_entry(const float4 *__restrict__ G, int g, const BoxRay &r, uint32_t &lo,
                                             uint32_t &hi, CastCounters *cc = nullptr) {
   const float4 *q = G + kGroupF4 * (size_t)g;
-  // children with no non-empty leaf below them are dropped before their box tests run
-  const uint2 head = *(const uint2 *)(q + kGroupMask / 4);
-  uint32_t m = 0;
-  // all 192 B of child boxes requested at once, before any child is tested: the loads of the
-  // second four children no longer wait behind the tests of the first four (incoherent cast
-  // 2.41 -> 2.34 ms, 1080p render 26.3 -> 26.0 ms)
-  float4 qv[12];
-#pragma unroll
-  for (int k = 0; k < 12; ++k) qv[k] = q[k];
-#pragma unroll
-  for (int h = 0; h < 2; ++h) {       // children in two halves of 4
-    const float4 sx = qv[0 + h], sy = qv[2 + h], sz = qv[4 + h], ex = qv[6 + h], ey = qv[8 + h], ez = qv[10 + h];
-    const float a_sx[4] = {sx.x, sx.y, sx.z, sx.w}, a_sy[4] = {sy.x, sy.y, sy.z, sy.w},
-                a_sz[4] = {sz.x, sz.y, sz.z, sz.w}, a_ex[4] = {ex.x, ex.y, ex.z, ex.w},
-                a_ey[4] = {ey.x, ey.y, ey.z, ey.w}, a_ez[4] = {ez.x, ez.y, ez.z, ez.w};
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      // forward octant of o: coordinate k of o + d*t (t >= 0) is >= o.k if d.k >= 0, <= o.k if d.k <= 0
-      const bool live = (head.x >> (4 * h + j)) & 1u;
-      const bool behind = !live || (a_ex[j] < r.hi.x) || (a_sx[j] > r.lo.x) || (a_ey[j] < r.hi.y) ||
-                          (a_sy[j] > r.lo.y) || (a_ez[j] < r.hi.z) || (a_sz[j] > r.lo.z);
-      if (cc) { cc->live += live ? 1 : 0; cc->slab += behind ? 0 : 1; }
-      const bool hit =
-          !behind && (kFinite ? slab_hit_finite(a_sx[j], a_sy[j], a_sz[j], a_ex[j], a_ey[j], a_ez[j], r.o, r.inv)
-                              : slab_hit(a_sx[j], a_sy[j], a_sz[j], a_ex[j], a_ey[j], a_ez[j], r.o, r.inv));
-      m |= hit ? (1u << (4 * h + j)) : 0u;
-    }
-  }
+  const float4 grid = q[0], cell = q[1], b0 = q[2], b1 = q[3], b2 = q[4];
+  const uint32_t head = (uint32_t)__float_as_int(grid.w), base = (uint32_t)__float_as_int(cell.w);
+  const uint32_t w[12] = {(uint32_t)__float_as_int(b0.x), (uint32_t)__float_as_int(b0.y), (uint32_t)__float_as_int(b0.z),
+                          (uint32_t)__float_as_int(b0.w), (uint32_t)__float_as_int(b1.x), (uint32_t)__float_as_int(b1.y),
+                          (uint32_t)__float_as_int(b1.z), (uint32_t)__float_as_int(b1.w), (uint32_t)__float_as_int(b2.x),
+                          (uint32_t)__float_as_int(b2.y), (uint32_t)__float_as_int(b2.z), (uint32_t)__float_as_int(b2.w)};
+  uint32_t m = group_children(v3(grid.x, grid.y, grid.z), v3(cell.x, cell.y, cell.z), w, r) & head & 0xffu;
+  if (cc) { cc->live += __builtin_popcount(head & 0xffu); cc->slab += __builtin_popcount(m); }
   const int c = r.canon;
   if (c & 1) m = ((m & 0x55u) << 1) | ((m >> 1) & 0x55u);
   if (c & 2) m = ((m & 0x33u) << 2) | ((m >> 2) & 0x33u);
   if (c & 4) m = ((m & 0x0Fu) << 4) | ((m >> 4) & 0x0Fu);
   lo = ((uint32_t)g << 8) | m;
-  hi = (head.y << 8) | ((head.x >> 8) & 0xffu);
-}
-
-// Initial traversal state.  Returns 0 = miss, 1 = traversal pending, 2 = root is a leaf.
-// The root's group (group 0, the root's children) is expanded by the first walk_step,
-// with the expansions of the other lanes, rather than here: a new ray is set up in the
-// divergent code that hands out work, where an expansion would run with few lanes.
-__device__ __forceinline__ int tree_begin(const DevTree &T, const TRay &r, int &sp) {
-  if (T.root_is_leaf) return 2;
-  if (!slab_hit(T.rsx, T.rsy, T.rsz, T.rex, T.rey, T.rez, r.o, r.inv)) return 0;
-  sp = -1;
-  return 1;
+  hi = (base << 8) | ((head >> 8) & 0xffu);
 }
 
 // One lane's closest-hit query, advanced in bounded steps so that a kernel can
 // interleave many of them (and batch their leaf tests) across a wave.
 enum : int { kWalkTrace = 1, kWalkLeaf = 2, kWalkDone = 3 };
 struct Walk {
-  TRay ray;
+  V3 o, d;
+  BoxRay box;
   int ex;              // validateNotSameAsObject's object, or -1
   int sp, state;
-  int lg, lk, llink, lcnt;   // pending leaf: child lk of group lg (lg < 0: the root)
+  int leaf, llink, lcnt;   // pending leaf: its node (-1: the root), first leaf entry and entry count
   bool hit;            // result once state == kWalkDone
   Hit h;
 };
 
-__device__ __forceinline__ void walk_begin(const DevTree &T, Walk &w, V3 o, V3 d, int exclude, uint32_t *stk,
-                                           int stride, CastCounters *cc) {
-  w.ray = make_tray(o, d);
-  set_prune(w.ray, T.margin);
+__device__ __forceinline__ void walk_begin(const DevTree &T, Walk &w, V3 o, V3 d, int exclude) {
+  w.o = o;
+  w.d = d;
   w.ex = exclude;
   w.hit = false;
-  const int st = tree_begin(T, w.ray, w.sp);
-  if (st == 0) {
-    w.state = kWalkDone;
-  } else if (st == 2) {
+  w.sp = -1;
+  w.leaf = -1;
+  if (T.root_is_leaf) {
+    w.llink = T.root_start;
+    w.lcnt = T.root_count;
     w.state = kWalkLeaf;
-    w.lg = -1; w.llink = T.root_start; w.lcnt = T.root_count;
-  } else {
-    w.state = kWalkTrace;
+    return;
   }
+  const bool alive = box_ray(o, d, T.reach, w.box) && box_kept(root_box(T), w.box);
+  w.state = alive ? kWalkTrace : kWalkDone;
 }
 
 // Pops one child: expands an interior child, or holds a leaf child as pending;
 // an exhausted stack ends the query with a miss.  A walk's first step (sp == -1 after
-// walk_begin) expands the root's group.
-// kFastSlab: expand with the NaN-free slab test whenever no expanding lane of the wave has an
-// infinite 1/d (kernels with registers to spare for the second copy of the child test).
-template <bool kFastSlab = true>
+// walk_begin) expands the root's group (group 0) with the expansions of the other lanes,
+// rather than in the divergent code that hands out work.
 __device__ __forceinline__ void walk_step(const DevTree &T, Walk &w, uint32_t *stk, int stride, CastCounters *cc) {
-  int child = 0;                      // group to expand; 0 (the root's) on a walk's first step
+  int child = 0;                      // group to expand
   if (w.sp >= 0) {
     uint32_t f = 0;
     while (w.sp >= 0) {
@@ -230,27 +162,21 @@ __device__ __forceinline__ void walk_step(const DevTree &T, Walk &w, uint32_t *s
     if (w.sp < 0) { w.state = kWalkDone; return; }
     const int i = __builtin_ctz(f & 0xffu);
     stk[2 * w.sp * stride] = f & ~(1u << i);
-    const int k = w.ray.canon ^ i;
+    const int k = w.box.canon ^ i;
     const uint32_t hi = stk[(2 * w.sp + 1) * stride];
     const uint32_t im = hi & 0xffu;
     if (!((im >> k) & 1u)) {
-      const int *Gi = (const int *)T.groups;
-      const size_t base = kGroupWords * (size_t)(f >> 8);
-      w.lg = (int)(f >> 8);
-      w.lk = k;
-      w.llink = Gi[base + kGroupLink + k];
-      w.lcnt = Gi[base + kGroupCount + k];
+      const int *E = (const int *)T.groups + kGroupWords * (size_t)(f >> 8) + kGroupEntry + k;
+      w.leaf = (int)(f >> 8) * 8 + k;
+      w.llink = E[0];
+      w.lcnt = E[1] - E[0];
       w.state = kWalkLeaf;
       return;
     }
     child = (int)(hi >> 8) + __builtin_popcount(im & ((1u << k) - 1u));
   }
   uint32_t lo2, hi2;
-  // the NaN-free form of the slab test when no expanding lane of the wave has an infinite 1/d
-  const bool finite = __builtin_isfinite(w.ray.inv.x) && __builtin_isfinite(w.ray.inv.y) &&
-                      __builtin_isfinite(w.ray.inv.z);
-  if (kFastSlab && __ballot(!finite) == 0) group_entry<true>(T.groups, child, w.ray, lo2, hi2, cc);
-  else group_entry<false>(T.groups, child, w.ray, lo2, hi2, cc);
+  group_entry(T.groups, child, w.box, lo2, hi2, cc);
   ++w.sp;
   stk[2 * w.sp * stride] = lo2;
   stk[(2 * w.sp + 1) * stride] = hi2;
@@ -331,8 +257,8 @@ __device__ __forceinline__ void walk_leaf_wave(const DevTree &T, Walk &w, bool p
   };
   // tests record j (of owner `owner`; its 64 B in r0..r3) for its owner; every lane takes part
   auto test_record = [&](int j, int owner, float4 r0, float4 r1, float4 r2, float4 r3) {
-    const V3 o = v3(__shfl(w.ray.o.x, owner), __shfl(w.ray.o.y, owner), __shfl(w.ray.o.z, owner));
-    const V3 d = v3(__shfl(w.ray.d.x, owner), __shfl(w.ray.d.y, owner), __shfl(w.ray.d.z, owner));
+    const V3 o = v3(__shfl(w.o.x, owner), __shfl(w.o.y, owner), __shfl(w.o.z, owner));
+    const V3 d = v3(__shfl(w.d.x, owner), __shfl(w.d.y, owner), __shfl(w.d.z, owner));
     const int pos = j - __shfl(start, owner);
     const int ex = __shfl(w.ex, owner);
     if (j < total) {
@@ -387,14 +313,11 @@ __device__ __forceinline__ void walk_leaf_wave(const DevTree &T, Walk &w, bool p
   if (key != ~0ull) {
     const float t = __uint_as_float((unsigned)(key >> 32));
     const int k = w.llink + (int)(key & 0xffffffffu);
-    const V3 p = w.ray.o + w.ray.d * t;
+    const V3 p = w.o + w.d * t;
     // the record's id is read beside the leaf box, before the box test that decides whether
     // it is needed
     const int rid = kIndexed ? __float_as_int(T.urecs[4 * T.lref[k] + 3].w) : __float_as_int(T.recs[4 * k + 3].w);
-    Box lb;
-    if (w.lg < 0) { lb.s = v3(T.rsx, T.rsy, T.rsz); lb.e = v3(T.rex, T.rey, T.rez); }
-    else lb = child_box(T.groups, w.lg, w.lk);
-    if (contains(lb, p)) {
+    if (leaf_accepts(T.nodes, root_box(T), w.leaf, w.o, w.d, p)) {
       hit = true;
       w.h.id = rid;
       w.h.t = t;
@@ -402,7 +325,7 @@ __device__ __forceinline__ void walk_leaf_wave(const DevTree &T, Walk &w, bool p
     }
   }
   w.hit = hit;
-  w.state = (hit || w.lg < 0) ? kWalkDone : kWalkTrace;
+  w.state = (hit || w.leaf < 0) ? kWalkDone : kWalkTrace;
 }
 
 }  // namespace dr
