@@ -46,12 +46,13 @@ __global__ __launch_bounds__(kCastBlock, 4) void k_cast(DevTree T, const float *
                                                       float *__restrict__ out_t, float *__restrict__ out_p,
                                                       int *__restrict__ stats, unsigned *__restrict__ work) {
   extern __shared__ uint32_t stk_base[];
-  __shared__ unsigned long long best_all[kCastBlock];   // per lane: best (t, record) key of its leaf
+  __shared__ LeafLds leaf_all[kWavesPerBlock];
   __shared__ int ins_all[kStats ? kCastBlock : 1];      // per lane: inside tests of its leaf (measurement)
   __shared__ int res_id_all[kWavesPerBlock][kSlots][kWaveChunk];
   __shared__ float res_t_all[kWavesPerBlock][kSlots][kWaveChunk];
   uint32_t *stk = stk_base + threadIdx.x;
-  unsigned long long *best = best_all + (threadIdx.x & ~63u);
+  LeafLds &leaf = leaf_all[threadIdx.x >> 6];
+  leaf_lds_init(leaf);
   int *ins = kStats ? ins_all + (threadIdx.x & ~63u) : nullptr;
   int *res_id = &res_id_all[threadIdx.x >> 6][0][0];
   float *res_t = &res_t_all[threadIdx.x >> 6][0][0];
@@ -184,7 +185,7 @@ __global__ __launch_bounds__(kCastBlock, 4) void k_cast(DevTree T, const float *
     const bool pend = r >= 0 && w.state == kWalkLeaf;
     const uint64_t pm = __ballot(pend);
     if (pm && (__popcll(pm) >= kLeafMin || __ballot(r >= 0 && w.state == kWalkTrace) == 0)) {
-      walk_leaf_wave<true>(T, w, pend, clip != 0, best, ins, cc);
+      walk_leaf_wave<true>(T, w, pend, clip != 0, leaf, ins, cc);
       if (pend && w.state == kWalkDone) finish();
     }
   }

@@ -404,7 +404,7 @@ struct BlockLds {
   float *samp_col;      // kBlockPixels * kRoundSamples * 3 sample colours
   float *acc;           // kBlockPixels * 3 pixel sums
   int *next_job;
-  unsigned long long *best;   // this wave's leaf-test slots (walk_leaf_wave)
+  LeafLds *leaf;        // this wave's (walk_leaf_wave)
   int *ins;             // this wave's inside-test counts (measurement launches only)
 };
 
@@ -530,7 +530,7 @@ __device__ __forceinline__ void render_block(const DevTree &T, const Tables &tb,
       const bool pend = job >= 0 && w.state == kWalkLeaf;
       const uint64_t pm = __ballot(pend);
       if (pm && (__popcll(pm) >= kLeafMin || __ballot(job >= 0 && w.state == kWalkTrace) == 0))
-        walk_leaf_wave(T, w, pend, clip, lds.best, kStats ? lds.ins : nullptr, cc);
+        walk_leaf_wave(T, w, pend, clip, *lds.leaf, kStats ? lds.ins : nullptr, cc);
       // ---- path updates of the finished casts, batched
       const uint64_t dm = __ballot(job >= 0 && w.state == kWalkDone);
       if (dm && (__popcll(dm) >= PathT::kShadeMin || __ballot(job >= 0 && w.state != kWalkDone) == 0)) {
@@ -563,10 +563,11 @@ __global__ __launch_bounds__(kRB, kRenderWaves) void k_render(DevTree T, Tables 
   extern __shared__ uint32_t lds[];
   __shared__ float acc[kBlockPixels * 3];
   __shared__ int next_job;
-  __shared__ unsigned long long best[kRB];
+  __shared__ LeafLds leaf[kRB / 64];
   __shared__ int ins[kStats ? kRB : 1];
   const BlockLds L = {lds + threadIdx.x, (float *)(lds + levels * kStackWordsPerLevel * kRB), acc, &next_job,
-                      best + (threadIdx.x & ~63u), kStats ? ins + (threadIdx.x & ~63u) : nullptr};
+                      leaf + (threadIdx.x >> 6), kStats ? ins + (threadIdx.x & ~63u) : nullptr};
+  leaf_lds_init(*L.leaf);
   RenderCounters rc;
   render_block<PathT, kStats>(T, tb, P, K, frame, start_block + (int)blockIdx.x, L, PathT::kRefillMin, &rc);
   if (kStats) flush_counters(rc, counts);
@@ -617,7 +618,7 @@ __global__ __launch_bounds__(kRB, kRenderWaves) void k_render_stream(DevTree T, 
   __shared__ int px_done[kStreamBlockRing];   // pixels written, cumulative per ring entry
   __shared__ unsigned next_job;
   __shared__ int end_k;                       // first stream block number past the range
-  __shared__ unsigned long long best_all[kRB];
+  __shared__ LeafLds leaf_all[kRB / 64];
   __shared__ int ins_all[kStats ? kRB : 1];
   const int spp = P.fsaa_x * P.fsaa_y;
   const int nslots = stream_slots(spp);
@@ -625,7 +626,8 @@ __global__ __launch_bounds__(kRB, kRenderWaves) void k_render_stream(DevTree T, 
   float *samp = (float *)(lds + levels * kStackWordsPerLevel * kRB);   // nslots * spp * 3
   int *owner = (int *)(samp + (size_t)nslots * spp * 3);             // nslots
   int *remaining = owner + nslots;                                    // nslots
-  unsigned long long *best = best_all + (threadIdx.x & ~63u);
+  LeafLds &leaf = leaf_all[threadIdx.x >> 6];
+  leaf_lds_init(leaf);
   int *ins = kStats ? ins_all + (threadIdx.x & ~63u) : nullptr;
   for (int t = threadIdx.x; t < nslots; t += kRB) { owner[t] = t; remaining[t] = spp; }
   for (int t = threadIdx.x; t < kStreamBlockRing; t += kRB) { blocks[t] = 0; px_done[t] = 0; }
@@ -745,7 +747,7 @@ __global__ __launch_bounds__(kRB, kRenderWaves) void k_render_stream(DevTree T, 
     const bool pend = live && w.state == kWalkLeaf;
     const uint64_t pm = __ballot(pend);
     if (pm && (__popcll(pm) >= kLeafMin || __ballot(live && w.state == kWalkTrace) == 0))
-      walk_leaf_wave(T, w, pend, clip, best, ins, cc);
+      walk_leaf_wave(T, w, pend, clip, leaf, ins, cc);
     // ---- path updates of the finished casts, batched
     const uint64_t dm = __ballot(live && w.state == kWalkDone);
     if (dm && (__popcll(dm) >= PathT::kStreamShadeMin || __ballot(live && w.state != kWalkDone) == 0)) {
@@ -804,17 +806,17 @@ constexpr int kVtxWords = 9;
 // each row of 16 lanes with DPP row shifts (1, 2, 4, 8; a lane without a source adds 0)
 // leaves the row totals in lanes 15, 31, 47 and 63, which are read out and added.
 template <int kCtrl>
-__device__ __forceinline__ float dpp_or_zero(float v) {   // the DPP source's bits, 0 where it has none
+__device__ __forceinline__ float dpp_f_or_zero(float v) {   // the DPP source's bits, 0 where it has none
   return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), kCtrl, 0xf, 0xf, false));
 }
 __device__ __forceinline__ float lane_value(float v, int l) {
   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
 }
 __device__ __forceinline__ float wave_sum(float v) {
-  v += dpp_or_zero<0x111>(v);   // row_shr:1
-  v += dpp_or_zero<0x112>(v);   // row_shr:2
-  v += dpp_or_zero<0x114>(v);   // row_shr:4
-  v += dpp_or_zero<0x118>(v);   // row_shr:8
+  v += dpp_f_or_zero<0x111>(v);   // row_shr:1
+  v += dpp_f_or_zero<0x112>(v);   // row_shr:2
+  v += dpp_f_or_zero<0x114>(v);   // row_shr:4
+  v += dpp_f_or_zero<0x118>(v);   // row_shr:8
   return (lane_value(v, 15) + lane_value(v, 31)) + (lane_value(v, 47) + lane_value(v, 63));
 }
 
@@ -869,8 +871,9 @@ __global__ __launch_bounds__(kRB, kRenderWaves) void k_backward(DevTree T, const
                                                                  int levels, int maxv) {
   extern __shared__ uint32_t lds[];
   __shared__ int next_job, cur_block;
-  __shared__ unsigned long long best_all[kRB];
-  unsigned long long *best = best_all + (threadIdx.x & ~63u);
+  __shared__ LeafLds leaf_all[kRB / 64];
+  LeafLds &leaf = leaf_all[threadIdx.x >> 6];
+  leaf_lds_init(leaf);
   uint32_t *stk = lds + threadIdx.x;
   float *gacc = (float *)(lds + levels * kStackWordsPerLevel * kRB);   // nmat*3 albedo, then nlights*3 emission
   float *vtx = vtx_all + (size_t)blockIdx.x * maxv * kVtxWords * kRB;
@@ -956,7 +959,7 @@ __global__ __launch_bounds__(kRB, kRenderWaves) void k_backward(DevTree T, const
       const bool pend = st.job >= 0 && w.state == kWalkLeaf;
       const uint64_t pm = __ballot(pend);
       if (pm && (__popcll(pm) >= kLeafMin || __ballot(st.job >= 0 && w.state == kWalkTrace) == 0))
-        walk_leaf_wave(T, w, pend, clip, best, nullptr, nullptr);
+        walk_leaf_wave(T, w, pend, clip, leaf, nullptr, nullptr);
       const uint64_t dm = __ballot(st.job >= 0 && w.state == kWalkDone);
       if (dm && (__popcll(dm) >= kShadeMin || __ballot(st.job >= 0 && w.state != kWalkDone) == 0)) {
         bool lit = false;
@@ -1063,9 +1066,10 @@ __global__ __launch_bounds__(kRB, kRenderWaves) void k_batch(const DevRequest *_
   __shared__ float acc[kBlockPixels * 3];
   __shared__ int next_job;
   __shared__ int item;
-  __shared__ unsigned long long best[kRB];
+  __shared__ LeafLds leaf[kRB / 64];
   const BlockLds L = {lds + threadIdx.x, (float *)(lds + levels * kStackWordsPerLevel * kRB), acc, &next_job,
-                      best + (threadIdx.x & ~63u), nullptr};
+                      leaf + (threadIdx.x >> 6), nullptr};
+  leaf_lds_init(*L.leaf);
   for (;;) {
     if (threadIdx.x == 0) item = atomicAdd(counter, 1);
     __syncthreads();

@@ -58,35 +58,43 @@ struct CastCounters {
 __device__ __forceinline__ bool edge_exact(float D, float S, float thr) {
   return D / __builtin_sqrtf(S) + kInsideTol >= thr;
 }
-// The same decision from the hardware reciprocal square root where it is certain: 1 = pass,
-// 0 = fail, 2 = too close to call.  q = D * rsq(S) is within about 2 ulp of the correctly
+// The same decision from the hardware reciprocal square root where it is certain.
+// q = D * rsq(S) is within about 2 ulp of the correctly
 // rounded quotient (rsq within 1 ulp, one product rounding, the quotient's two roundings), and
 // the sum with tol adds at most one ulp more.  An edge is decided only when q + tol lies more
 // than kEdgeMargin * (|q| + tol), about 34 ulp, from thr; S outside [1e-30, 1e30] (where
 // denormals or overflow could enter) is left to the exact form.
+// hi and lo are the left side's upper and lower bound less thr (a difference of fp32 values has
+// the sign of the comparison): lo >= 0 passes, hi < 0 fails.
 constexpr float kEdgeMargin = 4e-6f;
-__device__ __forceinline__ int edge_fast(float D, float S, float thr) {
-  if (!(S >= 1e-30f && S <= 1e30f)) return 2;
+__device__ __forceinline__ void edge_bounds(float D, float S, float thr, float &lo, float &hi) {
   const float q = D * __builtin_amdgcn_rsqf(S);
   const float r = q + kInsideTol;
   const float m = kEdgeMargin * (__builtin_fabsf(q) + kInsideTol);
-  return (r - m >= thr) ? 1 : ((r + m < thr) ? 0 : 2);
+  lo = (r - m) - thr;
+  hi = (r + m) - thr;
 }
 
 // Triangle::containsVertex minus the degenerate test (degenerate triangles have no record).
-// The three edge conditions are ANDed; each is decided by edge_fast where it is certain and by
-// the exact form otherwise, so the result is the reference's bit for bit.
+// The three edge conditions are ANDed; they are decided by edge_bounds where it is certain and by
+// the exact form otherwise, so the result is the reference's bit for bit.  p equals a vertex
+// (inside by definition) only if that vertex's S is 0, which the range of S leaves to the exact form.
 __device__ __forceinline__ bool inside(V3 p, V3 a, V3 b, V3 c, float thr0, float thr1, float thr2) {
-  if (eq(p, a) || eq(p, b) || eq(p, c)) return true;
   const V3 ab = b - a, bc = c - b, ca = a - c;
   const V3 ax = p - a, bx = p - b, cx = p - c;
   const float D0 = dot(ab, ax), S0 = dot(ax, ax), D1 = dot(bc, bx), S1 = dot(bx, bx), D2 = dot(ca, cx),
               S2 = dot(cx, cx);
-  const int e0 = edge_fast(D0, S0, thr0), e1 = edge_fast(D1, S1, thr1), e2 = edge_fast(D2, S2, thr2);
-  if (e0 == 0 || e1 == 0 || e2 == 0) return false;
-  if ((e0 & e1 & e2) == 1) return true;
-  return (e0 == 1 || edge_exact(D0, S0, thr0)) && (e1 == 1 || edge_exact(D1, S1, thr1)) &&
-         (e2 == 1 || edge_exact(D2, S2, thr2));
+  float l0, l1, l2, h0, h1, h2;
+  edge_bounds(D0, S0, thr0, l0, h0);
+  edge_bounds(D1, S1, thr1, l1, h1);
+  edge_bounds(D2, S2, thr2, l2, h2);
+  if (min3(S0, S1, S2) >= 1e-30f && max3(S0, S1, S2) <= 1e30f) {
+    if (min3(h0, h1, h2) < 0.0f) return false;
+    if (l0 >= 0.0f && l1 >= 0.0f && l2 >= 0.0f) return true;   // (three tests: a NaN must not pass)
+  } else if (eq(p, a) || eq(p, b) || eq(p, c)) {
+    return true;
+  }
+  return edge_exact(D0, S0, thr0) && edge_exact(D1, S1, thr1) && edge_exact(D2, S2, thr2);
 }
 
 // Traversal stack.  A level holds two words, [2*level][lane] and [2*level+1][lane]:
@@ -183,40 +191,55 @@ __device__ __forceinline__ void walk_step(const DevTree &T, Walk &w, uint32_t *s
   if (cc) cc->expand++;
 }
 
-// Inclusive prefix sum of v over the 64 lanes of the wave (every lane active): DPP row
-// shifts by 1, 2, 4 and 8 (a lane without a source adds 0) scan each row of 16 lanes, and
-// each row adds the totals of the rows before it, read from lanes 15, 31 and 47 into scalar
-// registers.  `total` gets the sum over all lanes.  Unlike a scan over __shfl_up, it needs
-// no per-lane address registers, which the compiler would otherwise keep live across the
-// caller's loop.
-template <int kCtrl>
-__device__ __forceinline__ int dpp_shr_or_zero(int v) {
-  return __builtin_amdgcn_update_dpp(0, v, kCtrl, 0xf, 0xf, false);
+// Inclusive prefix sum and maximum over the 64 lanes of the wave (every lane active): DPP row
+// shifts by 1, 2, 4 and 8 scan each row of 16 lanes, then lane 15 of rows 0 and 2 is added to
+// the row after it and lane 31 to the upper half (a lane without a source takes 0).
+template <int kCtrl, int kRows = 0xf>
+__device__ __forceinline__ int dpp_or_zero(int v) {
+  return __builtin_amdgcn_update_dpp(0, v, kCtrl, kRows, 0xf, false);
 }
 __device__ __forceinline__ int wave_incl_scan(int v, int &total) {
-  v += dpp_shr_or_zero<0x111>(v);   // row_shr:1
-  v += dpp_shr_or_zero<0x112>(v);   // row_shr:2
-  v += dpp_shr_or_zero<0x114>(v);   // row_shr:4
-  v += dpp_shr_or_zero<0x118>(v);   // row_shr:8
-  const int r0 = __builtin_amdgcn_readlane(v, 15), r1 = __builtin_amdgcn_readlane(v, 31),
-            r2 = __builtin_amdgcn_readlane(v, 47), r3 = __builtin_amdgcn_readlane(v, 63);
-  total = (r0 + r1) + (r2 + r3);
-  const int row = (int)__lane_id() >> 4;
-  return v + (row > 0 ? r0 : 0) + (row > 1 ? r1 : 0) + (row > 2 ? r2 : 0);
+  v += dpp_or_zero<0x111>(v);        // row_shr:1
+  v += dpp_or_zero<0x112>(v);        // row_shr:2
+  v += dpp_or_zero<0x114>(v);        // row_shr:4
+  v += dpp_or_zero<0x118>(v);        // row_shr:8
+  v += dpp_or_zero<0x142, 0xa>(v);   // row_bcast:15 into rows 1 and 3
+  v += dpp_or_zero<0x143, 0xc>(v);   // row_bcast:31 into rows 2 and 3
+  total = __builtin_amdgcn_readlane(v, 63);
+  return v;
 }
+__device__ __forceinline__ int wave_incl_max(int v) {   // v >= 0
+  v = max(v, dpp_or_zero<0x111>(v));
+  v = max(v, dpp_or_zero<0x112>(v));
+  v = max(v, dpp_or_zero<0x114>(v));
+  v = max(v, dpp_or_zero<0x118>(v));
+  v = max(v, dpp_or_zero<0x142, 0xa>(v));
+  v = max(v, dpp_or_zero<0x143, 0xc>(v));
+  return v;
+}
+
+// One wave's LDS for walk_leaf_wave.
+struct LeafLds {
+  unsigned long long best[64];   // per lane: the smallest key of its leaf
+  int first[64];                 // per record of a round: the lane whose leaf starts there; 0 between calls
+};
+__device__ __forceinline__ void leaf_lds_init(LeafLds &L) { L.first[__lane_id()] = 0; }
 
 // castInLeaf for every pending lane of the wave at once, with all 64 lanes sharing
 // the records.  Must be called by every lane of the wave (wave-uniform control flow);
-// `pending` marks the lanes whose leaf is tested; `best` (and `ins`, counting the
-// records that reach the inside test, for measurement launches) hold one slot per
-// lane of the wave in LDS.
+// `pending` marks the lanes whose leaf is tested; `lds` is the wave's own
+// (and `ins`, counting the records that reach the inside test, for measurement launches).
 //   * The records of the pending leaves are numbered 0..total-1 in lane order (wave
 //     prefix sum of the counts); lane j tests records j, j + 64, ...
-//   * A record's owner is the last lane whose first record number is <= the record's
-//     (counted over the prefix sums in two levels, below); its ray, exclusion and first
-//     record come from the owner with __shfl.
+//   * A record's owner is the last lane whose first record number is <= the record's: the
+//     lanes whose leaf starts in a round leave their number at that place in LDS, and a
+//     prefix maximum spreads it; its ray, exclusion and first record come from the owner
+//     with __shfl.  (Renders are bound by vector instructions: counting the prefix sums <=
+//     the record's in two levels took 45 vector and 7 LDS instructions of a round's 330,
+//     this takes 12 and 3.  With the shorter inside() above, 1080p 16 spp 21.2 -> 19.7 ms, the
+//     256x256 frame 586 -> 501 us, 4M incoherent rays 1.30 -> 1.28 ms.)
 //   * A record that passes Triangle::cast with t < FLT_MAX offers the 64-bit key
-//     (t bits << 32 | record's position in its leaf) to the owner's slot in `best`
+//     (t bits << 32 | leaf entry) to the owner's slot in `best`
 //     (LDS, one uint64 per lane) with an atomic min.  t > 0, so the keys order by t
 //     first and by position second: the owner gets the first record with the smallest
 //     t, which is what the sequential strict '<' scan keeps (Octree.impl.cuh:595-606).
@@ -228,38 +251,32 @@ __device__ __forceinline__ int wave_incl_scan(int v, int &total) {
 // cast 2.31 -> 2.12 ms with the lref read ahead; 1080p render 25.6 -> 24.1 ms and the
 // 64-request batch 247 -> 228 ms with the owner search ahead).
 template <bool kIndexed = false>
-__device__ __forceinline__ void walk_leaf_wave(const DevTree &T, Walk &w, bool pending, bool clip,
-                                               unsigned long long *best, int *ins, CastCounters *cc) {
+__device__ __forceinline__ void walk_leaf_wave(const DevTree &T, Walk &w, bool pending, bool clip, LeafLds &lds,
+                                               int *ins, CastCounters *cc) {
   const int lane = (int)__lane_id();
   const int cnt = pending ? w.lcnt : 0;
   int total;
   const int incl = wave_incl_scan(cnt, total);
   const int start = incl - cnt;
-  if (pending) __hip_atomic_store(&best[lane], ~0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
-  if (cc && pending) __hip_atomic_store(&ins[lane], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
-  const int link = pending ? w.llink : 0;
-  // The owner of record j is the last lane whose first record number is <= j (the numbers
-  // never decrease from lane to lane), i.e. the count of lanes 1..63 whose number is <= j.
-  // Level 1 counts among lanes 8, 16, ..., 56, whose numbers sit in scalar registers for the
-  // whole batch; level 2 among the 7 lanes after the multiple of 8 found, fetched together.
-  int coarse[7];
-#pragma unroll
-  for (int m = 0; m < 7; m++) coarse[m] = __builtin_amdgcn_readlane(start, 8 * (m + 1));
-  // record j's owner (wave-uniform call)
-  auto owner_of = [&](int j) {
-    int b = 0;
-#pragma unroll
-    for (int m = 0; m < 7; m++) b += coarse[m] <= j ? 8 : 0;
-    int owner = b;
-#pragma unroll
-    for (int i = 1; i < 8; i++) owner += __shfl(start, b + i) <= j ? 1 : 0;
-    return owner;
+  auto put = [](auto *p, auto v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT); };
+  auto get = [](auto *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT); };
+  if (pending) put(&lds.best[lane], ~0ull);
+  if (cc && pending) put(&ins[lane], 0);
+  const int link = (pending ? w.llink : 0) - start;      // leaf entry of record j: link + j
+  // owner of record base + lane (wave-uniform call; one call per round, in order)
+  int last = 0;                                          // the previous round's last owner
+  auto owner_of = [&](int base) {
+    const bool here = cnt > 0 && (unsigned)(start - base) < 64u;
+    if (here) put(&lds.first[start - base], lane);
+    const int v = max(wave_incl_max(get(&lds.first[lane])), last);
+    if (here) put(&lds.first[start - base], 0);
+    last = __builtin_amdgcn_readlane(v, 63);
+    return v;
   };
   // tests record j (of owner `owner`; its 64 B in r0..r3) for its owner; every lane takes part
-  auto test_record = [&](int j, int owner, float4 r0, float4 r1, float4 r2, float4 r3) {
+  auto test_record = [&](int j, int owner, int entry, float4 r0, float4 r1, float4 r2, float4 r3) {
     const V3 o = v3(__shfl(w.o.x, owner), __shfl(w.o.y, owner), __shfl(w.o.z, owner));
     const V3 d = v3(__shfl(w.d.x, owner), __shfl(w.d.y, owner), __shfl(w.d.z, owner));
-    const int pos = j - __shfl(start, owner);
     const int ex = __shfl(w.ex, owner);
     if (j < total) {
       const V3 a = v3(r0.x, r0.y, r0.z), n = v3(r0.w, r1.x, r1.y);
@@ -273,8 +290,8 @@ __device__ __forceinline__ void walk_leaf_wave(const DevTree &T, Walk &w, bool p
           const V3 b = v3(r1.z, r1.w, r2.x), c = v3(r2.y, r2.z, r2.w);
           if (inside(p, a, b, c, r3.x, r3.y, r3.z)) {
             const unsigned long long key =
-                ((unsigned long long)__float_as_uint(t) << 32) | (unsigned long long)(unsigned)pos;
-            __hip_atomic_fetch_min(&best[owner], key, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+                ((unsigned long long)__float_as_uint(t) << 32) | (unsigned long long)(unsigned)entry;
+            __hip_atomic_fetch_min(&lds.best[owner], key, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
           }
         }
       }
@@ -284,23 +301,21 @@ __device__ __forceinline__ void walk_leaf_wave(const DevTree &T, Walk &w, bool p
   // is found while the current round's records are fetched and tested, so a round's record
   // loads start at once.
   const float4 *R = kIndexed ? T.urecs : T.recs;
-  int own = owner_of(lane);
+  int own = owner_of(0);
+  int el = __shfl(link, own) + lane;                     // every lane takes part
   int kn = 0;
-  {
-    const int kel0 = __shfl(link, own) + lane - __shfl(start, own);   // every lane takes part
-    if (lane < total) kn = kIndexed ? T.lref[kel0] : kel0;
-  }
+  if (lane < total) kn = kIndexed ? T.lref[el] : el;
   for (int base = 0; base < total; base += 64) {
     const int j = base + lane;
-    const int owner = own;
+    const int owner = own, entry = el;
     const int k = j < total ? kn : 0;      // (lanes past the last record read record 0)
     const float4 r0 = R[4 * k + 0], r1 = R[4 * k + 1], r2 = R[4 * k + 2], r3 = R[4 * k + 3];
     if (base + 64 < total) {
-      own = owner_of(j + 64);
-      const int kel = __shfl(link, own) + (j + 64) - __shfl(start, own);
-      if (j + 64 < total) kn = kIndexed ? T.lref[kel] : kel;
+      own = owner_of(base + 64);
+      el = __shfl(link, own) + j + 64;
+      if (j + 64 < total) kn = kIndexed ? T.lref[el] : el;
     }
-    test_record(j, owner, r0, r1, r2, r3);
+    test_record(j, owner, entry, r0, r1, r2, r3);
   }
   if (!pending) return;
   if (cc) {
@@ -308,11 +323,11 @@ __device__ __forceinline__ void walk_leaf_wave(const DevTree &T, Walk &w, bool p
     cc->plane += cnt;
     cc->inside += __hip_atomic_load(&ins[lane], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
   }
-  const unsigned long long key = __hip_atomic_load(&best[lane], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+  const unsigned long long key = get(&lds.best[lane]);
   bool hit = false;
   if (key != ~0ull) {
     const float t = __uint_as_float((unsigned)(key >> 32));
-    const int k = w.llink + (int)(key & 0xffffffffu);
+    const int k = (int)(key & 0xffffffffu);
     const V3 p = w.o + w.d * t;
     // the record's id is read beside the leaf box, before the box test that decides whether
     // it is needed
