@@ -45,12 +45,12 @@ __global__ __launch_bounds__(kCastBlock, 4) void k_cast(DevTree T, const float *
                                                       const int *__restrict__ exclude, int *__restrict__ out_id,
                                                       float *__restrict__ out_t, float *__restrict__ out_p,
                                                       int *__restrict__ stats, unsigned *__restrict__ work) {
-  extern __shared__ uint32_t stk_base[];
+  extern __shared__ __align__(16) uint2 stk_base[];
   __shared__ LeafLds leaf_all[kWavesPerBlock];
   __shared__ int ins_all[kStats ? kCastBlock : 1];      // per lane: inside tests of its leaf (measurement)
   __shared__ int res_id_all[kWavesPerBlock][kSlots][kWaveChunk];
   __shared__ float res_t_all[kWavesPerBlock][kSlots][kWaveChunk];
-  uint32_t *stk = stk_base + threadIdx.x;
+  uint2 *stk = stk_base + threadIdx.x;
   LeafLds &leaf = leaf_all[threadIdx.x >> 6];
   leaf_lds_init(leaf);
   int *ins = kStats ? ins_all + (threadIdx.x & ~63u) : nullptr;
@@ -164,7 +164,7 @@ __global__ __launch_bounds__(kCastBlock, 4) void k_cast(DevTree T, const float *
           r = slot;
           const float2 *R = (const float2 *)(rays + 6 * (size_t)r);
           const float2 q0 = R[0], q1 = R[1], q2 = R[2];
-          walk_begin(T, w, v3(q0.x, q0.y, q1.x), v3(q1.y, q2.x, q2.y), exclude ? exclude[r] : -1);
+          walk_begin(T, w, v3(q0.x, q0.y, q1.x), v3(q1.y, q2.x, q2.y), exclude ? exclude[r] : -1, stk);
           if (w.state == kWalkDone) finish();
         } else {
           exhausted = true;

@@ -5,13 +5,14 @@
 // skipped if no real point o + d * t with t >= 0 lies within a rounding error of the boxes
 // below it.  The test runs on the scaled distance T = t * max|d.k|, per axis between
 //   near = (min - o) * iv - er    and    far = (max - o) * iv + er,    iv = max|d.k| / d.k,
-// and keeps the child if max(near, 0) <= far over the three axes.
+// and keeps the child if max(near, 0) <= far over the three axes.  A plane's distance is one fused
+// product, plane * iv + c, with cn = -o * iv - er and cf = -o * iv + er formed once per ray.
 //
 // er covers every rounding on the way.  With u = 2^-24, M the largest magnitude of a box
 // coordinate and O the largest of o: o + d t misses p by at most u (2 M + O) per axis; iv (one
-// hardware reciprocal, one product) is off by 3 u relative; the grid plane, its differences and
-// products below by at most u (8 M + 4 O) |iv|.  Together less than u (13 M + 8 O) |iv|, and
-// er = 16 u (M + O) |iv|.
+// hardware reciprocal, one product) is off by 3 u relative; the roundings of cn or cf, of the
+// grid's origin and cell and of the plane come to at most u (6 M + 4 O) |iv|.  Together less than
+// u (11 M + 8 O) |iv|, and er = 16 u (M + O) |iv|.
 // An axis the ray hardly moves along has its |iv| cut to kMaxIv.  Its interval then only has to
 // hold the largest T that a hit can have, at most 1.01 (M + O): er's slack of 3 u (M + O) |iv| is
 // above 190 (M + O) there.
@@ -37,7 +38,7 @@ constexpr float kBoxSlack = 9.5367431640625e-7f;   // 16 * 2^-24
 
 // A ray prepared for the box test.
 struct BoxRay {
-  V3 o, iv, er;
+  V3 iv, cn, cf;
   int canon;     // canonicalOrder (Octree.impl.cuh:181-183): the children are visited in the order canon ^ i
 };
 
@@ -65,7 +66,6 @@ DR_HD bool box_ray(V3 o, V3 d, float reach, BoxRay &r) {
   if (d.y < 0) c += 2;
   if (d.x < 0) c += 4;
   r.canon = c;
-  r.o = o;
   // the reciprocals of very short or long directions are taken of the direction scaled by a power of two
   const float sc = dm < 1e-30f ? 1.2676506e30f : (dm > 1e30f ? 7.8886091e-31f : 1.0f);
   const float ds = dm * sc;
@@ -75,19 +75,19 @@ DR_HD bool box_ray(V3 o, V3 d, float reach, BoxRay &r) {
   const float s = om + reach;
   if (!(s < 1e27f)) ix = iy = iz = 0.0f;
   const float e = s < 1e27f ? kBoxSlack * s : 0.0f;
-  r.er = v3(e * ix, e * iy, e * iz);
   r.iv = v3(d.x < 0 ? -ix : ix, d.y < 0 ? -iy : iy, d.z < 0 ? -iz : iz);
+  const V3 oi = v3(-o.x * r.iv.x, -o.y * r.iv.y, -o.z * r.iv.z);
+  r.cn = v3(oi.x - e * ix, oi.y - e * iy, oi.z - e * iz);
+  r.cf = v3(oi.x + e * ix, oi.y + e * iy, oi.z + e * iz);
   return able;
 }
 
 // The test on one box in full precision (the root's).
 DR_HD bool box_kept(const Box &b, const BoxRay &r) {
-  const float nx = ((r.iv.x < 0 ? b.e.x : b.s.x) - r.o.x) * r.iv.x - r.er.x;
-  const float ny = ((r.iv.y < 0 ? b.e.y : b.s.y) - r.o.y) * r.iv.y - r.er.y;
-  const float nz = ((r.iv.z < 0 ? b.e.z : b.s.z) - r.o.z) * r.iv.z - r.er.z;
-  const float fx = ((r.iv.x < 0 ? b.s.x : b.e.x) - r.o.x) * r.iv.x + r.er.x;
-  const float fy = ((r.iv.y < 0 ? b.s.y : b.e.y) - r.o.y) * r.iv.y + r.er.y;
-  const float fz = ((r.iv.z < 0 ? b.s.z : b.e.z) - r.o.z) * r.iv.z + r.er.z;
+  const bool px = r.iv.x < 0, py = r.iv.y < 0, pz = r.iv.z < 0;
+  const float nx = __builtin_fmaf(px ? b.e.x : b.s.x, r.iv.x, r.cn.x), fx = __builtin_fmaf(px ? b.s.x : b.e.x, r.iv.x, r.cf.x);
+  const float ny = __builtin_fmaf(py ? b.e.y : b.s.y, r.iv.y, r.cn.y), fy = __builtin_fmaf(py ? b.s.y : b.e.y, r.iv.y, r.cf.y);
+  const float nz = __builtin_fmaf(pz ? b.e.z : b.s.z, r.iv.z, r.cn.z), fz = __builtin_fmaf(pz ? b.s.z : b.e.z, r.iv.z, r.cf.z);
   return !(__builtin_fmaxf(max3(nx, ny, nz), 0.0f) > min3(fx, fy, fz));
 }
 
@@ -107,9 +107,9 @@ DR_HD uint32_t group_children(V3 origin, V3 cell, const uint32_t w[12], const Bo
   const uint32_t ny0 = py ? w[8] : w[2], ny1 = py ? w[9] : w[3], fy0 = py ? w[2] : w[8], fy1 = py ? w[3] : w[9];
   const uint32_t nz0 = pz ? w[10] : w[4], nz1 = pz ? w[11] : w[5], fz0 = pz ? w[4] : w[10], fz1 = pz ? w[5] : w[11];
   const float sx = cell.x * r.iv.x, sy = cell.y * r.iv.y, sz = cell.z * r.iv.z;
-  const float bx = (origin.x - r.o.x) * r.iv.x, by = (origin.y - r.o.y) * r.iv.y, bz = (origin.z - r.o.z) * r.iv.z;
-  const float bnx = bx - r.er.x, bny = by - r.er.y, bnz = bz - r.er.z;
-  const float bfx = bx + r.er.x, bfy = by + r.er.y, bfz = bz + r.er.z;
+  const float bnx = __builtin_fmaf(origin.x, r.iv.x, r.cn.x), bfx = __builtin_fmaf(origin.x, r.iv.x, r.cf.x);
+  const float bny = __builtin_fmaf(origin.y, r.iv.y, r.cn.y), bfy = __builtin_fmaf(origin.y, r.iv.y, r.cf.y);
+  const float bnz = __builtin_fmaf(origin.z, r.iv.z, r.cn.z), bfz = __builtin_fmaf(origin.z, r.iv.z, r.cf.z);
   uint32_t skip = 0;
 #ifdef __HIP_DEVICE_COMPILE__
 #pragma unroll

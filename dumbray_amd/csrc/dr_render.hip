@@ -400,7 +400,7 @@ struct RefPath {
 // ------------------------------------------------------------------ forward
 // LDS used by one block render.
 struct BlockLds {
-  uint32_t *stk;        // this lane's first stack word ([word][lane])
+  uint2 *stk;           // this lane's first stack level ([level][lane])
   float *samp_col;      // kBlockPixels * kRoundSamples * 3 sample colours
   float *acc;           // kBlockPixels * 3 pixel sums
   int *next_job;
@@ -512,7 +512,7 @@ __device__ __forceinline__ void render_block(const DevTree &T, const Tables &tb,
               const float zero[3] = {0.0f, 0.0f, 0.0f};
               finish(zero);
             } else {
-              walk_begin(T, w, ps.ray_o(), ps.ray_d(), ps.ray_excl());
+              walk_begin(T, w, ps.ray_o(), ps.ray_d(), ps.ray_excl(), lds.stk);
               if (kStats) { rc->paths++; rc->segments++; }
             }
           } else {
@@ -538,7 +538,7 @@ __device__ __forceinline__ void render_block(const DevTree &T, const Tables &tb,
           if (ps.shade(P, K, tb, w)) {
             finish(ps.color());
           } else {
-            walk_begin(T, w, ps.ray_o(), ps.ray_d(), ps.ray_excl());
+            walk_begin(T, w, ps.ray_o(), ps.ray_d(), ps.ray_excl(), lds.stk);
             if (kStats) { rc->segments++; rc->photons += ps.photon() ? 1 : 0; }
           }
         }
@@ -560,12 +560,12 @@ template <class PathT, bool kStats = false>
 __global__ __launch_bounds__(kRB, kRenderWaves) void k_render(DevTree T, Tables tb, dr_render_params P, FrameK K,
                                                                float *__restrict__ frame, int start_block, int levels,
                                                                unsigned long long *__restrict__ counts = nullptr) {
-  extern __shared__ uint32_t lds[];
+  extern __shared__ __align__(16) uint32_t lds[];
   __shared__ float acc[kBlockPixels * 3];
   __shared__ int next_job;
   __shared__ LeafLds leaf[kRB / 64];
   __shared__ int ins[kStats ? kRB : 1];
-  const BlockLds L = {lds + threadIdx.x, (float *)(lds + levels * kStackWordsPerLevel * kRB), acc, &next_job,
+  const BlockLds L = {(uint2 *)lds + threadIdx.x, (float *)(lds + levels * kStackWordsPerLevel * kRB), acc, &next_job,
                       leaf + (threadIdx.x >> 6), kStats ? ins + (threadIdx.x & ~63u) : nullptr};
   leaf_lds_init(*L.leaf);
   RenderCounters rc;
@@ -613,7 +613,7 @@ __global__ __launch_bounds__(kRB, kRenderWaves) void k_render_stream(DevTree T, 
                                                                       int end_block, int levels,
                                                                       unsigned *__restrict__ work,
                                                                       unsigned long long *__restrict__ counts) {
-  extern __shared__ uint32_t lds[];
+  extern __shared__ __align__(16) uint32_t lds[];
   __shared__ int blocks[kStreamBlockRing];    // (block id + 1) << 8 | stream block number & 255
   __shared__ int px_done[kStreamBlockRing];   // pixels written, cumulative per ring entry
   __shared__ unsigned next_job;
@@ -622,7 +622,7 @@ __global__ __launch_bounds__(kRB, kRenderWaves) void k_render_stream(DevTree T, 
   __shared__ int ins_all[kStats ? kRB : 1];
   const int spp = P.fsaa_x * P.fsaa_y;
   const int nslots = stream_slots(spp);
-  uint32_t *stk = lds + threadIdx.x;
+  uint2 *stk = (uint2 *)lds + threadIdx.x;
   float *samp = (float *)(lds + levels * kStackWordsPerLevel * kRB);   // nslots * spp * 3
   int *owner = (int *)(samp + (size_t)nslots * spp * 3);             // nslots
   int *remaining = owner + nslots;                                    // nslots
@@ -730,7 +730,7 @@ __global__ __launch_bounds__(kRB, kRenderWaves) void k_render_stream(DevTree T, 
             if (PathT::kStreamBlackInUpdate) w.state = kWalkDone;
             else finish(0.0f, 0.0f, 0.0f);
           } else {
-            walk_begin(T, w, ps.ray_o(), ps.ray_d(), ps.ray_excl());
+            walk_begin(T, w, ps.ray_o(), ps.ray_d(), ps.ray_excl(), stk);
             if (kStats) { rc.paths++; rc.segments++; }
           }
         }
@@ -764,7 +764,7 @@ __global__ __launch_bounds__(kRB, kRenderWaves) void k_render_stream(DevTree T, 
           const bool black = PathT::kStreamBlackInUpdate && nopath;
           finish(black ? 0.0f : c0, black ? 0.0f : c1, black ? 0.0f : c2);
         } else {
-          walk_begin(T, w, ps.ray_o(), ps.ray_d(), ps.ray_excl());
+          walk_begin(T, w, ps.ray_o(), ps.ray_d(), ps.ray_excl(), stk);
           if (kStats) { rc.segments++; rc.photons += ps.photon() ? 1 : 0; }
         }
       }
@@ -869,12 +869,12 @@ __global__ __launch_bounds__(kRB, kRenderWaves) void k_backward(DevTree T, const
                                                                  float *__restrict__ vtx_all,
                                                                  int *__restrict__ next_block, int nblocks,
                                                                  int levels, int maxv) {
-  extern __shared__ uint32_t lds[];
+  extern __shared__ __align__(16) uint32_t lds[];
   __shared__ int next_job, cur_block;
   __shared__ LeafLds leaf_all[kRB / 64];
   LeafLds &leaf = leaf_all[threadIdx.x >> 6];
   leaf_lds_init(leaf);
-  uint32_t *stk = lds + threadIdx.x;
+  uint2 *stk = (uint2 *)lds + threadIdx.x;
   float *gacc = (float *)(lds + levels * kStackWordsPerLevel * kRB);   // nmat*3 albedo, then nlights*3 emission
   float *vtx = vtx_all + (size_t)blockIdx.x * maxv * kVtxWords * kRB;
   const int ngrad = 3 * (P.nmat + P.nlights);
@@ -944,7 +944,7 @@ __global__ __launch_bounds__(kRB, kRenderWaves) void k_backward(DevTree T, const
               // SphericalSegmentLense::getPixelColor scales the sample colour by its filter
               for (int c = 0; c < 3; c++)
                 wdl[c] = spw * g[c] * (P.lens == DR_SPHERICAL_SEGMENT_LENS ? P.lens_p[4 + c] : 1.0f);
-              walk_begin(T, w, st.o, st.d, st.restrict_tri);
+              walk_begin(T, w, st.o, st.d, st.restrict_tri, stk);
             }
           } else {
             exhausted = true;
@@ -992,7 +992,7 @@ __global__ __launch_bounds__(kRB, kRenderWaves) void k_backward(DevTree T, const
             photons = true;
           }
           if (photons && !next_photon(P, st)) advance();
-          if (!fin) walk_begin(T, w, st.o, st.d, st.restrict_tri);
+          if (!fin) walk_begin(T, w, st.o, st.d, st.restrict_tri, stk);
         }
         // dL/demission of this update's lit photons
         wave_add3(gacc, lit, lkey, ev);
@@ -1062,12 +1062,12 @@ __global__ void k_zero(int *counter, int n) {
 template <class PathT>
 __global__ __launch_bounds__(kRB, kRenderWaves) void k_batch(const DevRequest *__restrict__ reqs, const int4 *__restrict__ items,
                                                 int nitems, int *__restrict__ counter, int levels, int refill_min) {
-  extern __shared__ uint32_t lds[];
+  extern __shared__ __align__(16) uint32_t lds[];
   __shared__ float acc[kBlockPixels * 3];
   __shared__ int next_job;
   __shared__ int item;
   __shared__ LeafLds leaf[kRB / 64];
-  const BlockLds L = {lds + threadIdx.x, (float *)(lds + levels * kStackWordsPerLevel * kRB), acc, &next_job,
+  const BlockLds L = {(uint2 *)lds + threadIdx.x, (float *)(lds + levels * kStackWordsPerLevel * kRB), acc, &next_job,
                       leaf + (threadIdx.x >> 6), nullptr};
   leaf_lds_init(*L.leaf);
   for (;;) {

@@ -97,10 +97,15 @@ __device__ __forceinline__ bool inside(V3 p, V3 a, V3 b, V3 c, float thr0, float
   return edge_exact(D0, S0, thr0) && edge_exact(D1, S1, thr1) && edge_exact(D2, S2, thr2);
 }
 
-// Traversal stack.  A level holds two words, [2*level][lane] and [2*level+1][lane]:
-//   lo = group << 8 | mask of children still to visit (bit i = child canon ^ i)
-//   hi = first interior child's group << 8 | interior mask (bit k = child k)
-// so popping an interior child needs no memory read.
+// Traversal stack: per level and lane two words, read and written together,
+//   x = group << 8 | mask of children still to visit (bit i = child canon ^ i)
+//   y = first interior child's group << 8 | interior mask (bit k = child k)
+// so popping an interior child needs no memory read.  A level is on the stack only while it has
+// children to visit: the last child's pop takes it off, and a group with none is not pushed, so a
+// step never searches for work and a walk ends in the step that runs out of it.  (With empty
+// levels left on the stack, each pop looped over LDS reads with part of the wave: 1080p 16 spp
+// 19.9 -> 18.4 ms, 99,991 bounce rays 280 -> 245 us, the 256x256 frame 503 -> 462 us with the
+// fused planes of dr_group.h.)
 constexpr int kStackWordsPerLevel = 2;
 
 // The children of group g to visit -> stack entry: those with a non-empty leaf below them that
@@ -137,7 +142,7 @@ struct Walk {
   Hit h;
 };
 
-__device__ __forceinline__ void walk_begin(const DevTree &T, Walk &w, V3 o, V3 d, int exclude) {
+__device__ __forceinline__ void walk_begin(const DevTree &T, Walk &w, V3 o, V3 d, int exclude, uint2 *stk) {
   w.o = o;
   w.d = d;
   w.ex = exclude;
@@ -152,43 +157,34 @@ __device__ __forceinline__ void walk_begin(const DevTree &T, Walk &w, V3 o, V3 d
   }
   const bool alive = box_ray(o, d, T.reach, w.box) && box_kept(root_box(T), w.box);
   w.state = alive ? kWalkTrace : kWalkDone;
+  // a level whose one child is group 0: the root's group is expanded by the walk's first step, with
+  // the expansions of the other lanes, rather than in the divergent code that hands out work
+  w.sp = 0;
+  stk[0] = make_uint2(1u, 1u << w.box.canon);
 }
 
-// Pops one child: expands an interior child, or holds a leaf child as pending;
-// an exhausted stack ends the query with a miss.  A walk's first step (sp == -1 after
-// walk_begin) expands the root's group (group 0) with the expansions of the other lanes,
-// rather than in the divergent code that hands out work.
-__device__ __forceinline__ void walk_step(const DevTree &T, Walk &w, uint32_t *stk, int stride, CastCounters *cc) {
-  int child = 0;                      // group to expand
-  if (w.sp >= 0) {
-    uint32_t f = 0;
-    while (w.sp >= 0) {
-      f = stk[2 * w.sp * stride];
-      if (f & 0xffu) break;
-      --w.sp;
-    }
-    if (w.sp < 0) { w.state = kWalkDone; return; }
-    const int i = __builtin_ctz(f & 0xffu);
-    stk[2 * w.sp * stride] = f & ~(1u << i);
-    const int k = w.box.canon ^ i;
-    const uint32_t hi = stk[(2 * w.sp + 1) * stride];
-    const uint32_t im = hi & 0xffu;
-    if (!((im >> k) & 1u)) {
-      const int *E = (const int *)T.groups + kGroupWords * (size_t)(f >> 8) + kGroupEntry + k;
-      w.leaf = (int)(f >> 8) * 8 + k;
-      w.llink = E[0];
-      w.lcnt = E[1] - E[0];
-      w.state = kWalkLeaf;
-      return;
-    }
-    child = (int)(hi >> 8) + __builtin_popcount(im & ((1u << k) - 1u));
+// Pops one child: expands an interior child, or holds a leaf child as pending.
+__device__ __forceinline__ void walk_step(const DevTree &T, Walk &w, uint2 *stk, int stride, CastCounters *cc) {
+  const uint2 f = stk[w.sp * stride];
+  const int k = w.box.canon ^ __builtin_ctz(f.x);
+  const uint32_t rest = f.x & (f.x - 1);
+  stk[w.sp * stride].x = rest;
+  w.sp -= (rest & 0xffu) ? 0 : 1;
+  const uint32_t im = f.y & 0xffu;
+  if (!((im >> k) & 1u)) {
+    const int *E = (const int *)T.groups + kGroupWords * (size_t)(f.x >> 8) + kGroupEntry + k;
+    w.leaf = (int)(f.x >> 8) * 8 + k;
+    w.llink = E[0];
+    w.lcnt = E[1] - E[0];
+    w.state = kWalkLeaf;
+    return;
   }
-  uint32_t lo2, hi2;
-  group_entry(T.groups, child, w.box, lo2, hi2, cc);
-  ++w.sp;
-  stk[2 * w.sp * stride] = lo2;
-  stk[(2 * w.sp + 1) * stride] = hi2;
+  const int child = (int)(f.y >> 8) + __builtin_popcount(im & ((1u << k) - 1u));
+  uint2 e;
+  group_entry(T.groups, child, w.box, e.x, e.y, cc);
   if (cc) cc->expand++;
+  if (e.x & 0xffu) stk[++w.sp * stride] = e;
+  w.state = w.sp < 0 ? kWalkDone : kWalkTrace;
 }
 
 // Inclusive prefix sum and maximum over the 64 lanes of the wave (every lane active): DPP row
@@ -340,7 +336,7 @@ __device__ __forceinline__ void walk_leaf_wave(const DevTree &T, Walk &w, bool p
     }
   }
   w.hit = hit;
-  w.state = (hit || w.leaf < 0) ? kWalkDone : kWalkTrace;
+  w.state = (hit || w.sp < 0) ? kWalkDone : kWalkTrace;
 }
 
 }  // namespace dr
