@@ -56,6 +56,7 @@ struct Path {
 // A value that is the same in every lane (a function of the kernel's parameters), moved to
 // a scalar register.  Call with every lane that holds it agreeing on it.
 __device__ __forceinline__ float uni(float v) { return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v))); }
+__device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
 __device__ __forceinline__ uint32_t uni(uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); }
 __device__ __forceinline__ UDiv uni(UDiv D) { return {uni(D.d), uni(D.m)}; }
 __device__ __forceinline__ UDiv udiv_uniform(uint32_t d) { return uni(make_udiv(d)); }
@@ -81,22 +82,45 @@ __device__ __forceinline__ FrameK frame_k_uniform(const dr_render_params &P) {
   return K;
 }
 
-// Common job start: camera ray of sample `s` of local pixel `lp`.  Returns false
-// (and leaves the lane idle) for pixels outside the image.
-__device__ __forceinline__ bool start_path(const dr_render_params &P, const FrameK &K, int block, int lp, int s,
-                                           uint32_t samp0, Path &st) {
+// The first ray of a path: sample `samp` of pixel `pix`, kNoPixel for a pixel outside the image.
+constexpr uint32_t kNoPixel = 0xffffffffu;
+struct PathStart {
+  uint32_t pix, samp;
+  V3 o, d;
+};
+
+// Job start: camera ray of sample `s` of pixel `lp` of block `block`.
+__device__ __forceinline__ PathStart path_start(const dr_render_params &P, const FrameK &K, int block, int lp, int s,
+                                                uint32_t samp0) {
+  PathStart ps;
   int x, y;
-  if (!block_pixel(K, P.width, P.height, block, lp, x, y)) return false;
-  st.pix = (uint32_t)y * (uint32_t)P.width + (uint32_t)x;
-  st.samp = samp0 + (uint32_t)s;
+  ps.pix = kNoPixel;
+  ps.samp = samp0 + (uint32_t)s;
+  ps.o = ps.d = v3(0.0f, 0.0f, 0.0f);
+  if (!block_pixel(K, P.width, P.height, block, lp, x, y)) return ps;
+  ps.pix = (uint32_t)y * (uint32_t)P.width + (uint32_t)x;
   const int i = (int)udiv((uint32_t)s, K.fy), j = s - i * P.fsaa_y;
   float u[4];
-  rng4(P, st.pix, st.samp, 0, 0, u);
-  camera_ray(P, K, x, y, i, j, u[0], u[1], u[2], u[3], st.o, st.d);
+  rng4(P, ps.pix, ps.samp, 0, 0, u);
+  camera_ray(P, K, x, y, i, j, u[0], u[1], u[2], u[3], ps.o, ps.d);
+  return ps;
+}
+__device__ __forceinline__ void begin_path(Path &st, const PathStart &s) {
+  st.pix = s.pix;
+  st.samp = s.samp;
+  st.o = s.o;
+  st.d = s.d;
   st.layer = 0;
   st.phase = 0;
   st.restrict_tri = -1;
   for (int c = 0; c < 3; c++) { st.beta[c] = 1.0f; st.L[c] = 0.0f; }
+}
+// Starts the job's path, or returns false (and leaves the lane idle) for a pixel outside the image.
+__device__ __forceinline__ bool start_path(const dr_render_params &P, const FrameK &K, int block, int lp, int s,
+                                           uint32_t samp0, Path &st) {
+  const PathStart ps = path_start(P, K, block, lp, s, samp0);
+  if (ps.pix == kNoPixel) return false;
+  begin_path(st, ps);
   return true;
 }
 
@@ -154,21 +178,20 @@ struct Tables {
 
 // Path updates of the benchmark plugins (DR_PLUGINS_BENCHMARK).
 struct BenchPath {
-  // k_render_stream: a job outside the image is written at once, and the job's block is read
-  // back from the block ring when its pixel is written (29.5 ms at 1080p 16 spp, against
-  // 30.8 ms with the other choices, which suit RefPath)
-  static constexpr bool kStreamBlackInUpdate = false, kStreamBlockInRegister = false;
-  // Finished casts that trigger the path updates and idle lanes that trigger new path jobs, in
-  // render_block and in k_render_stream (1080p 16 spp, split 8 / depth 24: 27.2 ms at 32 / 8,
-  // 26.4-26.5 ms at 24 or 20 / 4 in the streamed kernel; 0.67 ms at 32 / 8 against 0.70 ms at
-  // 24 / 4 for the 256x256 frame in render_block)
-  static constexpr int kShadeMin = 32, kRefillMin = 8, kStreamShadeMin = 24, kStreamRefillMin = 4;
+  // render_block: finished casts that trigger the path updates, idle lanes that trigger new path
+  // jobs.  k_render_stream: finished casts of a wave with all lanes busy that trigger the path
+  // updates (in proportion with fewer lanes; 1080p 16 spp 16.4 / 15.9 / 15.8 ms at 16 / 24 / 32),
+  // idle lanes that pop the queue (1, 4, 10: 16.2, 15.9, 15.9 ms)
+  static constexpr int kShadeMin = 32, kRefillMin = 8, kStreamShadeMin = 32, kStreamRefillMin = 4;
   static constexpr bool kStreamFrameInKernel = false;
   Path st;
   __device__ __forceinline__ bool start(const dr_render_params &P, const FrameK &K, int block, int lp, int s,
                                         uint32_t samp0) {
     return start_path(P, K, block, lp, s, samp0, st);
   }
+  __device__ __forceinline__ void begin(const PathStart &s) { begin_path(st, s); }
+  __device__ __forceinline__ uint32_t pixel() const { return st.pix; }
+  __device__ __forceinline__ uint32_t sample() const { return st.samp; }
   __device__ __forceinline__ V3 ray_o() const { return st.o; }
   __device__ __forceinline__ V3 ray_d() const { return st.d; }
   __device__ __forceinline__ int ray_excl() const { return st.restrict_tri; }
@@ -219,12 +242,7 @@ struct BenchPath {
 // sample are computed again where they are used; both are functions of the vertex and
 // of counter-based random numbers, so the order of evaluation does not change them.
 struct RefPath {
-  // k_render_stream: a job outside the image goes through the path-update phase, and the
-  // job's block stays in a register (example scene 8.5 ms, against 9.4-9.9 ms otherwise:
-  // fewer spilled registers)
-  static constexpr bool kStreamBlackInUpdate = true, kStreamBlockInRegister = true;
-  // the same thresholds (example scene, streamed: 8.12 ms at 32 / 8, 8.01 at 44 / 8, 7.94 at
-  // 44 / 4, 9.37 at 64 / 8)
+  // the same thresholds (reference plugins at 1080p, 1 spp: 3.23 / 3.12 / 3.26 ms at 32 / 44 / 52)
   static constexpr int kShadeMin = 32, kRefillMin = 8, kStreamShadeMin = 44, kStreamRefillMin = 4;
   static constexpr bool kStreamFrameInKernel = true;
   uint32_t pix, samp;
@@ -239,20 +257,23 @@ struct RefPath {
 
   __device__ __forceinline__ bool start(const dr_render_params &P, const FrameK &K, int block, int lp, int s,
                                         uint32_t samp0) {
-    int x, y;
-    if (!block_pixel(K, P.width, P.height, block, lp, x, y)) return false;
-    pix = (uint32_t)y * (uint32_t)P.width + (uint32_t)x;
-    samp = samp0 + (uint32_t)s;
-    const int i = (int)udiv((uint32_t)s, K.fy), j = s - i * P.fsaa_y;
-    float u[4];
-    rng4(P, pix, samp, 0, 0, u);
-    camera_ray(P, K, x, y, i, j, u[0], u[1], u[2], u[3], o, d);
+    const PathStart ps = path_start(P, K, block, lp, s, samp0);
+    if (ps.pix == kNoPixel) return false;
+    begin(ps);
+    return true;
+  }
+  __device__ __forceinline__ void begin(const PathStart &s) {
+    pix = s.pix;
+    samp = s.samp;
+    o = s.o;
+    d = s.d;
     layer = 0;
     phase = 0;
     excl = -1;
     for (int c = 0; c < 3; c++) { beta[c] = 1.0f; L[c] = 0.0f; }
-    return true;
   }
+  __device__ __forceinline__ uint32_t pixel() const { return pix; }
+  __device__ __forceinline__ uint32_t sample() const { return samp; }
   __device__ __forceinline__ V3 ray_o() const { return o; }
   __device__ __forceinline__ V3 ray_d() const { return d; }
   __device__ __forceinline__ int ray_excl() const { return excl; }
@@ -438,12 +459,10 @@ __device__ __forceinline__ void flush_counters(const RenderCounters &c, unsigned
   }
 }
 
-// Framebuffer pixel `lp` of block `block`: the colour of this iteration, set (iteration 1)
-// or blended with weight 1/iteration (DumbRenderer.cu:64, BlockBasedFrameBuffer.impl.cuh:125-156).
-__device__ __forceinline__ void store_pixel(const dr_render_params &P, const FrameK &K, float *__restrict__ frame,
-                                            int block, int lp, const float a[3]) {
-  int x, y;
-  if (!block_pixel(K, P.width, P.height, block, lp, x, y)) return;
+// Framebuffer pixel `lp` of block `block` (inside the image): the colour of this iteration, set
+// (iteration 1) or blended with weight 1/iteration (DumbRenderer.cu:64, BlockBasedFrameBuffer.impl.cuh:125-156).
+__device__ __forceinline__ void store_pixel(const FrameK &K, float *__restrict__ frame, int block, int lp,
+                                            const float a[3]) {
   float4 *f = (float4 *)frame + (size_t)kBlockPixels * block + lp;
   const float4 col = make_float4(a[0], a[1], a[2], 1.0f);
   const float amount = K.amount;
@@ -551,7 +570,9 @@ __device__ __forceinline__ void render_block(const DevTree &T, const Tables &tb,
     }
     __syncthreads();
   }
-  if (threadIdx.x < kBlockPixels) store_pixel(P, K, frame, block, threadIdx.x, lds.acc + 3 * threadIdx.x);
+  int x, y;
+  if (threadIdx.x < kBlockPixels && block_pixel(K, P.width, P.height, block, threadIdx.x, x, y))
+    store_pixel(K, frame, block, threadIdx.x, lds.acc + 3 * threadIdx.x);
   __syncthreads();
 }
 
@@ -575,200 +596,255 @@ __global__ __launch_bounds__(kRB, kRenderWaves) void k_render(DevTree T, Tables 
 
 // ------------------------------------------------------------------ streamed blocks
 // k_render_stream: the same path loop with no barrier between framebuffer blocks.  A
-// workgroup is persistent and takes blocks from a counter in global memory; its lanes take
-// path jobs from one stream that runs through those blocks in turn (job q: pixel q / spp of
-// the stream, sample q % spp; stream pixel u is pixel u % 128 of the workgroup's block
-// number u / 128), so lanes whose paths end near the end of a block start the next block's
-// paths instead of waiting for the block's longest path.  In the one-block-per-workgroup
-// kernel those waits took 21% of the path loop's cycles and the barrier after it 7% at
-// 1080p, 16 spp.
-//   * Sample colours are staged in a ring of `nslots` pixel slots of spp samples
-//     (nslots * spp <= kStreamSamples).  Stream pixel u uses slot u % nslots and may start
-//     once the slot's owner is u, i.e. once pixel u - nslots has been written out.
-//   * The lane that finishes a pixel's last sample sums its spp staged colours in sample
-//     order, as render_block does, writes the pixel, and hands the slot to u + nslots.
+// workgroup is persistent and takes tiles (2^tile_shift pixels of a block, 128 at most) from a
+// counter in global memory; its waves take path jobs from one stream that runs through those
+// tiles in turn (job q: pixel q / spp of the stream, sample q % spp; stream pixel u is pixel
+// u % 2^tile_shift of the workgroup's tile number u >> tile_shift), so lanes whose paths end near
+// the end of a tile start the next tile's paths instead of waiting for the tile's longest path.
+//   * A wave takes `chunk` jobs at a time (64 at most, all of one tile) and forms their camera rays
+//     with as many lanes, into a queue in LDS; lanes that become idle pop the next entry.
+//   * With one sample per pixel a finished path writes its pixel.
+//   * With more, sample colours are staged in a ring of nslots = 2^slot_shift pixel slots of spp
+//     samples.  Stream pixel u uses slot u % nslots and may start once that is in its turn u / nslots,
+//     i.e. once pixel u - nslots has been written out.  A slot's word holds its turn << 9 | samples to
+//     come.  The lane that finishes a pixel's last sample sums its spp staged colours in sample
+//     order, as render_block does, writes the pixel, and begins the slot's next turn.
 //     Frames are therefore bit-identical to render_block's.
-//   * Block number k of the workgroup is fetched by the lane that takes its first job, and
-//     only once block k - 1 has been fetched, so block ids rise with k and the blocks past
+//   * Tile number k of the workgroup is fetched by the wave that forms its first jobs, and
+//     only once tile k - 1 has been fetched, so tile ids rise with k and the tiles past
 //     the launch's range form a suffix of the stream.  The ids sit in a ring of
-//     kStreamBlockRing entries; a job of block number k starts only once every pixel of block
-//     number k - kStreamBlockRing has been written (pixels written per ring entry are
+//     kStreamRing entries; a job of tile number k is formed only once every pixel of tile
+//     number k - kStreamRing has been written (pixels written per ring entry are
 //     counted cumulatively), so no job still needs an entry when it is reused.
-//   * Progress: the oldest pixel not yet written can always start (its slot's previous
-//     owner is written, its block's ring entry and the entry before it are fetched), and
-//     jobs are taken in stream order, so its jobs are held by lanes; lanes whose job must
-//     wait keep retrying while the other lanes work.
+//   * Progress: jobs are formed and popped in order within a wave.  Every job before the oldest one
+//     not yet started is held by a lane, and a lane's path always ends; so its tile's ring entry
+//     and its pixel's slot become free, the entries before it in its queue have been popped, and
+//     its wave pops it once lanes of the wave are idle.
 constexpr int kStreamSamples = 2048;      // staged sample colours per workgroup
-constexpr int kStreamMaxSlots = 1024;     // pixel slots at low sample counts
-constexpr int kStreamBlockRing = 16;
+constexpr int kStreamRing = 64;
 constexpr int kStreamMaxSpp = 256;        // higher sample counts take render_block's rounds
 
-__host__ __device__ constexpr int stream_slots(int spp) {
-  return (kStreamSamples / spp) < kStreamMaxSlots ? (kStreamSamples / spp) : kStreamMaxSlots;
+// log2 of the pixel slots for `samples` staged colours, -1 for no staging
+constexpr int stream_slot_shift(int spp, int samples) {
+  int n = 0;
+  while ((2 << n) * spp <= samples) n++;
+  return spp == 1 ? -1 : n;
+}
+// LDS words of one wave's queue of path starts: direction, pixel, stream
+// pixel, and the origin for lenses that sample it.
+__host__ __device__ constexpr int stream_queue_words(bool origins) { return 64 * (origins ? 8 : 5); }
+constexpr size_t stream_lds(int levels, int spp, int slot_shift, bool origins) {
+  const size_t nslots = slot_shift < 0 ? 0 : (size_t)1 << slot_shift;
+  return ((size_t)levels * kStackWordsPerLevel * kRB + nslots * (3 * spp + 1) +
+          (kRB / 64) * (size_t)stream_queue_words(origins)) * 4;
 }
 
 template <class PathT, bool kStats>
 __global__ __launch_bounds__(kRB, kRenderWaves) void k_render_stream(DevTree T, Tables tb, dr_render_params P,
                                                                       FrameK K, float *__restrict__ frame, int start_block,
-                                                                      int end_block, int levels,
+                                                                      int ntiles, int tile_shift, int chunk, int slot_shift,
+                                                                      int levels,
                                                                       unsigned *__restrict__ work,
                                                                       unsigned long long *__restrict__ counts) {
   extern __shared__ __align__(16) uint32_t lds[];
-  __shared__ int blocks[kStreamBlockRing];    // (block id + 1) << 8 | stream block number & 255
-  __shared__ int px_done[kStreamBlockRing];   // pixels written, cumulative per ring entry
+  __shared__ int tiles[kStreamRing];          // (tile id + 1) << 8 | tile number & 255
+  __shared__ int px_done[kStreamRing];        // pixels written, cumulative per ring entry
   __shared__ unsigned next_job;
-  __shared__ int end_k;                       // first stream block number past the range
+  __shared__ int end_k;                       // first tile number past the range
   __shared__ LeafLds leaf_all[kRB / 64];
   __shared__ int ins_all[kStats ? kRB : 1];
   const int spp = P.fsaa_x * P.fsaa_y;
-  const int nslots = stream_slots(spp);
+  const int nslots = slot_shift < 0 ? 0 : 1 << slot_shift;
+  const bool origins = P.lens == DR_SPHERICAL_SEGMENT_LENS;
   uint2 *stk = (uint2 *)lds + threadIdx.x;
   float *samp = (float *)(lds + levels * kStackWordsPerLevel * kRB);   // nslots * spp * 3
-  int *owner = (int *)(samp + (size_t)nslots * spp * 3);             // nslots
-  int *remaining = owner + nslots;                                    // nslots
+  int *turn = (int *)(samp + (size_t)nslots * spp * 3);              // nslots
+  float *queue = (float *)(turn + nslots) + (threadIdx.x >> 6) * stream_queue_words(origins);   // [word][entry]
   LeafLds &leaf = leaf_all[threadIdx.x >> 6];
   leaf_lds_init(leaf);
   int *ins = kStats ? ins_all + (threadIdx.x & ~63u) : nullptr;
-  for (int t = threadIdx.x; t < nslots; t += kRB) { owner[t] = t; remaining[t] = spp; }
-  for (int t = threadIdx.x; t < kStreamBlockRing; t += kRB) { blocks[t] = 0; px_done[t] = 0; }
+  for (int t = threadIdx.x; t < nslots; t += kRB) turn[t] = spp;
+  for (int t = threadIdx.x; t < kStreamRing; t += kRB) { tiles[t] = 0; px_done[t] = 0; }
   if (threadIdx.x == 0) { next_job = 0; end_k = 0x7fffffff; }
   __syncthreads();
 
   RenderCounters rc;
   CastCounters *cc = kStats ? &rc.cast : nullptr;
-  const int nrange = end_block - start_block;
   const uint32_t samp0 = (uint32_t)(P.iteration > 1 ? P.iteration - 1 : 0) * (uint32_t)spp;
   const float spw = uni(1.0f / (((float)P.fsaa_x) * ((float)P.fsaa_y)));
   if constexpr (PathT::kStreamFrameInKernel) K = frame_k_uniform(P);
-  const UDiv Dspp = udiv_uniform((uint32_t)spp), Dslots = udiv_uniform((uint32_t)nslots);
+  const UDiv Dspp = udiv_uniform((uint32_t)spp);
   const bool clip = P.cull_backfaces != 0;
   const int lane = (int)__lane_id();
   const uint64_t below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
   PathT ps;
   Walk w;
   w.state = kWalkDone;
-  int q = -1;             // stream job of this lane, or -1
-  bool live = false;      // the job has started
-  bool exhausted = false; // the stream has ended for this lane
-  bool nopath = false;    // the job's pixel is outside the image
-  int blk = 0;            // the job's block (PathT::kStreamBlockInRegister)
-  // stages this lane's sample colour (the lens filter applied: getPixelColor, see
-  // render_block); the lane that completes the pixel writes it out
-  auto finish = [&](float l0, float l1, float l2) {
-    const int u = (int)udiv((uint32_t)q, Dspp), s = q - u * spp, slot = u - (int)udiv((uint32_t)u, Dslots) * nslots;
-    float *dst = samp + 3 * ((size_t)slot * spp + s);
-    dst[0] = l0;
-    dst[1] = l1;
-    dst[2] = l2;
-    __threadfence_block();
-    if (atomicSub(&remaining[slot], 1) == 1) {
-      float a[3] = {0.0f, 0.0f, 0.0f};
-      const float *src = samp + 3 * (size_t)slot * spp;
-      for (int k = 0; k < spp; k++)
-        for (int c = 0; c < 3; c++) a[c] += src[3 * k + c] * spw;
-      // the job's block (its ring entry stays until every pixel of the block is written)
-      const int b = PathT::kStreamBlockInRegister
-                        ? blk
-                        : (*(volatile int *)&blocks[(u / kBlockPixels) & (kStreamBlockRing - 1)] >> 8) - 1;
-      store_pixel(P, K, frame, b, u % kBlockPixels, a);
-      remaining[slot] = spp;
-      atomicAdd(&px_done[(u / kBlockPixels) & (kStreamBlockRing - 1)], 1);
-      __threadfence_block();
-      owner[slot] = u + nslots;
-    }
-    q = -1;
-    live = false;
+  int u = 0;              // stream pixel of this lane's path
+  bool live = false;      // the lane has a path
+  // the wave's queue (wave-uniform): entries [qpos, qlen) of the jobs from qbase on
+  unsigned qbase = 0;
+  int qpos = 0, qlen = 0;
+  bool taken = false;     // the jobs from qbase on are this wave's and not formed yet
+  bool ended = false;     // the stream has no more jobs for this wave
+  // pixel p of tile e of the ring: its block and place in it
+  auto tile_block = [&](int e) { return start_block + (((e >> 8) - 1) >> (7 - tile_shift)); };
+  auto tile_pixel = [&](int e, int p) {
+    return ((((e >> 8) - 1) & ((1 << (7 - tile_shift)) - 1)) << tile_shift) + (p & ((1 << tile_shift) - 1));
+  };
+  auto pixel_written = [&](const float a[3]) {
+    const int kk = (u >> tile_shift) & (kStreamRing - 1);
+    // (the tile's ring entry stays until every pixel of the tile is written)
+    const int e = *(volatile int *)&tiles[kk];
+    if (ps.pixel() != kNoPixel) store_pixel(K, frame, tile_block(e), tile_pixel(e, u), a);
+    atomicAdd(&px_done[kk], 1);
   };
   for (;;) {
-    // ---- idle lanes take the next jobs of the stream
-    const bool want = (q < 0) && !exhausted;
-    const uint64_t wmask = __ballot(want);
-    if (wmask && (__popcll(wmask) >= PathT::kStreamRefillMin || __ballot(live) == 0)) {
-      const int leader = __ffsll((unsigned long long)wmask) - 1;
-      unsigned base = 0;
-      if (lane == leader) base = atomicAdd(&next_job, (unsigned)__popcll(wmask));
-      base = __shfl(base, leader);
-      if (want) q = (int)(base + (unsigned)__popcll(wmask & below));
-    }
-    // ---- jobs taken but not started: their block and their pixel slot
-    if (q >= 0 && !live) {
-      const int u = (int)udiv((uint32_t)q, Dspp), s = q - u * spp;
-      const int k = u / kBlockPixels;
-      const int kk = k & (kStreamBlockRing - 1);
-      if (k >= *(volatile int *)&end_k) {
-        q = -1;
-        exhausted = true;
-      } else if (*(volatile int *)&px_done[kk] >= kBlockPixels * (k / kStreamBlockRing)) {
-        // (block number k - kStreamBlockRing is written: the ring entry is this block's)
-        int e = *(volatile int *)&blocks[kk];
-        if ((e & 0xff) != (k & 0xff) || e == 0) {
-          // the first job of block number k fetches its id once k - 1 has one
-          const int prev = k > 0 ? *(volatile int *)&blocks[(k - 1) & (kStreamBlockRing - 1)] : 0;
-          const bool prev_ok = k == 0 || (prev != 0 && (prev & 0xff) == ((k - 1) & 0xff));
-          if (q == k * kBlockPixels * spp && prev_ok) {
-            const int id = (int)atomicAdd(work, 1u);
-            if (id >= nrange) {
-              atomicMin(&end_k, k);
-              q = -1;
-              exhausted = true;
-              e = 0;
-            } else {
-              e = ((start_block + id + 1) << 8) | (k & 0xff);
-              blocks[kk] = e;
+    // ---- path updates of the finished casts, batched.  The thresholds here and of the leaf tests are
+    // shares of the lanes that have a path: a wave near the end of the frame, with few, would otherwise
+    // hold each finished cast until its slowest ray (517x389 at 1 spp: 1067 -> 968 us)
+    const uint64_t dm = __ballot(live && w.state == kWalkDone);
+    bool fresh = false;   // the lane has a new ray
+    const uint64_t lm = __ballot(live);
+    if (dm && __popcll(dm) * 64 >= __popcll(lm) * PathT::kStreamShadeMin) {
+      if (live && w.state == kWalkDone) {
+        const bool outside = ps.pixel() == kNoPixel;
+        if (outside || ps.shade(P, K, tb, w)) {
+          // stages the sample's colour (the lens filter applied: getPixelColor, see render_block; a job
+          // outside the image stages black); the lane that completes the pixel writes it out
+          const float *col = ps.color();
+          float c[3] = {col[0], col[1], col[2]};
+          if (origins)
+            for (int k = 0; k < 3; k++) c[k] = c[k] * P.lens_p[4 + k];
+          if (outside) c[0] = c[1] = c[2] = 0.0f;
+          if (nslots == 0) {
+            const float a[3] = {0.0f + c[0] * spw, 0.0f + c[1] * spw, 0.0f + c[2] * spw};
+            pixel_written(a);
+          } else {
+            const int slot = u & (nslots - 1);
+            float *src = samp + 3 * (size_t)slot * spp;
+            float *dst = src + 3 * (int)(ps.sample() - samp0);
+            dst[0] = c[0];
+            dst[1] = c[1];
+            dst[2] = c[2];
+            __threadfence_block();
+            const int left = atomicSub(&turn[slot], 1);
+            if ((left & 511) == 1) {
+              float a[3] = {0.0f, 0.0f, 0.0f};
+              for (int k = 0; k < spp; k++)
+                for (int j = 0; j < 3; j++) a[j] += src[3 * k + j] * spw;
+              pixel_written(a);
+              __threadfence_block();
+              *(volatile int *)&turn[slot] = (((left >> 9) + 1) << 9) | spp;
             }
-          } else {
-            e = 0;
           }
-        }
-        if (e != 0 && (e & 0xff) == (k & 0xff) &&
-            *(volatile int *)&owner[u - (int)udiv((uint32_t)u, Dslots) * nslots] == u) {
-          live = true;
-          if (PathT::kStreamBlockInRegister) blk = (e >> 8) - 1;
-          nopath = !ps.start(P, K, (e >> 8) - 1, u % kBlockPixels, s, samp0);
-          if (nopath) {
-            // a pixel outside the image: a black sample
-            if (PathT::kStreamBlackInUpdate) w.state = kWalkDone;
-            else finish(0.0f, 0.0f, 0.0f);
-          } else {
-            walk_begin(T, w, ps.ray_o(), ps.ray_d(), ps.ray_excl(), stk);
-            if (kStats) { rc.paths++; rc.segments++; }
-          }
+          live = false;
+        } else {
+          fresh = true;
+          if (kStats) { rc.segments++; rc.photons += ps.photon() ? 1 : 0; }
         }
       }
     }
+    // ---- the queue is empty: the next jobs of the stream, and their camera rays
+    if (qpos == qlen && !ended) {
+      if (!taken) {
+        unsigned q = 0;
+        if (lane == 0) q = atomicAdd(&next_job, (unsigned)chunk);
+        qbase = (unsigned)__builtin_amdgcn_readfirstlane((int)q);
+        taken = true;
+      }
+      // the tile of these jobs (wave-uniform); its first jobs' wave fetches its id once the tile before has one
+      const int k = uni((int)udiv(qbase, Dspp)) >> tile_shift;
+      const int kk = k & (kStreamRing - 1);
+      bool past = k >= uni(*(volatile int *)&end_k);
+      int e = 0;
+      if (!past && uni(*(volatile int *)&px_done[kk]) >= (k / kStreamRing) << tile_shift) {   // the ring entry is tile k's
+        e = uni(*(volatile int *)&tiles[kk]);
+        if ((e & 0xff) != (k & 0xff)) e = 0;
+        if (e == 0 && qbase == (unsigned)((k << tile_shift) * spp)) {
+          const int prev = k > 0 ? uni(*(volatile int *)&tiles[(k - 1) & (kStreamRing - 1)]) : 0;
+          if (k == 0 || (prev != 0 && (prev & 0xff) == ((k - 1) & 0xff))) {
+            int id = 0;
+            if (lane == 0) id = (int)atomicAdd(work, 1u);
+            id = __builtin_amdgcn_readfirstlane(id);
+            if (id >= ntiles) {
+              if (lane == 0) atomicMin(&end_k, k);
+              past = true;
+            } else {
+              e = ((id + 1) << 8) | (k & 0xff);
+              if (lane == 0) *(volatile int *)&tiles[kk] = e;
+            }
+          }
+        }
+      }
+      ended = past;
+      if (e != 0) {
+        taken = false;
+        qpos = 0;
+        qlen = chunk;
+        if (lane < chunk) {
+          const int q = (int)qbase + lane;
+          const int uq = (int)udiv((uint32_t)q, Dspp), s = q - uq * spp;
+          const PathStart st = path_start(P, K, tile_block(e), tile_pixel(e, uq), s, samp0);
+          queue[0 * 64 + lane] = st.d.x;
+          queue[1 * 64 + lane] = st.d.y;
+          queue[2 * 64 + lane] = st.d.z;
+          queue[3 * 64 + lane] = __int_as_float((int)st.pix);
+          queue[4 * 64 + lane] = __int_as_float(uq);
+          if (origins) {
+            queue[5 * 64 + lane] = st.o.x;
+            queue[6 * 64 + lane] = st.o.y;
+            queue[7 * 64 + lane] = st.o.z;
+          }
+        }
+        __threadfence_block();
+      }
+    }
+    // ---- idle lanes pop the next entries whose pixel slot is free
+    const uint64_t idle = __ballot(!live);
+    if (qpos < qlen && idle && (__popcll(idle) >= PathT::kStreamRefillMin || idle == ~0ull)) {
+      const int entry = qpos + __popcll(idle & below);
+      const bool some = !live && entry < qlen;
+      int uq = 0;
+      bool free = false;
+      if (some) {
+        uq = __float_as_int(queue[4 * 64 + entry]);
+        // (turns are compared in the 23 bits a slot's word keeps)
+        free = nslots == 0 || (((*(volatile int *)&turn[uq & (nslots - 1)] >> 9) ^ (uq >> slot_shift)) & 0x7fffff) == 0;
+      }
+      const uint64_t stuck = __ballot(some && !free);
+      const bool take = some && (stuck == 0 || lane < __ffsll((unsigned long long)stuck) - 1);
+      qpos += __popcll(__ballot(take));
+      if (take) {
+        PathStart st;
+        st.d = v3(queue[0 * 64 + entry], queue[1 * 64 + entry], queue[2 * 64 + entry]);
+        st.pix = (uint32_t)__float_as_int(queue[3 * 64 + entry]);
+        st.samp = samp0 + (qbase + (uint32_t)entry - (uint32_t)uq * (uint32_t)spp);
+        st.o = v3(P.cam[0], P.cam[1], P.cam[2]);
+        if (origins) st.o = v3(queue[5 * 64 + entry], queue[6 * 64 + entry], queue[7 * 64 + entry]);
+        u = uq;
+        live = true;
+        ps.begin(st);
+        fresh = true;
+        if (kStats && st.pix != kNoPixel) { rc.paths++; rc.segments++; }
+      }
+    }
     if (__ballot(live) == 0) {
-      if (__ballot(q >= 0 || !exhausted) == 0) break;
-      if (__ballot(q >= 0) != 0) __builtin_amdgcn_s_sleep(1);   // jobs waiting for a slot or a block id
+      if (qpos == qlen && ended) break;
+      __builtin_amdgcn_s_sleep(1);   // the next jobs wait for a slot or a tile id
       continue;
+    }
+    if (fresh) {
+      walk_begin(T, w, ps.ray_o(), ps.ray_d(), ps.ray_excl(), stk);
+      if (ps.pixel() == kNoPixel) w.state = kWalkDone;
     }
     // ---- one traversal step of every ray in flight
     if (live && w.state == kWalkTrace) walk_step(T, w, stk, kRB, cc);
     // ---- leaf tests, batched
     const bool pend = live && w.state == kWalkLeaf;
     const uint64_t pm = __ballot(pend);
-    if (pm && (__popcll(pm) >= kLeafMin || __ballot(live && w.state == kWalkTrace) == 0))
+    if (pm && (__popcll(pm) * (64 / kLeafMin) >= __popcll(__ballot(live)) || __ballot(live && w.state == kWalkTrace) == 0))
       walk_leaf_wave(T, w, pend, clip, leaf, ins, cc);
-    // ---- path updates of the finished casts, batched
-    const uint64_t dm = __ballot(live && w.state == kWalkDone);
-    if (dm && (__popcll(dm) >= PathT::kStreamShadeMin || __ballot(live && w.state != kWalkDone) == 0)) {
-      if (live && w.state == kWalkDone) {
-        if ((PathT::kStreamBlackInUpdate && nopath) || ps.shade(P, K, tb, w)) {
-          const float *col = ps.color();
-          float c0 = col[0], c1 = col[1], c2 = col[2];
-          if (P.lens == DR_SPHERICAL_SEGMENT_LENS) {
-            c0 = c0 * P.lens_p[4];
-            c1 = c1 * P.lens_p[5];
-            c2 = c2 * P.lens_p[6];
-          }
-          // (a job outside the image stages black; its pixel is never written)
-          const bool black = PathT::kStreamBlackInUpdate && nopath;
-          finish(black ? 0.0f : c0, black ? 0.0f : c1, black ? 0.0f : c2);
-        } else {
-          walk_begin(T, w, ps.ray_o(), ps.ray_d(), ps.ray_excl(), stk);
-          if (kStats) { rc.segments++; rc.photons += ps.photon() ? 1 : 0; }
-        }
-      }
-    }
   }
   if (kStats) flush_counters(rc, counts);
   // ---- the last wave out resets the block counter for the next launch
@@ -1127,28 +1203,52 @@ static int launch_render(dr_scene s, const dr_render_params *p, float *frame, in
   const Tables tb = tables_of(s, p);
   const bool ref = p->plugins == DR_PLUGINS_REFERENCE;
   const int spp = p->fsaa_x * p->fsaa_y;
-  // streamed blocks (k_render_stream) when each workgroup gets at least two blocks, unless the
-  // sample count or the stream length is too large; one block per workgroup otherwise
+  // streamed tiles (k_render_stream) unless the sample count or the stream length is too large; one
+  // block per workgroup otherwise
   const long long nrange = end_block - start_block;
-  if (spp <= kStreamMaxSpp && (nrange + 1) * kBlockPixels * spp < (1ll << 31) && end_block < (1 << 23)) {
-    const int nslots = stream_slots(spp);
-    const size_t lds_s =
-        ((size_t)levels * kStackWordsPerLevel * kRB + (size_t)nslots * spp * 3 + 2 * (size_t)nslots) * 4;
+  if (spp <= kStreamMaxSpp && (nrange + 4) * kBlockPixels * spp < (1ll << 31) && end_block < (1 << 23)) {
+    const bool origins = p->lens == DR_SPHERICAL_SEGMENT_LENS;
     auto kern = counts ? (ref ? k_render_stream<RefPath, true> : k_render_stream<BenchPath, true>)
                        : (ref ? k_render_stream<RefPath, false> : k_render_stream<BenchPath, false>);
+    int slot_shift = stream_slot_shift(spp, kStreamSamples), per_cu = 0;
+    size_t lds_s = stream_lds(levels, spp, slot_shift, origins);
     if (lds_s > 64 * 1024)
       DR_HIP_CHECK(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_s));
-    int per_cu = 0;
     DR_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, kRB, lds_s));
-    const long long resident = (long long)s->num_cu * std::max(per_cu, 1);
-    const int groups = (int)std::min<long long>(nrange, resident);
-    if (nrange >= 2 * resident) {
-      unsigned *work = (unsigned *)s->work.p + 2 * (s->work_slot.fetch_add(1) % kWorkSlots);
-      hipLaunchKernelGGL(kern, dim3(groups), dim3(kRB), lds_s, (hipStream_t)stream, s->tree, tb, *p, frame_k(*p),
-                         frame, start_block, end_block, levels, work, counts);
-      DR_HIP_CHECK(hipGetLastError());
-      return DR_OK;
+    // deep trees, whose stacks leave no room for all the slots beside the registers' three workgroups a
+    // CU: half the slots if that gives a workgroup more (1080p 16 spp: 15.8 ms with 2,048 samples
+    // staged and three, 17.6 ms with 1,024 and three, 22.4 ms with 2,048 and two)
+    if (per_cu < kRenderWaves && slot_shift > 3) {
+      const size_t half = stream_lds(levels, spp, slot_shift - 1, origins);
+      int more = 0;
+      DR_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&more, kern, kRB, half));
+      if (more > per_cu) {
+        per_cu = more;
+        lds_s = half;
+        slot_shift--;
+      }
     }
+    const long long resident = (long long)s->num_cu * std::max(per_cu, 1);
+    // Tiles: 32 a workgroup, so that the last ones even out over the chip, but of at least 64 jobs: a
+    // tile costs an atomic on one address and its waves wait for its id.  (Whole blocks: 517x389 at
+    // 1 spp 968 us, 256x256 at 4 spp 461 us in one block per workgroup, 1080p at 16 spp 17.7 ms; so:
+    // 715 us, 310 us, 15.9 ms.  Tiles of 32 jobs: 910 us, 345 us; 8 a workgroup: 17.1 ms at 1080p.)
+    int tile_shift = 7;
+    while (tile_shift > 3 && (spp << tile_shift) >= 128 && (nrange << (7 - tile_shift)) < 32 * resident) tile_shift--;
+    const long long ntiles = nrange << (7 - tile_shift);
+    const long long groups = std::min<long long>(ntiles, resident);
+    // jobs a wave takes at a time: 1/32 of its share, between 8 and 64 (a wave's queue is its own: at
+    // the end of a small frame its entries wait while other waves are idle; 517x389 at 1 spp 784 us
+    // with 16, 715 us with 8), and a divisor of a tile's
+    const long long per_wave = nrange * kBlockPixels * spp / (groups * (kRB / 64));
+    int chunk = 64;
+    while (chunk > 8 && (chunk > per_wave / 32 || (spp << tile_shift) % chunk != 0)) chunk /= 2;
+    unsigned *work = (unsigned *)s->work.p + 2 * (s->work_slot.fetch_add(1) % kWorkSlots);
+    hipLaunchKernelGGL(kern, dim3((unsigned)groups), dim3(kRB), lds_s, (hipStream_t)stream, s->tree, tb, *p, frame_k(*p),
+                       frame, start_block, (int)ntiles, tile_shift, chunk, slot_shift, levels, work,
+                       counts);
+    DR_HIP_CHECK(hipGetLastError());
+    return DR_OK;
   }
   const size_t lds = ((size_t)levels * kStackWordsPerLevel * kRB + (size_t)kBlockPixels * kRoundSamples * 3) * 4;
   auto kernel = counts ? (ref ? k_render<RefPath, true> : k_render<BenchPath, true>)

@@ -217,7 +217,7 @@ __device__ __forceinline__ int wave_incl_max(int v) {   // v >= 0
 // One wave's LDS for walk_leaf_wave.
 struct LeafLds {
   unsigned long long best[64];   // per lane: the smallest key of its leaf
-  int first[64];                 // per record of a round: the lane whose leaf starts there; 0 between calls
+  unsigned char first[64];       // per record of a round: the lane whose leaf starts there; 0 between calls
 };
 __device__ __forceinline__ void leaf_lds_init(LeafLds &L) { L.first[__lane_id()] = 0; }
 
@@ -263,9 +263,9 @@ __device__ __forceinline__ void walk_leaf_wave(const DevTree &T, Walk &w, bool p
   int last = 0;                                          // the previous round's last owner
   auto owner_of = [&](int base) {
     const bool here = cnt > 0 && (unsigned)(start - base) < 64u;
-    if (here) put(&lds.first[start - base], lane);
-    const int v = max(wave_incl_max(get(&lds.first[lane])), last);
-    if (here) put(&lds.first[start - base], 0);
+    if (here) put(&lds.first[start - base], (unsigned char)lane);
+    const int v = max(wave_incl_max((int)get(&lds.first[lane])), last);
+    if (here) put(&lds.first[start - base], (unsigned char)0);
     last = __builtin_amdgcn_readlane(v, 63);
     return v;
   };
