@@ -16,6 +16,7 @@
 
 #include <algorithm>
 #include <new>
+#include <type_traits>
 #include <vector>
 
 namespace dr {
@@ -24,7 +25,8 @@ constexpr int kRB = 256;               // lanes per workgroup
 constexpr int kRoundSamples = 16;      // samples per pixel staged in LDS per round
 constexpr int kBlockPixels = 128;      // BlockBasedFrameBuffer<8,16>
 constexpr int kLeafMin = 16;           // pending leaves that trigger the (wave-shared) leaf tests
-constexpr int kShadeMin = 32;          // finished casts that trigger the adjoint's path updates
+constexpr int kShadeMin = 32;          // finished casts of a busy wave that trigger the adjoint's path updates
+constexpr int kAdjointRefillMin = 4;   // idle lanes that pop the adjoint's queue
 // Idle lanes a wave collects before it starts new path jobs (1, 8, 16, 32 measured
 // 34.9 / 35.0 / 35.3 / 38.4 ms at 1080p 16 spp, 0.84 / 0.77 / 0.80 / 0.90 ms at 256x256
 // 4 spp, 15.7 / 15.3 / 15.6 / 16.3 ms for the example scene at 1 spp, one block per
@@ -38,7 +40,6 @@ constexpr int kRenderWaves = 3;
 
 // Per-lane path state.
 struct Path {
-  int job = -1;
   uint32_t pix = 0, samp = 0;
   int layer = 0, phase = 0, light = 0;  // phase 0: geometry ray, 1: light photon
   V3 o, d;
@@ -867,16 +868,22 @@ __global__ __launch_bounds__(kRB, kRenderWaves) void k_render_stream(DevTree T, 
 // is formed backwards and dL/dalbedo += w dL/dI beta_k dA_k S_k.  dL/demission is
 // added during the replay: w dL/dI beta_k A_k (cos_i/pi)(cos_l A/d^2).
 // Rays are step-wise walks as in render_block.  The grid is persistent (one vertex-record
-// slice per workgroup): a workgroup takes the next framebuffer block from a counter in
-// global memory when it has finished one, so blocks of uneven cost spread over the grid as
-// hardware dispatch of one workgroup per block would spread them (a fixed assignment g,
-// g + gridDim.x, ... measured 20.9 ms against 15.7 ms for one workgroup per block on the
-// 512x512 16-spp adjoint).
+// slice per workgroup).  Paths are independent, so there is no barrier in the loop: each wave takes
+// `chunk` jobs of one framebuffer block at a time from a counter in global memory, forms their
+// camera rays and loss gradients with as many lanes into a queue in LDS, and its idle lanes pop the
+// next entry, as in k_render_stream.  (With one block per workgroup at a time the lanes waited for
+// each block's longest path: 512x512 16 spp 10.6 -> 7.3 ms.)
 // Reductions: the lanes of a wave that add to the same parameter in the same path
 // update are summed across the wave first (one LDS atomic per distinct material or
-// light and channel); the workgroup's LDS sums of one framebuffer block then go to
-// the FP64 outputs with one global atomic per parameter, and restart from zero.
+// light and channel), and the workgroup's LDS sums go to the FP64 outputs with one global atomic
+// per parameter.  The LDS sums are FP64 and go out once, at the end; where FP64 sums would take
+// LDS from a workgroup per CU (about 900 materials) they are FP32 and every wave moves them out
+// after kFlushJobs of its jobs, and where LDS has no room for those (about 12,000) the terms go to
+// the outputs.
 constexpr int kVtxWords = 9;
+enum : int { kSumsGlobal, kSumsFp32, kSumsFp64 };
+constexpr int kFlushJobs = 2048;
+constexpr int kAdjointQueueWords = 64 * 11;   // direction, pixel, sample, loss gradient, origin
 
 // Sum of v over the 64 lanes of the wave, returned to every lane: an inclusive scan within
 // each row of 16 lanes with DPP row shifts (1, 2, 4, 8; a lane without a source adds 0)
@@ -902,17 +909,18 @@ __device__ __forceinline__ float wave_sum(float v) {
 // 64 materials and 4 lights)
 constexpr int kWaveSumMin = 16;
 
-// Adds v[0..2] of every lane with `has` to acc[3 * key + c], one key at a time: the lanes
+// Adds v[0..2] of every lane with `has` to sum 3 * key + c (add(index, value)), one key at a time: the lanes
 // sharing a key are summed across the wave first (one atomic per channel) when there are at
 // least kWaveSumMin of them, and add their own terms otherwise.  Wave-uniform call.
-__device__ __forceinline__ void wave_add3(float *acc, bool has, int key, const float v[3]) {
+template <class Add>
+__device__ __forceinline__ void wave_add3(Add add, bool has, int key, const float v[3]) {
   const int lane = (int)__lane_id();
   uint64_t act = __ballot(has);
   if (__popcll(act) < kWaveSumMin) {          // too few terms for any sum across the wave to pay
     if (has) {
-      atomicAdd(&acc[3 * key + 0], v[0]);
-      atomicAdd(&acc[3 * key + 1], v[1]);
-      atomicAdd(&acc[3 * key + 2], v[2]);
+      add(3 * key + 0, v[0]);
+      add(3 * key + 1, v[1]);
+      add(3 * key + 2, v[2]);
     }
     return;
   }
@@ -923,35 +931,37 @@ __device__ __forceinline__ void wave_add3(float *acc, bool has, int key, const f
     if (__popcll(__ballot(sel)) >= kWaveSumMin) {
       const float s0 = wave_sum(sel ? v[0] : 0.0f), s1 = wave_sum(sel ? v[1] : 0.0f), s2 = wave_sum(sel ? v[2] : 0.0f);
       if (lane == leader) {
-        atomicAdd(&acc[3 * k + 0], s0);
-        atomicAdd(&acc[3 * k + 1], s1);
-        atomicAdd(&acc[3 * k + 2], s2);
+        add(3 * k + 0, s0);
+        add(3 * k + 1, s1);
+        add(3 * k + 2, s2);
       }
     } else if (sel) {
-      atomicAdd(&acc[3 * k + 0], v[0]);
-      atomicAdd(&acc[3 * k + 1], v[1]);
-      atomicAdd(&acc[3 * k + 2], v[2]);
+      add(3 * k + 0, v[0]);
+      add(3 * k + 1, v[1]);
+      add(3 * k + 2, v[2]);
     }
     has = has && !sel;
     act = __ballot(has);
   }
 }
 
+template <int kSums>
 __global__ __launch_bounds__(kRB, kRenderWaves) void k_backward(DevTree T, const float4 *__restrict__ shade,
                                                                  dr_render_params P, FrameK FK,
                                                                  const float *__restrict__ dl,
                                                                  double *__restrict__ g_albedo,
                                                                  double *__restrict__ g_emission,
                                                                  float *__restrict__ vtx_all,
-                                                                 int *__restrict__ next_block, int nblocks,
-                                                                 int levels, int maxv) {
+                                                                 int *__restrict__ next_unit, int nblocks, int chunk,
+                                                                 int unit_chunks, int levels, int maxv) {
   extern __shared__ __align__(16) uint32_t lds[];
-  __shared__ int next_job, cur_block;
   __shared__ LeafLds leaf_all[kRB / 64];
   LeafLds &leaf = leaf_all[threadIdx.x >> 6];
   leaf_lds_init(leaf);
   uint2 *stk = (uint2 *)lds + threadIdx.x;
-  float *gacc = (float *)(lds + levels * kStackWordsPerLevel * kRB);   // nmat*3 albedo, then nlights*3 emission
+  float *queue = (float *)(lds + levels * kStackWordsPerLevel * kRB) + (threadIdx.x >> 6) * kAdjointQueueWords;   // [word][entry]
+  using Acc = std::conditional_t<kSums == kSumsFp64, double, float>;
+  Acc *gacc = (Acc *)(lds + levels * kStackWordsPerLevel * kRB + (kRB / 64) * kAdjointQueueWords);   // nmat*3 albedo, then nlights*3 emission
   float *vtx = vtx_all + (size_t)blockIdx.x * maxv * kVtxWords * kRB;
   const int ngrad = 3 * (P.nmat + P.nlights);
   const int spp = P.fsaa_x * P.fsaa_y;
@@ -959,164 +969,204 @@ __global__ __launch_bounds__(kRB, kRenderWaves) void k_backward(DevTree T, const
   const float spw = uni(1.0f / (((float)P.fsaa_x) * ((float)P.fsaa_y)));
   const UDiv Dspp = udiv_uniform((uint32_t)spp);
   const bool clip = P.cull_backfaces != 0;
+  const bool origins = P.lens == DR_SPHERICAL_SEGMENT_LENS;
   const int lane = (int)__lane_id();
   const uint64_t below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-  for (int t = threadIdx.x; t < ngrad; t += kRB) gacc[t] = 0.0f;
-  const int njobs = kBlockPixels * spp;
+  if (kSums != kSumsGlobal)
+    for (int t = threadIdx.x; t < ngrad; t += kRB) gacc[t] = (Acc)0;
+  __syncthreads();
+  auto add = [&](int i, float v) {
+    if constexpr (kSums != kSumsGlobal) atomicAdd(&gacc[i], (Acc)v);
+    else atomicAdd(i < 3 * P.nmat ? &g_albedo[i] : &g_emission[i - 3 * P.nmat], (double)v);
+  };
+  // units of unit_chunks chunks, numbered block by block
+  const int nchunks = kBlockPixels * spp / chunk, parts = (nchunks + unit_chunks - 1) / unit_chunks;
   auto V_ = [&](int k, int w) -> float & { return vtx[((size_t)k * kVtxWords + w) * kRB + threadIdx.x]; };
-
-  for (;;) {
-    if (threadIdx.x == 0) {
-      next_job = 0;
-      cur_block = atomicAdd(next_block, 1);
-    }
-    __syncthreads();
-    const int block = cur_block;      // read before the barriers that end this iteration
-    if (block >= nblocks) break;
-    Path st;
-    Walk w;
-    w.state = kWalkDone;
-    int K = 0;                      // vertices recorded for the current path
-    bool fin = false;               // the current path has ended; its albedo terms are pending
-    float wdl[3] = {0, 0, 0};       // spw * dL/dI (* lens filter) of the current pixel
-    bool exhausted = false;
-    // the vertex's reflection factor and dA/dalbedo, then the next bounce (or the path's end)
-    auto advance = [&]() {
-      const dr_material M = P.materials[st.mid];
-      float f5 = 0.0f;
-      const bool metal = st.kind == DR_METAL && st.has_sample;
-      if (metal) f5 = schlick5(st.nu, st.sdir);
-      for (int c = 0; c < 3; c++) V_(K - 1, 1 + c) = metal ? M.albedo[c] + (1.0f - M.albedo[c]) * f5 : M.albedo[c];
-      V_(K - 1, 8) = metal ? 1.0f - f5 : 1.0f;
-      V_(K - 1, 7) = st.has_sample ? st.sweight : 0.0f;
-      if (!st.has_sample) { fin = true; return; }
-      for (int c = 0; c < 3; c++) st.beta[c] = st.beta[c] * (V_(K - 1, 1 + c) * st.sweight);
-      st.o = st.p;
-      st.d = st.sdir;
-      st.restrict_tri = st.h;
-      st.layer++;
-      st.phase = 0;
-    };
-    for (;;) {
-      const bool want = (st.job < 0) && !exhausted;
-      const uint64_t wmask = __ballot(want);
-      // new path jobs once kRenderRefillMin lanes are idle (or no lane is busy), as in render_block
-      // (thresholds 1, 4, 8, 16 measured 21.3 / 21.2 / 21.2 / 21.5 ms for the 512x512 adjoint)
-      if (wmask && (__popcll(wmask) >= kRenderRefillMin || __ballot(st.job >= 0) == 0)) {
-        const int leader = __ffsll((unsigned long long)wmask) - 1;
-        int base = 0;
-        if (lane == leader) base = atomicAdd(&next_job, __popcll(wmask));
-        base = __shfl(base, leader);
-        if (want) {
-          const int slot = base + __popcll(wmask & below);
-          if (slot < njobs) {
-            st.job = slot;
-            const int lp = (int)udiv((uint32_t)slot, Dspp), s = slot - lp * spp;
-            K = 0;
-            if (!start_path(P, FK, block, lp, s, samp0, st)) {
-              st.job = -1;
-            } else {
-              const float *g = dl + 4 * ((size_t)kBlockPixels * block + lp);
-              // SphericalSegmentLense::getPixelColor scales the sample colour by its filter
-              for (int c = 0; c < 3; c++)
-                wdl[c] = spw * g[c] * (P.lens == DR_SPHERICAL_SEGMENT_LENS ? P.lens_p[4 + c] : 1.0f);
-              walk_begin(T, w, st.o, st.d, st.restrict_tri, stk);
-            }
-          } else {
-            exhausted = true;
-          }
-        }
-      }
-      if (__ballot(st.job >= 0) == 0) {
-        if (__ballot(!exhausted) == 0) break;
-        continue;
-      }
-      if (st.job >= 0 && w.state == kWalkTrace) walk_step(T, w, stk, kRB, nullptr);
-      const bool pend = st.job >= 0 && w.state == kWalkLeaf;
-      const uint64_t pm = __ballot(pend);
-      if (pm && (__popcll(pm) >= kLeafMin || __ballot(st.job >= 0 && w.state == kWalkTrace) == 0))
-        walk_leaf_wave(T, w, pend, clip, leaf, nullptr, nullptr);
-      const uint64_t dm = __ballot(st.job >= 0 && w.state == kWalkDone);
-      if (dm && (__popcll(dm) >= kShadeMin || __ballot(st.job >= 0 && w.state != kWalkDone) == 0)) {
-        bool lit = false;
-        float ev[3] = {0.0f, 0.0f, 0.0f};
-        int lkey = 0;
-        if (st.job >= 0 && w.state == kWalkDone) {
-          bool photons = false;
-          if (st.phase == 0) {
-            if (!w.hit) fin = true;
-            else {
-              setup_vertex(P, FK, shade, w.h, w.d, st);
-              V_(K, 0) = __int_as_float(st.mid);
-              for (int c = 0; c < 4; c++) V_(K, 4 + c) = 0.0f;
-              K++;
-              photons = st.kind == DR_LAMBERT;
-              if (!photons) advance();
-            }
-          } else {
-            const V3 e = w.h.p - st.p;
-            lit = w.hit && (w.h.id == st.h || (e.x * e.x + e.y * e.y + e.z * e.z) <= (8.0f * kVecEps));
-            if (lit) {
-              const dr_material M = P.materials[st.mid];
-              const float *E = P.lights[st.light].emission;
-              for (int c = 0; c < 3; c++) {
-                V_(K - 1, 4 + c) += st.gl_k * E[c];
-                ev[c] = wdl[c] * st.beta[c] * M.albedo[c] * st.gl_k;
-              }
-              lkey = P.nmat + st.light;
-            }
-            photons = true;
-          }
-          if (photons && !next_photon(P, st)) advance();
-          if (!fin) walk_begin(T, w, st.o, st.d, st.restrict_tri, stk);
-        }
-        // dL/demission of this update's lit photons
-        wave_add3(gacc, lit, lkey, ev);
-        // dL/dalbedo of the paths that ended: S_k backwards, then beta_k forwards
-        if (__ballot(fin)) {
-          if (fin) {
-            float Ln[3] = {0, 0, 0};
-            for (int k = K - 1; k >= 0; k--)
-              for (int c = 0; c < 3; c++) {
-                const float S = V_(k, 4 + c) + V_(k, 7) * Ln[c];
-                Ln[c] = V_(k, 1 + c) * S;
-                V_(k, 4 + c) = S;
-              }
-          }
-          float beta[3] = {1, 1, 1};
-          int kmax = fin ? K : 0;
-#pragma unroll
-          for (int off = 32; off >= 1; off >>= 1) kmax = max(kmax, __shfl_xor(kmax, off));
-          for (int k = 0; k < kmax; k++) {
-            const bool has = fin && k < K;
-            float av[3] = {0.0f, 0.0f, 0.0f};
-            int m = 0;
-            if (has) {
-              m = __float_as_int(V_(k, 0));
-              const float dA = V_(k, 8);
-              for (int c = 0; c < 3; c++) {
-                av[c] = wdl[c] * beta[c] * dA * V_(k, 4 + c);
-                beta[c] = beta[c] * (V_(k, 1 + c) * V_(k, 7));
-              }
-            }
-            wave_add3(gacc, has, m, av);
-          }
-          if (fin) { st.job = -1; fin = false; }
-        }
-      }
-    }
-    __syncthreads();
-    // this block's sums into the FP64 gradients
-    for (int t = threadIdx.x; t < ngrad; t += kRB) {
-      const float v = gacc[t];
-      if (v != 0.0f) {
+  // sums t, t + step, ... into the FP64 gradients
+  auto flush = [&](int t0, int step) {
+    for (int t = t0; t < ngrad; t += step) {
+      Acc v;
+      if constexpr (kSums == kSumsFp32) v = atomicExch(&gacc[t], (Acc)0);
+      else v = gacc[t];
+      if (v != (Acc)0) {
         if (t < 3 * P.nmat) atomicAdd(&g_albedo[t], (double)v);
         else atomicAdd(&g_emission[t - 3 * P.nmat], (double)v);
       }
-      gacc[t] = 0.0f;
     }
-    __syncthreads();
+  };
+
+  Path st;
+  Walk w;
+  w.state = kWalkDone;
+  int K = 0;                      // vertices recorded for the current path
+  bool live = false;              // the lane has a path
+  bool fin = false;               // the current path has ended; its albedo terms are pending
+  float wdl[3] = {0, 0, 0};       // spw * dL/dI (* lens filter) of the current pixel
+  // the wave's queue (wave-uniform): entries [qpos, qlen); the unit's next chunks [cnext, cend) of block `block`
+  int qpos = 0, qlen = 0, block = 0, cnext = 0, cend = 0, jobs = 0;
+  bool ended = false;
+  // the vertex's reflection factor and dA/dalbedo, then the next bounce (or the path's end)
+  auto advance = [&]() {
+    const dr_material M = P.materials[st.mid];
+    float f5 = 0.0f;
+    const bool metal = st.kind == DR_METAL && st.has_sample;
+    if (metal) f5 = schlick5(st.nu, st.sdir);
+    for (int c = 0; c < 3; c++) V_(K - 1, 1 + c) = metal ? M.albedo[c] + (1.0f - M.albedo[c]) * f5 : M.albedo[c];
+    V_(K - 1, 8) = metal ? 1.0f - f5 : 1.0f;
+    V_(K - 1, 7) = st.has_sample ? st.sweight : 0.0f;
+    if (!st.has_sample) { fin = true; return; }
+    for (int c = 0; c < 3; c++) st.beta[c] = st.beta[c] * (V_(K - 1, 1 + c) * st.sweight);
+    st.o = st.p;
+    st.d = st.sdir;
+    st.restrict_tri = st.h;
+    st.layer++;
+    st.phase = 0;
+  };
+  for (;;) {
+    // ---- path updates of the finished casts, batched (the threshold in proportion to the busy
+    // lanes, as in k_render_stream)
+    bool fresh = false;           // the lane has a new ray
+    const uint64_t dm = __ballot(live && w.state == kWalkDone);
+    if (dm && __popcll(dm) * 64 >= __popcll(__ballot(live)) * kShadeMin) {
+      bool lit = false;
+      float ev[3] = {0.0f, 0.0f, 0.0f};
+      int lkey = 0;
+      if (live && w.state == kWalkDone) {
+        bool photons = false;
+        if (st.phase == 0) {
+          if (!w.hit) fin = true;
+          else {
+            setup_vertex(P, FK, shade, w.h, w.d, st);
+            V_(K, 0) = __int_as_float(st.mid);
+            for (int c = 0; c < 4; c++) V_(K, 4 + c) = 0.0f;
+            K++;
+            photons = st.kind == DR_LAMBERT;
+            if (!photons) advance();
+          }
+        } else {
+          const V3 e = w.h.p - st.p;
+          lit = w.hit && (w.h.id == st.h || (e.x * e.x + e.y * e.y + e.z * e.z) <= (8.0f * kVecEps));
+          if (lit) {
+            const dr_material M = P.materials[st.mid];
+            const float *E = P.lights[st.light].emission;
+            for (int c = 0; c < 3; c++) {
+              V_(K - 1, 4 + c) += st.gl_k * E[c];
+              ev[c] = wdl[c] * st.beta[c] * M.albedo[c] * st.gl_k;
+            }
+            lkey = P.nmat + st.light;
+          }
+          photons = true;
+        }
+        if (photons && !next_photon(P, st)) advance();
+        fresh = !fin;
+      }
+      // dL/demission of this update's lit photons
+      wave_add3(add, lit, lkey, ev);
+      // dL/dalbedo of the paths that ended: S_k backwards, then beta_k forwards
+      if (__ballot(fin)) {
+        if (fin) {
+          float Ln[3] = {0, 0, 0};
+          for (int k = K - 1; k >= 0; k--)
+            for (int c = 0; c < 3; c++) {
+              const float S = V_(k, 4 + c) + V_(k, 7) * Ln[c];
+              Ln[c] = V_(k, 1 + c) * S;
+              V_(k, 4 + c) = S;
+            }
+        }
+        float beta[3] = {1, 1, 1};
+        int kmax = fin ? K : 0;
+#pragma unroll
+        for (int off = 32; off >= 1; off >>= 1) kmax = max(kmax, __shfl_xor(kmax, off));
+        for (int k = 0; k < kmax; k++) {
+          const bool has = fin && k < K;
+          float av[3] = {0.0f, 0.0f, 0.0f};
+          int m = 0;
+          if (has) {
+            m = __float_as_int(V_(k, 0));
+            const float dA = V_(k, 8);
+            for (int c = 0; c < 3; c++) {
+              av[c] = wdl[c] * beta[c] * dA * V_(k, 4 + c);
+              beta[c] = beta[c] * (V_(k, 1 + c) * V_(k, 7));
+            }
+          }
+          wave_add3(add, has, m, av);
+        }
+        if (fin) { live = false; fin = false; }
+      }
+    }
+    // ---- the queue is empty: the next chunk of the unit, or the next unit
+    if (qpos == qlen && !ended) {
+      if (cnext == cend) {
+        int unit = 0;
+        if (lane == 0) unit = atomicAdd(next_unit, 1);
+        unit = uni(unit);
+        block = unit / parts;
+        cnext = (unit - block * parts) * unit_chunks;
+        cend = min(cnext + unit_chunks, nchunks);
+        ended = block >= nblocks;
+        if (kSums == kSumsFp32 && !ended && jobs >= kFlushJobs) {
+          flush(lane, 64);
+          jobs = 0;
+        }
+      }
+      if (!ended) {
+        if (lane < chunk) {
+          const int q = cnext * chunk + lane;
+          const int lp = (int)udiv((uint32_t)q, Dspp);
+          const PathStart ps = path_start(P, FK, block, lp, q - lp * spp, samp0);
+          const float *g = dl + 4 * ((size_t)kBlockPixels * block + lp);
+          queue[0 * 64 + lane] = ps.d.x;
+          queue[1 * 64 + lane] = ps.d.y;
+          queue[2 * 64 + lane] = ps.d.z;
+          queue[3 * 64 + lane] = __int_as_float((int)ps.pix);
+          queue[4 * 64 + lane] = __int_as_float((int)ps.samp);
+          // SphericalSegmentLense::getPixelColor scales the sample colour by its filter
+          for (int c = 0; c < 3; c++) queue[(5 + c) * 64 + lane] = spw * g[c] * (origins ? P.lens_p[4 + c] : 1.0f);
+          if (origins) {
+            queue[8 * 64 + lane] = ps.o.x;
+            queue[9 * 64 + lane] = ps.o.y;
+            queue[10 * 64 + lane] = ps.o.z;
+          }
+        }
+        __threadfence_block();
+        qpos = 0;
+        qlen = chunk;
+        cnext++;
+        jobs += chunk;
+      }
+    }
+    // ---- idle lanes pop the next entries
+    const uint64_t idle = __ballot(!live);
+    if (qpos < qlen && idle && (__popcll(idle) >= kAdjointRefillMin || idle == ~0ull)) {
+      const int entry = qpos + __popcll(idle & below);
+      const bool take = !live && entry < qlen;
+      qpos += __popcll(__ballot(take));
+      if (take) {
+        PathStart ps;
+        ps.d = v3(queue[0 * 64 + entry], queue[1 * 64 + entry], queue[2 * 64 + entry]);
+        ps.pix = (uint32_t)__float_as_int(queue[3 * 64 + entry]);
+        ps.samp = (uint32_t)__float_as_int(queue[4 * 64 + entry]);
+        for (int c = 0; c < 3; c++) wdl[c] = queue[(5 + c) * 64 + entry];
+        ps.o = v3(P.cam[0], P.cam[1], P.cam[2]);
+        if (origins) ps.o = v3(queue[8 * 64 + entry], queue[9 * 64 + entry], queue[10 * 64 + entry]);
+        live = fresh = ps.pix != kNoPixel;     // (a pixel outside the image has no paths)
+        begin_path(st, ps);
+        K = 0;
+      }
+    }
+    if (__ballot(live) == 0) {
+      if (qpos == qlen && ended) break;
+      continue;
+    }
+    if (fresh) walk_begin(T, w, st.o, st.d, st.restrict_tri, stk);
+    if (live && w.state == kWalkTrace) walk_step(T, w, stk, kRB, nullptr);
+    const bool pend = live && w.state == kWalkLeaf;
+    const uint64_t pm = __ballot(pend);
+    if (pm && (__popcll(pm) * (64 / kLeafMin) >= __popcll(__ballot(live)) || __ballot(live && w.state == kWalkTrace) == 0))
+      walk_leaf_wave(T, w, pend, clip, leaf, nullptr, nullptr);
   }
+  __syncthreads();
+  if (kSums != kSumsGlobal) flush(threadIdx.x, kRB);
 }
 
 // ------------------------------------------------------------------ batched requests
@@ -1275,26 +1325,43 @@ extern "C" int dr_render_stats(dr_scene s, const dr_render_params *p, float *fra
 
 namespace dr {
 
-// Launch shape of the adjoint: LDS bytes (traversal stacks + gradient sums) and the size
-// of one workgroup's vertex records.
-static int backward_shape(dr_scene s, const dr_render_params *p, int &levels, int &maxv, size_t &lds, size_t &slice) {
-  levels = s->max_depth > 0 ? s->max_depth : 1;
-  maxv = p->max_bounces + 1;
-  lds = ((size_t)levels * kStackWordsPerLevel * kRB + 3 * (size_t)(p->nmat + p->nlights)) * 4;
-  slice = (size_t)maxv * kVtxWords * kRB * sizeof(float);
-  if (lds > 160 * 1024) return fail(DR_ERR_ARG, "dr_backward: too many materials and lights for LDS");
-  if (lds > 64 * 1024)
-    DR_HIP_CHECK(hipFuncSetAttribute((const void *)k_backward, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-  return DR_OK;
+static decltype(&k_backward<kSumsFp64>) backward_kernel(int sums) {
+  return sums == kSumsFp64 ? k_backward<kSumsFp64> : (sums == kSumsFp32 ? k_backward<kSumsFp32> : k_backward<kSumsGlobal>);
 }
-
-// Workgroups of the persistent adjoint grid: one per resident slot, at most one per
-// framebuffer block, and at most as many as `vtx_bytes` of vertex records hold.
-static int backward_groups(dr_scene s, size_t lds, size_t slice, int nblocks, size_t vtx_bytes, int &groups) {
+// Launch shape of the adjoint.
+struct BackwardShape {
+  int sums;               // kSums* of k_backward
+  int levels, maxv;
+  size_t lds, slice;      // LDS bytes, and bytes of one workgroup's vertex records
+  int nblocks, groups, chunk, unit_chunks;
+};
+// Workgroups of the persistent grid: one per resident slot, at most one per 256 paths, and at
+// most as many as `vtx_bytes` of vertex records hold.
+static int backward_shape(dr_scene s, const dr_render_params *p, size_t vtx_bytes, BackwardShape &B) {
+  B.levels = s->max_depth > 0 ? s->max_depth : 1;
+  B.maxv = p->max_bounces + 1;
+  B.nblocks = block_count(p);
+  B.slice = (size_t)B.maxv * kVtxWords * kRB * sizeof(float);
+  const size_t stacks = (size_t)B.levels * kStackWordsPerLevel * kRB * 4, queues = (kRB / 64) * (size_t)kAdjointQueueWords * 4;
+  const size_t ngrad = 3 * (size_t)(p->nmat + p->nlights);
+  if (stacks + 4 * ngrad > 160 * 1024) return fail(DR_ERR_ARG, "dr_backward: too many materials and lights for LDS");
+  // (LeafLds of the four waves beside them)
+  const size_t fixed = stacks + queues + (kRB / 64) * sizeof(LeafLds);
+  B.sums = fixed + 8 * ngrad <= 160 * 1024 / kRenderWaves ? kSumsFp64 : (fixed + 4 * ngrad <= 160 * 1024 ? kSumsFp32 : kSumsGlobal);
+  B.lds = stacks + queues + (B.sums == kSumsFp64 ? 8 : (B.sums == kSumsFp32 ? 4 : 0)) * ngrad;
+  const void *kern = (const void *)backward_kernel(B.sums);
+  if (B.lds > 64 * 1024) DR_HIP_CHECK(hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)B.lds));
   int per_cu = 0;
-  DR_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_backward, kRB, lds));
+  DR_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, kRB, B.lds));
   const long long resident = (long long)s->num_cu * std::max(per_cu, 1);
-  groups = (int)std::min<long long>({(long long)nblocks, resident, (long long)(vtx_bytes / slice)});
+  const long long jobs = (long long)B.nblocks * kBlockPixels * p->fsaa_x * p->fsaa_y;
+  B.groups = (int)std::min<long long>({(jobs + kRB - 1) / kRB, resident, (long long)(vtx_bytes / B.slice)});
+  // jobs a wave takes at a time: 1/32 of its share, between 8 and 64
+  const long long per_wave = jobs / ((long long)std::max(B.groups, 1) * (kRB / 64));
+  B.chunk = 64;
+  while (B.chunk > 8 && B.chunk > per_wave / 32) B.chunk /= 2;
+  B.unit_chunks = 1;
+  while (jobs / B.chunk / B.unit_chunks + B.nblocks >= (1 << 30)) B.unit_chunks *= 2;
   return DR_OK;
 }
 
@@ -1307,24 +1374,23 @@ static int check_backward(dr_scene s, const dr_render_params *p, const float *dl
   return DR_OK;
 }
 
-// Scratch of one adjoint launch: the block counter, then `groups` vertex-record slices.
+// Scratch of one adjoint launch: the unit counter, then `groups` vertex-record slices.
 constexpr size_t kCounterBytes = 256;
 
 static void launch_backward(dr_scene s, const dr_render_params *p, const float *dl, double *ga, double *ge,
-                            void *scratch_mem, int groups, int nblocks, int levels, int maxv, size_t lds,
-                            hipStream_t stream) {
+                            void *scratch_mem, const BackwardShape &B, hipStream_t stream) {
   int *counter = (int *)scratch_mem;
   float *vtx = (float *)((char *)scratch_mem + kCounterBytes);
   hipLaunchKernelGGL(k_zero, dim3(1), dim3(64), 0, stream, counter, 1);
-  hipLaunchKernelGGL(k_backward, dim3(groups), dim3(kRB), lds, stream, s->tree, tables_of(s, p).shade, *p, frame_k(*p),
-                     dl, ga, ge, vtx, counter, nblocks, levels, maxv);
+  hipLaunchKernelGGL(backward_kernel(B.sums), dim3(B.groups), dim3(kRB), B.lds, stream, s->tree, tables_of(s, p).shade,
+                     *p, frame_k(*p), dl, ga, ge, vtx, counter, B.nblocks, B.chunk, B.unit_chunks, B.levels, B.maxv);
 }
 
 }  // namespace dr
 
 namespace dr {
 
-// Block counter and vertex records of dr_backward_noalloc: a file-scope device array
+// Unit counter and vertex records of dr_backward_noalloc: a file-scope device array
 // (kNoAllocBytes on every device the library runs on, held until the process ends).  Host
 // code never passes `scratch` itself (its host-side name is not a device address): it
 // passes the address hipGetSymbolAddress gives for the current device, resolved once per
@@ -1355,20 +1421,16 @@ extern "C" int dr_backward_noalloc(dr_scene s, const dr_render_params *p, const 
                                    double *g_emission, void *stream) {
   int rc = dr::check_backward(s, p, dl_dframe, g_albedo, g_emission);
   if (rc != DR_OK) return rc;
-  int levels, maxv, groups, device = 0;
-  size_t lds, slice;
-  if ((rc = dr::backward_shape(s, p, levels, maxv, lds, slice)) != DR_OK) return rc;
-  if (slice > dr::kNoAllocBytes - dr::kCounterBytes)
+  int device = 0;
+  // as many persistent workgroups as the array holds vertex records for (after the unit counter)
+  dr::BackwardShape B;
+  if ((rc = dr::backward_shape(s, p, dr::kNoAllocBytes - dr::kCounterBytes, B)) != DR_OK) return rc;
+  if (B.slice > dr::kNoAllocBytes - dr::kCounterBytes)
     return dr::fail(DR_ERR_ARG, "dr_backward_noalloc: one workgroup's vertex records exceed the 40 MiB scratch array");
   DR_HIP_CHECK(hipGetDevice(&device));
   float *mem = nullptr;
   if ((rc = dr::noalloc_scratch_init(device, &mem)) != DR_OK) return rc;
-  const int nblocks = dr::block_count(p);
-  // as many persistent workgroups as the array holds vertex records for (after the block counter)
-  if ((rc = dr::backward_groups(s, lds, slice, nblocks, dr::kNoAllocBytes - dr::kCounterBytes, groups)) != DR_OK)
-    return rc;
-  dr::launch_backward(s, p, dl_dframe, g_albedo, g_emission, mem, groups, nblocks, levels, maxv, lds,
-                      (hipStream_t)stream);
+  dr::launch_backward(s, p, dl_dframe, g_albedo, g_emission, mem, B, (hipStream_t)stream);
   DR_HIP_CHECK(hipGetLastError());
   return DR_OK;
 }
@@ -1377,17 +1439,13 @@ extern "C" int dr_backward(dr_scene s, const dr_render_params *p, const float *d
                            double *g_emission, void *stream) {
   int rc = dr::check_backward(s, p, dl_dframe, g_albedo, g_emission);
   if (rc != DR_OK) return rc;
-  int levels, maxv, groups;
-  size_t lds, slice;
-  if ((rc = dr::backward_shape(s, p, levels, maxv, lds, slice)) != DR_OK) return rc;
-  const int nblocks = dr::block_count(p);
-  if ((rc = dr::backward_groups(s, lds, slice, nblocks, SIZE_MAX, groups)) != DR_OK) return rc;
-  // block counter and vertex records: the scene's buffer for this stream, grown when a call needs more
+  dr::BackwardShape B;
+  if ((rc = dr::backward_shape(s, p, SIZE_MAX, B)) != DR_OK) return rc;
+  // unit counter and vertex records: the scene's buffer for this stream, grown when a call needs more
   void *mem = nullptr;
-  if ((rc = dr::scene_scratch(s, (hipStream_t)stream, dr::kCounterBytes + (size_t)groups * slice, &mem)) != DR_OK)
+  if ((rc = dr::scene_scratch(s, (hipStream_t)stream, dr::kCounterBytes + (size_t)B.groups * B.slice, &mem)) != DR_OK)
     return rc;
-  dr::launch_backward(s, p, dl_dframe, g_albedo, g_emission, mem, groups, nblocks, levels, maxv, lds,
-                      (hipStream_t)stream);
+  dr::launch_backward(s, p, dl_dframe, g_albedo, g_emission, mem, B, (hipStream_t)stream);
   DR_HIP_CHECK(hipGetLastError());
   return DR_OK;
 }

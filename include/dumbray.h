@@ -258,15 +258,15 @@ int dr_render_blocks(dr_scene s, const dr_render_params *p, float *frame, int st
  * by path replay (each path is re-traced from its Philox key, nothing is stored
  * between passes).  dl_dframe: device, same block layout as `frame` (alpha ignored).
  * Adds dL/dalbedo (Lambert albedo and mirror reflectance; device double[nmat*3]) and
- * dL/demission (device double[nlights*3]); the caller zeroes them.  Per-block
- * reductions in LDS precede one FP64 atomic per block and parameter.  The benchmark
+ * dL/demission (device double[nlights*3]); the caller zeroes them.  FP64
+ * sums in LDS precede one FP64 atomic per workgroup and parameter.  The benchmark
  * plugin set only; every lens (the spherical segment lens's filter scales dL/dI). */
 int dr_backward(dr_scene s, const dr_render_params *p, const float *dl_dframe, double *g_albedo, double *g_emission,
                 void *stream);
 
 /* dr_backward for callers that cannot allocate device memory (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc).  No counterpart in the
- * reference.  Same arguments and results as dr_backward; the block counter and the vertex
+ * reference.  Same arguments and results as dr_backward; the unit counter and the vertex
  * records of the path replay live in a 40 MiB array that the library holds on every device it runs on until
  * the process ends (its address is resolved by dr_device_open, or by the first call on a
  * device), and the persistent grid is sized to what that array holds (all resident
