@@ -27,13 +27,6 @@ constexpr int kBlockPixels = 128;      // BlockBasedFrameBuffer<8,16>
 constexpr int kLeafMin = 16;           // pending leaves that trigger the (wave-shared) leaf tests
 constexpr int kShadeMin = 32;          // finished casts of a busy wave that trigger the adjoint's path updates
 constexpr int kAdjointRefillMin = 4;   // idle lanes that pop the adjoint's queue
-// Idle lanes a wave collects before it starts new path jobs (1, 8, 16, 32 measured
-// 34.9 / 35.0 / 35.3 / 38.4 ms at 1080p 16 spp, 0.84 / 0.77 / 0.80 / 0.90 ms at 256x256
-// 4 spp, 15.7 / 15.3 / 15.6 / 16.3 ms for the example scene at 1 spp, one block per
-// workgroup; 4, 8, 16 gave 29.8 / 29.8 / 30.4 ms at 1080p on the streamed kernel).  Used by the
-// adjoint and as the batch autotuner's starting point; the render kernels take the estimator's
-// kRefillMin / kStreamRefillMin.
-constexpr int kRenderRefillMin = 8;
 // Waves per SIMD the render kernels are compiled for: the register cap this sets
 // (168 VGPRs) costs a few spills but beats 2 waves per SIMD clearly.
 constexpr int kRenderWaves = 3;
@@ -640,20 +633,32 @@ constexpr size_t stream_lds(int levels, int spp, int slot_shift, bool origins) {
           (kRB / 64) * (size_t)stream_queue_words(origins)) * 4;
 }
 
+// Words of LDS that other waves change (an atomic access stays an LDS instruction; a volatile one
+// would go through a flat address).
+__device__ __forceinline__ int lds_get(const int *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); }
+__device__ __forceinline__ void lds_put(int *p, int v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); }
+
+// LDS of a workgroup's stream beside the dynamic part (stream_lds).
+struct StreamLds {
+  int tiles[kStreamRing];          // (tile id + 1) << 8 | tile number & 255
+  int px_done[kStreamRing];        // pixels written, cumulative per ring entry
+  unsigned next_job;
+  int end_k;                       // first tile number past the range
+  LeafLds leaf[kRB / 64];
+};
+// The tiles of a stream and its launch shape.
+struct StreamShape {
+  int ntiles, tile_shift, chunk, slot_shift;
+};
+
+// One stream (every lane of the workgroup calls it): tiles from the counter `next_tile` until they run out.
+// ins: this wave's inside-test counts (measurement launches only).
 template <class PathT, bool kStats>
-__global__ __launch_bounds__(kRB, kRenderWaves) void k_render_stream(DevTree T, Tables tb, dr_render_params P,
-                                                                      FrameK K, float *__restrict__ frame, int start_block,
-                                                                      int ntiles, int tile_shift, int chunk, int slot_shift,
-                                                                      int levels,
-                                                                      unsigned *__restrict__ work,
-                                                                      unsigned long long *__restrict__ counts) {
-  extern __shared__ __align__(16) uint32_t lds[];
-  __shared__ int tiles[kStreamRing];          // (tile id + 1) << 8 | tile number & 255
-  __shared__ int px_done[kStreamRing];        // pixels written, cumulative per ring entry
-  __shared__ unsigned next_job;
-  __shared__ int end_k;                       // first tile number past the range
-  __shared__ LeafLds leaf_all[kRB / 64];
-  __shared__ int ins_all[kStats ? kRB : 1];
+__device__ __forceinline__ void stream_paths(const DevTree &T, const Tables &tb, const dr_render_params &P, FrameK K,
+                                             float *__restrict__ frame, int start_block, const StreamShape &S, int levels,
+                                             unsigned *next_tile, int refill_min, uint32_t *lds, StreamLds &sh, int *ins,
+                                             RenderCounters &rc) {
+  const int ntiles = S.ntiles, tile_shift = S.tile_shift, chunk = S.chunk, slot_shift = S.slot_shift;
   const int spp = P.fsaa_x * P.fsaa_y;
   const int nslots = slot_shift < 0 ? 0 : 1 << slot_shift;
   const bool origins = P.lens == DR_SPHERICAL_SEGMENT_LENS;
@@ -661,15 +666,13 @@ __global__ __launch_bounds__(kRB, kRenderWaves) void k_render_stream(DevTree T, 
   float *samp = (float *)(lds + levels * kStackWordsPerLevel * kRB);   // nslots * spp * 3
   int *turn = (int *)(samp + (size_t)nslots * spp * 3);              // nslots
   float *queue = (float *)(turn + nslots) + (threadIdx.x >> 6) * stream_queue_words(origins);   // [word][entry]
-  LeafLds &leaf = leaf_all[threadIdx.x >> 6];
+  LeafLds &leaf = sh.leaf[threadIdx.x >> 6];
   leaf_lds_init(leaf);
-  int *ins = kStats ? ins_all + (threadIdx.x & ~63u) : nullptr;
   for (int t = threadIdx.x; t < nslots; t += kRB) turn[t] = spp;
-  for (int t = threadIdx.x; t < kStreamRing; t += kRB) { tiles[t] = 0; px_done[t] = 0; }
-  if (threadIdx.x == 0) { next_job = 0; end_k = 0x7fffffff; }
+  for (int t = threadIdx.x; t < kStreamRing; t += kRB) { sh.tiles[t] = 0; sh.px_done[t] = 0; }
+  if (threadIdx.x == 0) { sh.next_job = 0; sh.end_k = 0x7fffffff; }
   __syncthreads();
 
-  RenderCounters rc;
   CastCounters *cc = kStats ? &rc.cast : nullptr;
   const uint32_t samp0 = (uint32_t)(P.iteration > 1 ? P.iteration - 1 : 0) * (uint32_t)spp;
   const float spw = uni(1.0f / (((float)P.fsaa_x) * ((float)P.fsaa_y)));
@@ -696,9 +699,9 @@ __global__ __launch_bounds__(kRB, kRenderWaves) void k_render_stream(DevTree T, 
   auto pixel_written = [&](const float a[3]) {
     const int kk = (u >> tile_shift) & (kStreamRing - 1);
     // (the tile's ring entry stays until every pixel of the tile is written)
-    const int e = *(volatile int *)&tiles[kk];
+    const int e = lds_get(&sh.tiles[kk]);
     if (ps.pixel() != kNoPixel) store_pixel(K, frame, tile_block(e), tile_pixel(e, u), a);
-    atomicAdd(&px_done[kk], 1);
+    atomicAdd(&sh.px_done[kk], 1);
   };
   for (;;) {
     // ---- path updates of the finished casts, batched.  The thresholds here and of the leaf tests are
@@ -736,7 +739,7 @@ __global__ __launch_bounds__(kRB, kRenderWaves) void k_render_stream(DevTree T, 
                 for (int j = 0; j < 3; j++) a[j] += src[3 * k + j] * spw;
               pixel_written(a);
               __threadfence_block();
-              *(volatile int *)&turn[slot] = (((left >> 9) + 1) << 9) | spp;
+              lds_put(&turn[slot], (((left >> 9) + 1) << 9) | spp);
             }
           }
           live = false;
@@ -750,30 +753,30 @@ __global__ __launch_bounds__(kRB, kRenderWaves) void k_render_stream(DevTree T, 
     if (qpos == qlen && !ended) {
       if (!taken) {
         unsigned q = 0;
-        if (lane == 0) q = atomicAdd(&next_job, (unsigned)chunk);
+        if (lane == 0) q = atomicAdd(&sh.next_job, (unsigned)chunk);
         qbase = (unsigned)__builtin_amdgcn_readfirstlane((int)q);
         taken = true;
       }
       // the tile of these jobs (wave-uniform); its first jobs' wave fetches its id once the tile before has one
       const int k = uni((int)udiv(qbase, Dspp)) >> tile_shift;
       const int kk = k & (kStreamRing - 1);
-      bool past = k >= uni(*(volatile int *)&end_k);
+      bool past = k >= uni(lds_get(&sh.end_k));
       int e = 0;
-      if (!past && uni(*(volatile int *)&px_done[kk]) >= (k / kStreamRing) << tile_shift) {   // the ring entry is tile k's
-        e = uni(*(volatile int *)&tiles[kk]);
+      if (!past && uni(lds_get(&sh.px_done[kk])) >= (k / kStreamRing) << tile_shift) {   // the ring entry is tile k's
+        e = uni(lds_get(&sh.tiles[kk]));
         if ((e & 0xff) != (k & 0xff)) e = 0;
         if (e == 0 && qbase == (unsigned)((k << tile_shift) * spp)) {
-          const int prev = k > 0 ? uni(*(volatile int *)&tiles[(k - 1) & (kStreamRing - 1)]) : 0;
+          const int prev = k > 0 ? uni(lds_get(&sh.tiles[(k - 1) & (kStreamRing - 1)])) : 0;
           if (k == 0 || (prev != 0 && (prev & 0xff) == ((k - 1) & 0xff))) {
             int id = 0;
-            if (lane == 0) id = (int)atomicAdd(work, 1u);
+            if (lane == 0) id = (int)atomicAdd(next_tile, 1u);
             id = __builtin_amdgcn_readfirstlane(id);
             if (id >= ntiles) {
-              if (lane == 0) atomicMin(&end_k, k);
+              if (lane == 0) atomicMin(&sh.end_k, k);
               past = true;
             } else {
               e = ((id + 1) << 8) | (k & 0xff);
-              if (lane == 0) *(volatile int *)&tiles[kk] = e;
+              if (lane == 0) lds_put(&sh.tiles[kk], e);
             }
           }
         }
@@ -803,7 +806,7 @@ __global__ __launch_bounds__(kRB, kRenderWaves) void k_render_stream(DevTree T, 
     }
     // ---- idle lanes pop the next entries whose pixel slot is free
     const uint64_t idle = __ballot(!live);
-    if (qpos < qlen && idle && (__popcll(idle) >= PathT::kStreamRefillMin || idle == ~0ull)) {
+    if (qpos < qlen && idle && (__popcll(idle) >= refill_min || idle == ~0ull)) {
       const int entry = qpos + __popcll(idle & below);
       const bool some = !live && entry < qlen;
       int uq = 0;
@@ -811,7 +814,7 @@ __global__ __launch_bounds__(kRB, kRenderWaves) void k_render_stream(DevTree T, 
       if (some) {
         uq = __float_as_int(queue[4 * 64 + entry]);
         // (turns are compared in the 23 bits a slot's word keeps)
-        free = nslots == 0 || (((*(volatile int *)&turn[uq & (nslots - 1)] >> 9) ^ (uq >> slot_shift)) & 0x7fffff) == 0;
+        free = nslots == 0 || (((lds_get(&turn[uq & (nslots - 1)]) >> 9) ^ (uq >> slot_shift)) & 0x7fffff) == 0;
       }
       const uint64_t stuck = __ballot(some && !free);
       const bool take = some && (stuck == 0 || lane < __ffsll((unsigned long long)stuck) - 1);
@@ -847,9 +850,23 @@ __global__ __launch_bounds__(kRB, kRenderWaves) void k_render_stream(DevTree T, 
     if (pm && (__popcll(pm) * (64 / kLeafMin) >= __popcll(__ballot(live)) || __ballot(live && w.state == kWalkTrace) == 0))
       walk_leaf_wave(T, w, pend, clip, leaf, ins, cc);
   }
+}
+
+template <class PathT, bool kStats>
+__global__ __launch_bounds__(kRB, kRenderWaves) void k_render_stream(DevTree T, Tables tb, dr_render_params P,
+                                                                      FrameK K, float *__restrict__ frame, int start_block,
+                                                                      StreamShape S, int levels,
+                                                                      unsigned *__restrict__ work,
+                                                                      unsigned long long *__restrict__ counts) {
+  extern __shared__ __align__(16) uint32_t lds[];
+  __shared__ StreamLds sh;
+  __shared__ int ins_all[kStats ? kRB : 1];
+  RenderCounters rc;
+  stream_paths<PathT, kStats>(T, tb, P, K, frame, start_block, S, levels, work, PathT::kStreamRefillMin, lds, sh,
+                              kStats ? ins_all + (threadIdx.x & ~63u) : nullptr, rc);
   if (kStats) flush_counters(rc, counts);
   // ---- the last wave out resets the block counter for the next launch
-  if (lane == 0) {
+  if (__lane_id() == 0) {
     __threadfence();
     const unsigned total = gridDim.x * (kRB / 64);
     if (atomicAdd(work + 1, 1u) == total - 1) {
@@ -1180,11 +1197,63 @@ struct DevRequest {
 };
 
 __global__ void k_zero(int *counter, int n) {
-  if (blockIdx.x == 0 && (int)threadIdx.x < n) counter[threadIdx.x] = 0;
+  for (int i = (int)threadIdx.x; i < n; i += (int)blockDim.x) counter[i] = 0;
 }
 
-// Persistent workgroups drain the queue of (request, first block, block count) items
-// of the requests of one plugin set.
+// A request of a batch as a stream; `weight`: the relative cost of a tile.
+struct StreamRequest {
+  int req;
+  float weight;
+  StreamShape S;
+};
+
+// The streamed requests of one plugin set: persistent workgroups, spread over the requests by cost
+// (first[workgroup]), each run one request's stream until its tiles are gone and then join the one
+// with the most work left.  A workgroup waits for its longest path once per request it works on.
+// (One block at a time from a queue of (request, blocks) items it did so for every block: 24 requests
+// of 128^2 to 512^2 at 1 to 16 spp 8.5 -> 6.5 ms.)
+template <class PathT>
+__global__ __launch_bounds__(kRB, kRenderWaves) void k_batch_stream(const DevRequest *__restrict__ reqs,
+                                                                    const StreamRequest *__restrict__ list, int n,
+                                                                    const int *__restrict__ first,
+                                                                    unsigned *__restrict__ next_tile, int levels,
+                                                                    int refill_min) {
+  extern __shared__ __align__(16) uint32_t lds[];
+  __shared__ StreamLds sh;
+  __shared__ int pick;
+  int i = first[blockIdx.x];
+  RenderCounters rc;
+  for (;;) {
+    i = uni(i);
+    // the requests are read-only while the kernel runs: the constant address space keeps their loads scalar
+    typedef const __attribute__((address_space(4))) DevRequest *ConstRequest;
+    const StreamRequest E = list[i];
+    const DevRequest &R = *(const DevRequest *)(ConstRequest)(uintptr_t)&reqs[uni(E.req)];
+    const Tables tb = {R.shade, R.faces};
+    const StreamShape S = {uni(E.S.ntiles), uni(E.S.tile_shift), uni(E.S.chunk), uni(E.S.slot_shift)};
+    stream_paths<PathT, false>(R.T, tb, R.P, R.K, R.frame, 0, S, levels, next_tile + i, refill_min, lds, sh, nullptr, rc);
+    // the request with the most work left
+    if (threadIdx.x < 64) {
+      int best = 0, at = -1;
+      for (int j = (int)threadIdx.x; j < n; j += 64) {
+        const int left = list[j].S.ntiles - (int)__hip_atomic_load(&next_tile[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const int key = left > 0 ? __float_as_int((float)left * list[j].weight) : 0;   // (positive floats order as ints)
+        if (key > best) { best = key; at = j; }
+      }
+      const int top = __builtin_amdgcn_readlane(wave_incl_max(best), 63);
+      const uint64_t who = __ballot(top > 0 && best == top);
+      if (threadIdx.x == 0) pick = -1;
+      if (who && (int)threadIdx.x == __ffsll((unsigned long long)who) - 1) pick = at;
+    }
+    __syncthreads();
+    i = pick;
+    if (i < 0) break;
+    __syncthreads();
+  }
+}
+
+// Requests of more than kStreamMaxSpp samples a pixel: persistent workgroups drain a queue of (request,
+// first block, block count) items, one block at a time.
 template <class PathT>
 __global__ __launch_bounds__(kRB, kRenderWaves) void k_batch(const DevRequest *__restrict__ reqs, const int4 *__restrict__ items,
                                                 int nitems, int *__restrict__ counter, int levels, int refill_min) {
@@ -1242,6 +1311,54 @@ static Tables tables_of(dr_scene s, const dr_render_params *p) {
 }  // namespace dr
 
 namespace dr {
+// Pixel slots of a stream, and the workgroups per CU of kernel `kern` with them.  Deep trees, whose
+// stacks leave no room for all the slots beside the registers' three workgroups a CU, get half the
+// slots if that gives a workgroup more (1080p 16 spp: 15.8 ms with 2,048 samples staged and three,
+// 17.6 ms with 1,024 and three, 22.4 ms with 2,048 and two).
+static int stream_slots(const void *kern, int levels, int spp, bool origins, int &slot_shift, int &per_cu) {
+  slot_shift = stream_slot_shift(spp, kStreamSamples);
+  const size_t all = stream_lds(levels, spp, slot_shift, origins);
+  if (all > 64 * 1024)
+    DR_HIP_CHECK(hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)all));
+  DR_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, kRB, all));
+  if (per_cu < kRenderWaves && slot_shift > 3) {
+    int more = 0;
+    DR_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&more, kern, kRB,
+                                                              stream_lds(levels, spp, slot_shift - 1, origins)));
+    if (more > per_cu) {
+      per_cu = more;
+      slot_shift--;
+    }
+  }
+  return DR_OK;
+}
+
+// The stream of `nblocks` blocks over `resident` workgroups.
+// Tiles: 32 a workgroup, so that the last ones even out over the chip, but of at least 64 jobs: a
+// tile costs an atomic on one address and its waves wait for its id.  (Whole blocks: 517x389 at
+// 1 spp 968 us, 256x256 at 4 spp 461 us in one block per workgroup, 1080p at 16 spp 17.7 ms; so:
+// 720 us, 308 us, 15.8 ms.  Tiles of 32 jobs: 910 us, 345 us; 8 a workgroup: 17.1 ms at 1080p.)
+// Jobs a wave takes at a time: 1/32 of its share, between 8 and 64 (a wave's queue is its own: at
+// the end of a small frame its entries wait while other waves are idle; 517x389 at 1 spp 784 us
+// with 16, 715 us with 8), and a divisor of a tile's.
+static StreamShape stream_shape(long long nblocks, int spp, int slot_shift, double resident) {
+  StreamShape S;
+  S.slot_shift = slot_shift;
+  S.tile_shift = 7;
+  while (S.tile_shift > 3 && (spp << S.tile_shift) >= 128 && (double)(nblocks << (7 - S.tile_shift)) < 32 * resident)
+    S.tile_shift--;
+  S.ntiles = (int)(nblocks << (7 - S.tile_shift));
+  const double groups = std::min((double)S.ntiles, resident);
+  const double per_wave = (double)nblocks * kBlockPixels * spp / (groups * (kRB / 64));
+  S.chunk = 64;
+  while (S.chunk > 8 && (S.chunk > per_wave / 32 || (spp << S.tile_shift) % S.chunk != 0)) S.chunk /= 2;
+  return S;
+}
+// Whether a render of `nblocks` blocks up to block `end_block` takes the streamed kernels.
+static bool streams(long long nblocks, int end_block, int spp) {
+  return spp <= kStreamMaxSpp && (nblocks + 4) * kBlockPixels * spp < (1ll << 31) && end_block < (1 << 23);
+}
+
 static int launch_render(dr_scene s, const dr_render_params *p, float *frame, int start_block, int end_block,
                          unsigned long long *counts, void *stream) {
   int rc = check_params(s, p);
@@ -1256,47 +1373,19 @@ static int launch_render(dr_scene s, const dr_render_params *p, float *frame, in
   // streamed tiles (k_render_stream) unless the sample count or the stream length is too large; one
   // block per workgroup otherwise
   const long long nrange = end_block - start_block;
-  if (spp <= kStreamMaxSpp && (nrange + 4) * kBlockPixels * spp < (1ll << 31) && end_block < (1 << 23)) {
+  if (streams(nrange, end_block, spp)) {
     const bool origins = p->lens == DR_SPHERICAL_SEGMENT_LENS;
     auto kern = counts ? (ref ? k_render_stream<RefPath, true> : k_render_stream<BenchPath, true>)
                        : (ref ? k_render_stream<RefPath, false> : k_render_stream<BenchPath, false>);
-    int slot_shift = stream_slot_shift(spp, kStreamSamples), per_cu = 0;
-    size_t lds_s = stream_lds(levels, spp, slot_shift, origins);
-    if (lds_s > 64 * 1024)
-      DR_HIP_CHECK(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_s));
-    DR_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, kRB, lds_s));
-    // deep trees, whose stacks leave no room for all the slots beside the registers' three workgroups a
-    // CU: half the slots if that gives a workgroup more (1080p 16 spp: 15.8 ms with 2,048 samples
-    // staged and three, 17.6 ms with 1,024 and three, 22.4 ms with 2,048 and two)
-    if (per_cu < kRenderWaves && slot_shift > 3) {
-      const size_t half = stream_lds(levels, spp, slot_shift - 1, origins);
-      int more = 0;
-      DR_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&more, kern, kRB, half));
-      if (more > per_cu) {
-        per_cu = more;
-        lds_s = half;
-        slot_shift--;
-      }
-    }
+    int slot_shift, per_cu;
+    if ((rc = stream_slots((const void *)kern, levels, spp, origins, slot_shift, per_cu)) != DR_OK) return rc;
+    const size_t lds_s = stream_lds(levels, spp, slot_shift, origins);
     const long long resident = (long long)s->num_cu * std::max(per_cu, 1);
-    // Tiles: 32 a workgroup, so that the last ones even out over the chip, but of at least 64 jobs: a
-    // tile costs an atomic on one address and its waves wait for its id.  (Whole blocks: 517x389 at
-    // 1 spp 968 us, 256x256 at 4 spp 461 us in one block per workgroup, 1080p at 16 spp 17.7 ms; so:
-    // 715 us, 310 us, 15.9 ms.  Tiles of 32 jobs: 910 us, 345 us; 8 a workgroup: 17.1 ms at 1080p.)
-    int tile_shift = 7;
-    while (tile_shift > 3 && (spp << tile_shift) >= 128 && (nrange << (7 - tile_shift)) < 32 * resident) tile_shift--;
-    const long long ntiles = nrange << (7 - tile_shift);
-    const long long groups = std::min<long long>(ntiles, resident);
-    // jobs a wave takes at a time: 1/32 of its share, between 8 and 64 (a wave's queue is its own: at
-    // the end of a small frame its entries wait while other waves are idle; 517x389 at 1 spp 784 us
-    // with 16, 715 us with 8), and a divisor of a tile's
-    const long long per_wave = nrange * kBlockPixels * spp / (groups * (kRB / 64));
-    int chunk = 64;
-    while (chunk > 8 && (chunk > per_wave / 32 || (spp << tile_shift) % chunk != 0)) chunk /= 2;
+    const StreamShape S = stream_shape(nrange, spp, slot_shift, (double)resident);
+    const long long groups = std::min<long long>(S.ntiles, resident);
     unsigned *work = (unsigned *)s->work.p + 2 * (s->work_slot.fetch_add(1) % kWorkSlots);
     hipLaunchKernelGGL(kern, dim3((unsigned)groups), dim3(kRB), lds_s, (hipStream_t)stream, s->tree, tb, *p, frame_k(*p),
-                       frame, start_block, (int)ntiles, tile_shift, chunk, slot_shift, levels, work,
-                       counts);
+                       frame, start_block, S, levels, work, counts);
     DR_HIP_CHECK(hipGetLastError());
     return DR_OK;
   }
@@ -1452,10 +1541,19 @@ extern "C" int dr_backward(dr_scene s, const dr_render_params *p, const float *d
 
 // ------------------------------------------------------------------ batch host side
 struct dr_batch_s {
-  int n = 0, levels = 1, num_cu = 1;
-  int nitems[2] = {0, 0};          // work items of the benchmark / reference plugin requests
-  dr_batch_tuning tuning{1, 2, 1};
-  dr::DevBuf reqs, items[2], counter;
+  int num_cu = 1;
+  int levels = 1;                  // of the deepest tree
+  dr_batch_tuning tuning{1, 1, 1};
+  dr::DevBuf reqs, counters;       // counters: one per streamed request and plugin set, then one per item queue
+  struct Streams {                 // the streamed requests of a plugin set
+    int n = 0;
+    size_t lds = 0;
+    dr::DevBuf list, first;
+  } streams[2];
+  struct Items {                   // work items of the others
+    int n = 0;
+    dr::DevBuf list;
+  } items[2];
   std::vector<dr::DevRequest> host_reqs;
   std::vector<dr_scene> scenes;      // references held until dr_batch_destroy
   std::vector<dr_shading> shadings;
@@ -1469,17 +1567,25 @@ namespace dr {
 static size_t batch_lds(int levels) {
   return ((size_t)levels * kStackWordsPerLevel * kRB + (size_t)kBlockPixels * kRoundSamples * 3) * 4;
 }
+static bool request_streams(const dr_render_params &P) {
+  const int nb = block_count(&P);
+  return streams(nb, nb, P.fsaa_x * P.fsaa_y);
+}
+// Relative cost of a pixel of a request.
+static double pixel_cost(const dr_render_params &P) {
+  return (double)P.fsaa_x * P.fsaa_y * (1.0 + P.max_bounces) * (1.0 + P.nlights);
+}
 
 // Queue of (request, first block, count) of the requests of plugin set `set` (0 =
-// benchmark, 1 = reference), heaviest per-block cost first.
+// benchmark, 1 = reference) that are not streamed, heaviest per-block cost first.
 static std::vector<int4> make_items(const std::vector<DevRequest> &R, int tile, int set) {
   std::vector<std::pair<double, int4>> v;
   for (int r = 0; r < (int)R.size(); r++) {
     const dr_render_params &P = R[r].P;
-    if ((P.plugins == DR_PLUGINS_REFERENCE) != (set == 1)) continue;
+    if ((P.plugins == DR_PLUGINS_REFERENCE) != (set == 1) || request_streams(P)) continue;
     const int nb = block_count(&P);
-    const double cost = (double)P.fsaa_x * P.fsaa_y * (1.0 + P.max_bounces) * (1.0 + P.nlights);
-    for (int b = 0; b < nb; b += tile) v.push_back({cost * std::min(tile, nb - b), make_int4(r, b, std::min(tile, nb - b), 0)});
+    for (int b = 0; b < nb; b += tile)
+      v.push_back({pixel_cost(P) * std::min(tile, nb - b), make_int4(r, b, std::min(tile, nb - b), 0)});
   }
   std::stable_sort(v.begin(), v.end(), [](const std::pair<double, int4> &a, const std::pair<double, int4> &b) {
     return a.first > b.first;
@@ -1490,99 +1596,68 @@ static std::vector<int4> make_items(const std::vector<DevRequest> &R, int tile, 
   return out;
 }
 
-// Queue resets, then one persistent kernel per plugin set that has requests (the
-// reference estimator's kernel after the benchmark one, on the same stream).
-static int launch_batch(const DevRequest *reqs_dev, const int4 *const items_dev[2], const int nitems[2], int *counter,
-                        int levels, const dr_batch_tuning &t, int num_cu, hipStream_t stream) {
-  hipLaunchKernelGGL(k_zero, dim3(1), dim3(64), 0, stream, counter, 2);
-  const dim3 grid(num_cu * t.groups_per_cu);
-  if (nitems[0] > 0)
-    hipLaunchKernelGGL(k_batch<BenchPath>, grid, dim3(kRB), batch_lds(levels), stream, reqs_dev, items_dev[0],
-                       nitems[0], counter, levels, t.refill_min);
-  if (nitems[1] > 0)
-    hipLaunchKernelGGL(k_batch<RefPath>, grid, dim3(kRB), batch_lds(levels), stream, reqs_dev, items_dev[1],
-                       nitems[1], counter + 1, levels, t.refill_min);
+// The streamed requests of plugin set `set`: their shapes, and the request each workgroup starts with.
+static int make_streams(dr_batch b, int set) {
+  dr_batch_s::Streams &st = b->streams[set];
+  const void *kern = set == 0 ? (const void *)k_batch_stream<BenchPath> : (const void *)k_batch_stream<RefPath>;
+  std::vector<int> ids;
+  double total = 0.0;
+  for (int r = 0; r < (int)b->host_reqs.size(); r++) {
+    const dr_render_params &P = b->host_reqs[r].P;
+    if ((P.plugins == DR_PLUGINS_REFERENCE) != (set == 1) || !request_streams(P)) continue;
+    ids.push_back(r);
+    total += pixel_cost(P) * block_count(&P);
+  }
+  st.n = (int)ids.size();
+  if (st.n == 0) return DR_OK;
+  const int grid = b->num_cu * b->tuning.groups_per_cu;
+  std::vector<StreamRequest> list(st.n);
+  std::vector<int> first(grid);
+  double before = 0.0;
+  for (int i = 0, g = 0; i < st.n; i++) {
+    const dr_render_params &P = b->host_reqs[ids[i]].P;
+    const int spp = P.fsaa_x * P.fsaa_y;
+    const bool origins = P.lens == DR_SPHERICAL_SEGMENT_LENS;
+    int slot_shift, per_cu;
+    const int rc = stream_slots(kern, b->levels, spp, origins, slot_shift, per_cu);
+    if (rc != DR_OK) return rc;
+    st.lds = std::max(st.lds, stream_lds(b->levels, spp, slot_shift, origins));
+    const double cost = pixel_cost(P) * block_count(&P);
+    list[i].req = ids[i];
+    list[i].S = stream_shape(block_count(&P), spp, slot_shift, std::max(1.0, grid * cost / total));
+    list[i].weight = (float)(pixel_cost(P) * (1 << list[i].S.tile_shift));
+    before += cost;
+    // workgroup g starts with the request that holds the share (g + 1/2) / grid of the cost
+    for (; g < grid && (i == st.n - 1 || (g + 0.5) * total < before * grid); g++) first[g] = i;
+  }
+  int rc = dev_upload(st.list, list.data(), list.size() * sizeof(StreamRequest));
+  if (rc == DR_OK) rc = dev_upload(st.first, first.data(), first.size() * sizeof(int));
+  return rc;
+}
+
+// Counter resets, then the persistent kernels of the plugin sets that have requests (one after the
+// other on the stream).
+static int launch_batch(dr_batch b, hipStream_t stream) {
+  int *counters = (int *)b->counters.p;
+  const int n0 = b->streams[0].n, ncounters = n0 + b->streams[1].n + 2;
+  const DevRequest *reqs = (const DevRequest *)b->reqs.p;
+  hipLaunchKernelGGL(k_zero, dim3(1), dim3(256), 0, stream, counters, ncounters);
+  const dim3 grid(b->num_cu * b->tuning.groups_per_cu);
+  for (int set = 0; set < 2; set++) {
+    const dr_batch_s::Streams &st = b->streams[set];
+    if (st.n == 0) continue;
+    hipLaunchKernelGGL(set == 0 ? k_batch_stream<BenchPath> : k_batch_stream<RefPath>, grid, dim3(kRB), st.lds, stream, reqs,
+                       (const StreamRequest *)st.list.p, st.n, (const int *)st.first.p,
+                       (unsigned *)counters + (set == 0 ? 0 : n0), b->levels, b->tuning.refill_min);
+  }
+  for (int set = 0; set < 2; set++) {
+    const dr_batch_s::Items &it = b->items[set];
+    if (it.n == 0) continue;
+    hipLaunchKernelGGL(set == 0 ? k_batch<BenchPath> : k_batch<RefPath>, grid, dim3(kRB), batch_lds(b->levels), stream, reqs,
+                       (const int4 *)it.list.p, it.n, counters + ncounters - 2 + set, b->levels, b->tuning.refill_min);
+  }
   DR_HIP_CHECK(hipGetLastError());
   return DR_OK;
-}
-
-// Times one tuning on the proxy (every request at 1x1 spp, iteration 1, scratch frames).
-static int time_tuning(const std::vector<DevRequest> &proxy, const dr_batch_tuning &t, int levels, int num_cu,
-                       hipStream_t stream, DevBuf &reqs_dev, DevBuf items_dev[2], int *counter, float &ms) {
-  int nitems[2];
-  const int4 *items_p[2];
-  int rc = DR_OK;
-  for (int set = 0; set < 2 && rc == DR_OK; set++) {
-    const std::vector<int4> items = make_items(proxy, t.tile_blocks, set);
-    nitems[set] = (int)items.size();
-    dev_free(items_dev[set]);
-    rc = dev_upload(items_dev[set], items.data(), items.size() * sizeof(int4));
-    items_p[set] = (const int4 *)items_dev[set].p;
-  }
-  if (rc != DR_OK) return rc;
-  hipEvent_t e0, e1;
-  DR_HIP_CHECK(hipEventCreate(&e0));
-  DR_HIP_CHECK(hipEventCreate(&e1));
-  rc = launch_batch((const DevRequest *)reqs_dev.p, items_p, nitems, counter, levels, t, num_cu, stream);
-  if (rc == DR_OK) {
-    DR_HIP_CHECK(hipEventRecord(e0, stream));
-    for (int k = 0; k < 2 && rc == DR_OK; k++)
-      rc = launch_batch((const DevRequest *)reqs_dev.p, items_p, nitems, counter, levels, t, num_cu, stream);
-    DR_HIP_CHECK(hipEventRecord(e1, stream));
-    DR_HIP_CHECK(hipEventSynchronize(e1));
-    DR_HIP_CHECK(hipEventElapsedTime(&ms, e0, e1));
-  }
-  (void)hipEventDestroy(e0);
-  (void)hipEventDestroy(e1);
-  return rc;
-}
-
-static int autotune(const std::vector<DevRequest> &R, int levels, int num_cu, hipStream_t stream,
-                    dr_batch_tuning &best) {
-  std::vector<DevRequest> proxy = R;
-  std::vector<DevBuf> frames(R.size());
-  int rc = DR_OK;
-  for (size_t r = 0; r < R.size() && rc == DR_OK; r++) {
-    proxy[r].P.fsaa_x = proxy[r].P.fsaa_y = 1;
-    proxy[r].P.iteration = 1;
-    proxy[r].K = frame_k(proxy[r].P);
-    frames[r].bytes = (size_t)block_count(&R[r].P) * kBlockPixels * 16;
-    hipError_t e = hipMalloc(&frames[r].p, frames[r].bytes);
-    if (e != hipSuccess) { frames[r].p = nullptr; rc = fail(DR_ERR_ALLOC, "dr_batch_create: scratch frames"); }
-    proxy[r].frame = (float *)frames[r].p;
-  }
-  DevBuf reqs_dev, items_dev[2], counter;
-  if (rc == DR_OK) rc = dev_upload(reqs_dev, proxy.data(), proxy.size() * sizeof(DevRequest));
-  const int zero[2] = {0, 0};
-  if (rc == DR_OK) rc = dev_upload(counter, zero, sizeof(zero));
-  best = dr_batch_tuning{1, 2, kRenderRefillMin};
-  float best_ms = 0.0f;
-  if (rc == DR_OK) rc = time_tuning(proxy, best, levels, num_cu, stream, reqs_dev, items_dev, (int *)counter.p, best_ms);
-  // coordinate descent: tile, then persistent groups per CU, then refill cadence (on the
-  // 64-request benchmark mix, refills of 1, 4, 8 and 16 idle lanes measured 286.2, 284.8,
-  // 283.3 and 283.3 ms; the 1-spp proxy cannot rank values that close, so the candidates
-  // stay near the best)
-  const int tiles[] = {1, 2, 4, 8}, groups[] = {1, 2, 3, 4}, refills[] = {4, 8, 16};
-  for (int axis = 0; axis < 3 && rc == DR_OK; axis++) {
-    const int *vals = axis == 0 ? tiles : (axis == 1 ? groups : refills);
-    const int nv = axis == 2 ? 3 : 4;
-    dr_batch_tuning base = best;
-    for (int i = 0; i < nv && rc == DR_OK; i++) {
-      dr_batch_tuning t = base;
-      int &field = axis == 0 ? t.tile_blocks : (axis == 1 ? t.groups_per_cu : t.refill_min);
-      if (field == vals[i]) continue;
-      field = vals[i];
-      float ms = 0.0f;
-      rc = time_tuning(proxy, t, levels, num_cu, stream, reqs_dev, items_dev, (int *)counter.p, ms);
-      if (rc == DR_OK && ms < best_ms) { best_ms = ms; best = t; }
-    }
-  }
-  dev_free(reqs_dev);
-  dev_free(items_dev[0]);
-  dev_free(items_dev[1]);
-  dev_free(counter);
-  for (auto &f : frames) dev_free(f);
-  return rc;
 }
 
 }  // namespace dr
@@ -1618,31 +1693,29 @@ extern "C" int dr_batch_create(const dr_request *reqs, int n, const dr_batch_tun
     int dev = 0;
     (void)hipGetDevice(&dev);
     if (hipDeviceGetAttribute(&b->num_cu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) b->num_cu = 1;
-    b->n = n;
     if (hipStreamCreate(&b->cap_stream) != hipSuccess) rc = dr::fail(DR_ERR_HIP, "dr_batch_create: stream");
   }
   if (rc == DR_OK) {
-    if (tuning) b->tuning = *tuning;
-    else rc = dr::autotune(b->host_reqs, b->levels, b->num_cu, b->cap_stream, b->tuning);
+    // by default as many workgroups as the registers allow and the streamed kernels' refill
+    b->tuning = tuning ? *tuning : dr_batch_tuning{1, dr::kRenderWaves, dr::BenchPath::kStreamRefillMin};
+    if (b->tuning.tile_blocks < 1 || b->tuning.groups_per_cu < 1 || b->tuning.refill_min < 1)
+      rc = dr::fail(DR_ERR_ARG, "dr_batch_create: tuning values must be >= 1");
   }
-  if (rc == DR_OK && (b->tuning.tile_blocks < 1 || b->tuning.groups_per_cu < 1 || b->tuning.refill_min < 1))
-    rc = dr::fail(DR_ERR_ARG, "dr_batch_create: tuning values must be >= 1");
   if (rc == DR_OK) {
     rc = dr::dev_upload(b->reqs, b->host_reqs.data(), b->host_reqs.size() * sizeof(dr::DevRequest));
     for (int set = 0; set < 2 && rc == DR_OK; set++) {
       const std::vector<int4> items = dr::make_items(b->host_reqs, b->tuning.tile_blocks, set);
-      b->nitems[set] = (int)items.size();
-      rc = dr::dev_upload(b->items[set], items.data(), items.size() * sizeof(int4));
+      b->items[set].n = (int)items.size();
+      rc = dr::dev_upload(b->items[set].list, items.data(), items.size() * sizeof(int4));
+      if (rc == DR_OK) rc = dr::make_streams(b, set);
     }
-    const int zero[2] = {0, 0};
-    if (rc == DR_OK) rc = dr::dev_upload(b->counter, zero, sizeof(zero));
+    const std::vector<int> zeros(b->streams[0].n + b->streams[1].n + 2, 0);
+    if (rc == DR_OK) rc = dr::dev_upload(b->counters, zeros.data(), zeros.size() * sizeof(int));
   }
   if (rc == DR_OK) {
     hipError_t e = hipStreamBeginCapture(b->cap_stream, hipStreamCaptureModeThreadLocal);
     if (e == hipSuccess) {
-      const int4 *items_p[2] = {(const int4 *)b->items[0].p, (const int4 *)b->items[1].p};
-      rc = dr::launch_batch((const dr::DevRequest *)b->reqs.p, items_p, b->nitems, (int *)b->counter.p, b->levels,
-                            b->tuning, b->num_cu, b->cap_stream);
+      rc = dr::launch_batch(b, b->cap_stream);
       hipError_t e2 = hipStreamEndCapture(b->cap_stream, &b->graph);
       if (rc == DR_OK && e2 != hipSuccess) rc = dr::fail(DR_ERR_HIP, "dr_batch_create: graph capture");
       if (rc == DR_OK && hipGraphInstantiate(&b->exec, b->graph, nullptr, nullptr, 0) != hipSuccess)
@@ -1674,9 +1747,12 @@ extern "C" void dr_batch_destroy(dr_batch b) {
   if (b->graph) (void)hipGraphDestroy(b->graph);
   if (b->cap_stream) (void)hipStreamDestroy(b->cap_stream);
   dr::dev_free(b->reqs);
-  dr::dev_free(b->items[0]);
-  dr::dev_free(b->items[1]);
-  dr::dev_free(b->counter);
+  for (int set = 0; set < 2; set++) {
+    dr::dev_free(b->items[set].list);
+    dr::dev_free(b->streams[set].list);
+    dr::dev_free(b->streams[set].first);
+  }
+  dr::dev_free(b->counters);
   for (dr_shading h : b->shadings) dr::shading_release(h);
   for (dr_scene sc : b->scenes) dr::scene_release(sc);
   delete b;

@@ -290,8 +290,8 @@ typedef struct {
 
 /* Launch shape of the batched kernel. */
 typedef struct {
-  int32_t tile_blocks;     /* framebuffer blocks per work item of the device queue */
-  int32_t groups_per_cu;   /* persistent workgroups per compute unit draining the queue */
+  int32_t tile_blocks;     /* framebuffer blocks per queue item (requests above 256 samples a pixel) */
+  int32_t groups_per_cu;   /* persistent workgroups per compute unit */
   int32_t refill_min;      /* idle lanes a wave collects before it takes new path jobs */
 } dr_batch_tuning;
 
@@ -299,12 +299,13 @@ typedef struct dr_batch_s *dr_batch;
 
 /* Many renders in one persistent launch (replaces BlockRenderer's per-device block
  * batches and host round trips, BlockRenderer.cu:74-97, FrameBuffer.impl.cuh:261-268,
- * 355-379).  Work items (request, tile of blocks) are queued longest first and
- * drained by persistent workgroups through one device atomic; the launch (queue
- * reset + kernel) is captured once in a hipGraph.  tuning == NULL runs the autotuner
- * (timed proxy renders into scratch frames; request frames are not touched).
+ * 355-379).  Persistent workgroups are spread over the requests by their cost; each runs one
+ * request's tiles as a stream until they are gone and then joins the request with the most
+ * work left (requests of more than 256 samples a pixel: a queue of blocks, longest first).
+ * The launch (counter reset + kernels) is captured once in a hipGraph.  tuning == NULL takes
+ * the library's own choice.
  * Requests of both plugin sets and every lens may be mixed: each plugin set has its own
- * queue and persistent kernel, launched one after the other in the same graph.
+ * persistent kernel, launched one after the other in the same graph.
  * Every request's frame equals what dr_render_blocks would produce for it. */
 int dr_batch_create(const dr_request *reqs, int n, const dr_batch_tuning *tuning, dr_batch *out);
 /* Replays the captured graph on `stream`. */

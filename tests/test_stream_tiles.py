@@ -150,3 +150,33 @@ def test_streamed_frame_equals_one_block_kernel(dev, width, height, spp, lens):
         torch.cuda.synchronize()
         bits = [f.data.cpu().numpy().view(np.int32) for f in frames]
         assert np.array_equal(bits[0], bits[1]) and np.array_equal(bits[0], bits[2]), iteration
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tuning", [None, dict(tile_blocks=3, groups_per_cu=1, refill_min=16),
+                                    dict(tile_blocks=1, groups_per_cu=4, refill_min=1)])
+def test_batch_of_streams_and_rounds(dev, tuning):
+    """One batch with streamed requests of every slot count, requests above the streamed kernel's 256
+    samples a pixel, and more requests than one wave looks over: each frame is its solo frame."""
+    import torch
+    import dumbray_amd as D
+    from dumbray_amd import plugins as PL
+    from dumbray_amd import scenes as S
+    sc = S.spheres_scene(4, seed=1)
+    tree = D.Octree(16, 12)
+    tree.push(sc.tris)
+    scene = tree.build().upload()
+    shapes = [(40, 24, (1, 1)), (24, 40, (17, 16)), (33, 17, (16, 16)), (130, 70, (2, 1)), (8, 16, (20, 20))]
+    shapes += [(8 + k % 5, 16 + k % 3, (1 + k % 3, 1)) for k in range(70)]
+    rs = [D.DumbRenderer(scene, sc.mat_id, sc.materials, sc.lights if k % 4 else [PL.spherical_light((9.0, 9.0, 9.0), (0.0, 5.0, 0.0), 0.5)],
+                         sc.camera, w, h, spp, 2, seed=k) for k, (w, h, spp) in enumerate(shapes)]
+    print(f"[case] batch of {len(rs)} streams and rounds, {tuning}", flush=True)
+    frames = [D.BlockBasedFrameBuffer(r.width, r.height) for r in rs]
+    batch = D.RenderBatch([(r, f, 1, 0) for r, f in zip(rs, frames)], tuning)
+    for replay in range(3):
+        for f in frames:
+            f.data.zero_()
+        batch.run()
+        torch.cuda.synchronize()
+        for k, (r, f) in enumerate(zip(rs, frames)):
+            assert torch.equal(f.data.view(torch.int32), r.render().data.view(torch.int32)), (replay, k)
