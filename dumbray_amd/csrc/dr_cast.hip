@@ -12,11 +12,13 @@ namespace dr {
 
 constexpr int kCastBlock = 256;
 constexpr int kWavesPerBlock = kCastBlock / 64;
-constexpr int kWaveChunk = 128;       // rays a wave takes from the global counter at a time
+constexpr int kWaveChunk = 128;       // most rays a wave takes from the global counter at a time
 // idle lanes that trigger a refill (incoherent batch: 12, 16, 20, 24, 28, 32 measured 2.16,
 // 2.11-2.12, 2.09, 2.07-2.08, 2.09, 2.11 ms)
 constexpr int kRefillMin = 24;
 constexpr int kLeafMin = 16;          // pending leaves that trigger the (wave-shared) leaf tests
+// ... and fewer in a wave with few rays left, which would otherwise hold each leaf until its slowest ray
+__device__ __forceinline__ int leaf_min(int rays) { return min(kLeafMin, (5 * rays + 15) >> 4); }
 
 // One bounded step per loop iteration.  A lane that is traversing pops one child:
 // an interior child is expanded and pushed, a leaf child is held as pending.
@@ -25,8 +27,8 @@ constexpr int kLeafMin = 16;          // pending leaves that trigger the (wave-s
 // them are idle (or no lane is busy), so the node expansions, which dominate the
 // work, run with most lanes of the wave active.
 //
-// Rays are handed out dynamically: a wave owns a range of kWaveChunk rays taken
-// from the global counter work[0]; lanes that need a ray take the next ones of the
+// Rays are handed out dynamically: a wave owns a range of `chunk` rays (kWaveChunk for a large
+// batch, see launch_cast) taken from the global counter work[0]; lanes that need a ray take the next ones of the
 // range, and the wave takes a new range when it runs out.  The last wave to exit
 // (counted in work[1]) sets both counters back to zero for the next launch.
 //
@@ -44,7 +46,7 @@ template <bool kStats>
 __global__ __launch_bounds__(kCastBlock, 4) void k_cast(DevTree T, const float *__restrict__ rays, int n, int clip,
                                                       const int *__restrict__ exclude, int *__restrict__ out_id,
                                                       float *__restrict__ out_t, float *__restrict__ out_p,
-                                                      int *__restrict__ stats, unsigned *__restrict__ work) {
+                                                      int *__restrict__ stats, unsigned *__restrict__ work, int chunk) {
   extern __shared__ __align__(16) uint2 stk_base[];
   __shared__ LeafLds leaf_all[kWavesPerBlock];
   __shared__ int ins_all[kStats ? kCastBlock : 1];      // per lane: inside tests of its leaf (measurement)
@@ -139,9 +141,9 @@ __global__ __launch_bounds__(kCastBlock, 4) void k_cast(DevTree T, const float *
       } else {
         const int leader = __ffsll((unsigned long long)wmask) - 1;
         unsigned nb = 0;
-        if (lane == leader) nb = atomicAdd(work, (unsigned)kWaveChunk);
+        if (lane == leader) nb = atomicAdd(work, (unsigned)chunk);
         nb = (unsigned)__builtin_amdgcn_readlane((int)nb, leader);   // wave-uniform: kept in scalar registers
-        const unsigned top = min(nb + (unsigned)kWaveChunk, (unsigned)n);
+        const unsigned top = min(nb + (unsigned)chunk, (unsigned)n);
         const unsigned len = nb < top ? top - nb : 0u;
         slot = idx < rem ? (int)(wcur + idx) : (idx - rem < len ? (int)(nb + idx - rem) : -1);
         wcur = nb + min(need - rem, len);
@@ -153,7 +155,7 @@ __global__ __launch_bounds__(kCastBlock, 4) void k_cast(DevTree T, const float *
           if (k == 0 && len0 > 0) flush(0, base0, len0);
           if (k == 1 && len1 > 0) flush(1, base1, len1);
           __builtin_amdgcn_wave_barrier();
-          for (int j = lane; j < kWaveChunk; j += 64) res_id[k * kWaveChunk + j] = kPendingId;
+          for (int j = lane; j < chunk; j += 64) res_id[k * kWaveChunk + j] = kPendingId;
           if (k == 0) { base0 = nb; len0 = (int)len; }
           else { base1 = nb; len1 = (int)len; }
           cur = k;
@@ -184,7 +186,7 @@ __global__ __launch_bounds__(kCastBlock, 4) void k_cast(DevTree T, const float *
     // ---- castInLeaf for the pending leaves, the whole wave sharing their records
     const bool pend = r >= 0 && w.state == kWalkLeaf;
     const uint64_t pm = __ballot(pend);
-    if (pm && (__popcll(pm) >= kLeafMin || __ballot(r >= 0 && w.state == kWalkTrace) == 0)) {
+    if (pm && (__popcll(pm) >= leaf_min(__popcll(__ballot(r >= 0))) || __ballot(r >= 0 && w.state == kWalkTrace) == 0)) {
       walk_leaf_wave<true>(T, w, pend, clip != 0, leaf, ins, cc);
       if (pend && w.state == kWalkDone) finish();
     }
@@ -212,16 +214,24 @@ static int launch_cast(dr_scene s, const float *rays, int n, unsigned flags, con
   const size_t lds = (size_t)levels * kStackWordsPerLevel * kCastBlock * sizeof(uint32_t);
   int per_cu = 0;
   DR_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_cast<false>, kCastBlock, lds));
+  // Rays a wave takes at a time.  A batch that the chip can hold at once is bound by its longest ray:
+  // it goes one ray a lane over as many waves as give every SIMD one, then over lanes (99,991 bounce
+  // rays 246 us with 128 a wave, 228 us with 32, 191 us with 64; 4,096 rays 101 us with 128, 183 us
+  // with 1 on four waves a SIMD, 81 us with 4 on one; 64 rays 46 -> 24 us).  A larger one takes
+  // whole ranges, with two of them staged.
+  int chunk = 1;
+  while (chunk < 64 && (long long)chunk * s->num_cu * 4 < n) chunk *= 2;
+  if ((long long)n > 2LL * 64 * kWavesPerBlock * s->num_cu * std::max(per_cu, 1)) chunk = kWaveChunk;
   // persistent grid: at most one block per resident slot, fewer for small batches
-  const long long need = ((long long)n + kWavesPerBlock * kWaveChunk - 1) / (kWavesPerBlock * kWaveChunk);
+  const long long need = ((long long)n + kWavesPerBlock * chunk - 1) / (kWavesPerBlock * chunk);
   const int blocks = (int)std::max(1LL, std::min<long long>(need, (long long)s->num_cu * std::max(per_cu, 1)));
   unsigned *work = (unsigned *)s->work.p + 2 * (s->work_slot.fetch_add(1) % kWorkSlots);
   if (stats)
     hipLaunchKernelGGL(k_cast<true>, dim3(blocks), dim3(kCastBlock), lds, (hipStream_t)stream, s->tree, rays, n, clip,
-                       (const int *)exclude, (int *)out_id, out_t, out_point, (int *)stats, work);
+                       (const int *)exclude, (int *)out_id, out_t, out_point, (int *)stats, work, chunk);
   else
     hipLaunchKernelGGL(k_cast<false>, dim3(blocks), dim3(kCastBlock), lds, (hipStream_t)stream, s->tree, rays, n,
-                       clip, (const int *)exclude, (int *)out_id, out_t, out_point, (int *)nullptr, work);
+                       clip, (const int *)exclude, (int *)out_id, out_t, out_point, (int *)nullptr, work, chunk);
   DR_HIP_CHECK(hipGetLastError());
   return DR_OK;
 }
