@@ -220,7 +220,7 @@ int dr_scene_create(dr_octree t, dr_scene *out) {
   s->faces_host.assign((size_t)s->ntris * dr::kFaceWords, 0.0f);   // texture coordinates start at 0
   for (int i = 0; i < s->ntris; i++) {
     const dr::Tri &tr = t->host.tris[i];
-    const dr::V3 n = dr::cross(tr.b - tr.a, tr.c - tr.a);
+    const dr::V3 n = dr::normalized(dr::cross(tr.b - tr.a, tr.c - tr.a));
     s->shade_host[i] = make_float4(n.x, n.y, n.z, 0.0f);
     float *F = &s->faces_host[(size_t)i * dr::kFaceWords];
     const float v[9] = {tr.a.x, tr.a.y, tr.a.z, tr.b.x, tr.b.y, tr.b.z, tr.c.x, tr.c.y, tr.c.z};

@@ -74,7 +74,7 @@ DR_HD bool box_ray(V3 o, V3 d, float reach, BoxRay &r) {
   // coordinates whose products with iv could overflow: every box is kept
   const float s = om + reach;
   if (!(s < 1e27f)) ix = iy = iz = 0.0f;
-  const float e = s < 1e27f ? kBoxSlack * s : 0.0f;
+  const float e = s < 1e27f ? __builtin_fmaf(kBoxSlack, s, 1e-36f) : 0.0f;   // (1e-36: products that underflow)
   r.iv = v3(d.x < 0 ? -ix : ix, d.y < 0 ? -iy : iy, d.z < 0 ? -iz : iz);
   const V3 oi = v3(-o.x * r.iv.x, -o.y * r.iv.y, -o.z * r.iv.z);
   r.cn = v3(oi.x - e * ix, oi.y - e * iy, oi.z - e * iz);
@@ -153,12 +153,25 @@ DR_HD bool ancestors_hit(const float4 *nodes, const Box &root, int node, V3 o, V
 // Whether leaf node `leaf` (-1: the tree is one leaf) accepts the hit at p of the ray (o, d):
 // castInLeaf's box test (Octree.impl.cuh:607-611), and the slab tests on the way to the leaf, its
 // own and its ancestors'.  One 32-B record decides unless the leaf pokes out of an ancestor.
-DR_HD bool leaf_accepts(const float4 *nodes, const Box &root, int leaf, V3 o, V3 d, V3 p) {
+//
+// A hit further than m = 16 u (M + O) inside a nested leaf's box on every axis is accepted at once
+// (11 operations instead of the slab test's 90 with its three divisions): with d.k > 0, p = fl(o + fl(d t))
+// misses o + d t by at most u (2 M + O), so (min - o) / d <= t - (m - u (2 M + O)) / |d|, and the slab
+// test's two roundings and its 1 / d add at most 3 u (M + O) / |d|; so its min side is <= t, and its max
+// side >= t by the same steps, on every axis: it passes, and by the argument of slab_nests so do the
+// ancestors'.  A zero d.k leaves o.k = p.k strictly inside (sides of -inf and +inf).  Directions so
+// short that 1 / d could overflow on an axis that moves take the long way.
+DR_HD bool leaf_accepts(const float4 *nodes, const Box &root, float reach, int leaf, V3 o, V3 d, V3 p) {
   if (leaf < 0) return contains(root, p);
   const float4 a = nodes[kNodeF4 * (size_t)leaf], b = nodes[kNodeF4 * (size_t)leaf + 1];
   Box lb;
   lb.s = v3(a.x, a.y, a.z);
   lb.e = v3(a.w, b.x, b.y);
+  const V3 ad = v3(__builtin_fabsf(d.x), __builtin_fabsf(d.y), __builtin_fabsf(d.z));
+  const float m = __builtin_fmaf(kBoxSlack, reach + max3(__builtin_fabsf(o.x), __builtin_fabsf(o.y), __builtin_fabsf(o.z)), 1e-36f);
+  const float deep = __builtin_fminf(min3(p.x - lb.s.x, p.y - lb.s.y, p.z - lb.s.z), min3(lb.e.x - p.x, lb.e.y - p.y, lb.e.z - p.z));
+  const bool shortest = min3(ad.x > 0 ? ad.x : 1.0f, ad.y > 0 ? ad.y : 1.0f, ad.z > 0 ? ad.z : 1.0f) > 1e-30f;
+  if (deep > m && shortest && bits_of(b.w) != 0) return true;
   if (!contains(lb, p)) return false;
   const V3 inv = v3(1.0f / d.x, 1.0f / d.y, 1.0f / d.z);
   if (!slab_hit(lb.s.x, lb.s.y, lb.s.z, lb.e.x, lb.e.y, lb.e.z, o, inv)) return false;

@@ -166,7 +166,7 @@ __device__ __forceinline__ void reflect_factor(const dr_render_params &P, const 
 
 // Shading tables of one scene.
 struct Tables {
-  const float4 *shade;   // per triangle: (n, material id bits)
+  const float4 *shade;   // per triangle: (unit normal, material id bits)
   const float *faces;    // per triangle: kFaceWords floats (vertices, vertex normals)
 };
 

@@ -201,9 +201,9 @@ DR_HD void camera_ray(const dr_render_params &P, const FrameK &K, int px, int py
   }
 }
 
-// Unit geometric normal n = (b-a)x(c-a) normalised, turned to face the incoming ray.
+// Unit geometric normal n = normalized((b-a)x(c-a)), turned to face the incoming ray.
 DR_HD V3 facing_normal(V3 n, V3 du) {
-  V3 nu = normalized(n);
+  V3 nu = n;
   if (dot(nu, du) > 0) nu = v3(-nu.x, -nu.y, -nu.z);
   return nu;
 }

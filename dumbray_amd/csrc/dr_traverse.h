@@ -121,10 +121,15 @@ __device__ __forceinline__ void group_entry(const float4 *__restrict__ G, int g,
                           (uint32_t)__float_as_int(b2.y), (uint32_t)__float_as_int(b2.z), (uint32_t)__float_as_int(b2.w)};
   uint32_t m = group_children(v3(grid.x, grid.y, grid.z), v3(cell.x, cell.y, cell.z), w, r) & head & 0xffu;
   if (cc) { cc->live += __builtin_popcount(head & 0xffu); cc->slab += __builtin_popcount(m); }
-  const int c = r.canon;
-  if (c & 1) m = ((m & 0x55u) << 1) | ((m >> 1) & 0x55u);
-  if (c & 2) m = ((m & 0x33u) << 2) | ((m >> 2) & 0x33u);
-  if (c & 4) m = ((m & 0x0Fu) << 4) | ((m >> 4) & 0x0Fu);
+  // bit k to bit k ^ canon: per set bit of canon the pairs that far apart trade places (a shift of 0
+  // trades nothing)
+  const uint32_t c1 = r.canon & 1, c2 = r.canon & 2, c4 = r.canon & 4;
+  uint32_t t = (m ^ (m >> c1)) & 0x55u;
+  m ^= t ^ (t << c1);
+  t = (m ^ (m >> c2)) & 0x33u;
+  m ^= t ^ (t << c2);
+  t = (m ^ (m >> c4)) & 0x0fu;
+  m ^= t ^ (t << c4);
   lo = ((uint32_t)g << 8) | m;
   hi = (base << 8) | ((head >> 8) & 0xffu);
 }
@@ -191,27 +196,29 @@ __device__ __forceinline__ void walk_step(const DevTree &T, Walk &w, uint2 *stk,
 // shifts by 1, 2, 4 and 8 scan each row of 16 lanes, then lane 15 of rows 0 and 2 is added to
 // the row after it and lane 31 to the upper half (a lane without a source takes 0).
 template <int kCtrl, int kRows = 0xf>
-__device__ __forceinline__ int dpp_or_zero(int v) {
-  return __builtin_amdgcn_update_dpp(0, v, kCtrl, kRows, 0xf, false);
+__device__ __forceinline__ uint32_t dpp_or_zero(uint32_t v) {   // (the compiler folds it into the sum or maximum)
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, kCtrl, kRows, 0xf, kRows == 0xf);
 }
-__device__ __forceinline__ int wave_incl_scan(int v, int &total) {
+__device__ __forceinline__ int wave_incl_scan(int count, int &total) {
+  uint32_t v = (uint32_t)count;
   v += dpp_or_zero<0x111>(v);        // row_shr:1
   v += dpp_or_zero<0x112>(v);        // row_shr:2
   v += dpp_or_zero<0x114>(v);        // row_shr:4
   v += dpp_or_zero<0x118>(v);        // row_shr:8
   v += dpp_or_zero<0x142, 0xa>(v);   // row_bcast:15 into rows 1 and 3
   v += dpp_or_zero<0x143, 0xc>(v);   // row_bcast:31 into rows 2 and 3
-  total = __builtin_amdgcn_readlane(v, 63);
-  return v;
+  total = __builtin_amdgcn_readlane((int)v, 63);
+  return (int)v;
 }
-__device__ __forceinline__ int wave_incl_max(int v) {   // v >= 0
+__device__ __forceinline__ int wave_incl_max(int x) {   // x >= 0
+  uint32_t v = (uint32_t)x;
   v = max(v, dpp_or_zero<0x111>(v));
   v = max(v, dpp_or_zero<0x112>(v));
   v = max(v, dpp_or_zero<0x114>(v));
   v = max(v, dpp_or_zero<0x118>(v));
   v = max(v, dpp_or_zero<0x142, 0xa>(v));
   v = max(v, dpp_or_zero<0x143, 0xc>(v));
-  return v;
+  return (int)v;
 }
 
 // One wave's LDS for walk_leaf_wave.
@@ -328,7 +335,7 @@ __device__ __forceinline__ void walk_leaf_wave(const DevTree &T, Walk &w, bool p
     // the record's id is read beside the leaf box, before the box test that decides whether
     // it is needed
     const int rid = kIndexed ? __float_as_int(T.urecs[4 * T.lref[k] + 3].w) : __float_as_int(T.recs[4 * k + 3].w);
-    if (leaf_accepts(T.nodes, root_box(T), w.leaf, w.o, w.d, p)) {
+    if (leaf_accepts(T.nodes, root_box(T), T.reach, w.leaf, w.o, w.d, p)) {
       hit = true;
       w.h.id = rid;
       w.h.t = t;

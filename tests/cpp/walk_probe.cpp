@@ -88,7 +88,7 @@ bool compact(const OctreeFlat &f, const std::vector<Tri> &tris, int g, V3 o, V3 
       if (tri_hit(tris[tri], o, d, t, p) && t < best) { best = t; id = tri; bp = p; }
     }
     const float4 *nodes = (const float4 *)f.nodes.data();
-    if (id >= 0 && leaf_accepts(nodes, f.root, 8 * g + k, o, d, bp)) {
+    if (id >= 0 && leaf_accepts(nodes, f.root, f.reach, 8 * g + k, o, d, bp)) {
       if (bits_of(f.nodes[(size_t)(8 * g + k) * kNodeWords + 7]) == 0) n.chains++;
       r.id = id;
       r.t = best;
