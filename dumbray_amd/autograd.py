@@ -24,7 +24,7 @@ class RenderFunction(torch.autograd.Function):
         ctx.renderer = renderer
         ctx.iteration = iteration
         ctx.dtypes = (albedo.dtype, emission.dtype)
-        return frame.data.clone()
+        return frame.data
 
     @staticmethod
     def backward(ctx, grad_frame):

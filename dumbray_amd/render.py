@@ -77,8 +77,18 @@ class BlockBasedFrameBuffer:
         self.width, self.height = int(width), int(height)
         self.data = torch.zeros((block_count(self.width, self.height) * BLOCK_SIZE, 4), dtype=torch.float32,
                                 device=self.device)
-        self._idx = torch.from_numpy(block_to_image_index(self.width, self.height)).to(self.data.device)
+        self._rows = None
         return True
+
+    @property
+    def _idx(self):
+        """Row of `data` for every row-major pixel, made when an image is first converted: a frame
+        that is only rendered into needs none, and its upload makes the host wait for the device."""
+        import torch
+
+        if self._rows is None:
+            self._rows = torch.from_numpy(block_to_image_index(self.width, self.height)).to(self.data.device)
+        return self._rows
 
     def getBlockSize(self) -> int:
         return BLOCK_SIZE
