@@ -124,72 +124,77 @@ __global__ __launch_bounds__(kCastBlock, 4) void k_cast(DevTree T, const float *
     }
   };
 
+  // The results, the staged ranges and the refill are looked at only after a ray has ended (or while
+  // idle lanes wait for a range): most iterations end none.  Looked at in every one they were a sixth
+  // of the loop's cycles, and three copies of finish() took registers (1M rays 502 -> 452 us, 99,991
+  // bounce rays 186 -> 177 us, 4M incoherent rays 1.26 -> 1.24 ms).  Smaller ranges near the end of the
+  // batch, to let the waves end together, cost more than they gave (1M rays 452 -> 499 us).
+  bool look = true;
   for (;;) {
-    retire(0, base0, len0);
-    retire(1, base1, len1);
-    // ---- refill idle lanes
-    const bool want = (r < 0) && !exhausted;
-    const uint64_t wmask = __ballot(want);
-    if (wmask && (__popcll(wmask) >= kRefillMin || __ballot(r >= 0) == 0)) {
+    const bool done = r >= 0 && w.state == kWalkDone;
+    if (look || __ballot(done) != 0) {
+      if (done) finish();
+      retire(0, base0, len0);
+      retire(1, base1, len1);
+      // ---- refill idle lanes
+      const uint64_t wmask = __ballot(r < 0);
       const unsigned need = (unsigned)__popcll(wmask);
-      const unsigned idx = (unsigned)__popcll(wmask & below);
       const unsigned rem = wend - wcur;
-      int slot;
-      if (rem >= need) {
-        slot = (int)(wcur + idx);
-        wcur += need;
-      } else {
-        const int leader = __ffsll((unsigned long long)wmask) - 1;
-        unsigned nb = 0;
-        if (lane == leader) nb = atomicAdd(work, (unsigned)chunk);
-        nb = (unsigned)__builtin_amdgcn_readlane((int)nb, leader);   // wave-uniform: kept in scalar registers
-        const unsigned top = min(nb + (unsigned)chunk, (unsigned)n);
-        const unsigned len = nb < top ? top - nb : 0u;
-        slot = idx < rem ? (int)(wcur + idx) : (idx - rem < len ? (int)(nb + idx - rem) : -1);
-        wcur = nb + min(need - rem, len);
-        wend = nb + len;
-        if (len > 0) {
-          // the new range takes the slot the current range does not hold; an unfinished
-          // range still there is written out as far as it is done
-          const int k = (cur == 0 ? len0 : len1) > 0 ? 1 - cur : cur;
-          if (k == 0 && len0 > 0) flush(0, base0, len0);
-          if (k == 1 && len1 > 0) flush(1, base1, len1);
-          __builtin_amdgcn_wave_barrier();
-          for (int j = lane; j < chunk; j += 64) res_id[k * kWaveChunk + j] = kPendingId;
-          if (k == 0) { base0 = nb; len0 = (int)len; }
-          else { base1 = nb; len1 = (int)len; }
-          cur = k;
+      look = false;
+      if (rem > 0 || !exhausted) {
+        if (need >= kRefillMin || need == 64) {
+          const unsigned idx = (unsigned)__popcll(wmask & below);
+          int slot = idx < rem ? (int)(wcur + idx) : -1;
+          if (rem >= need) {
+            wcur += need;
+          } else if (exhausted) {
+            wcur = wend;
+          } else {
+            unsigned nb = 0;
+            if (lane == 0) nb = atomicAdd(work, (unsigned)chunk);
+            nb = (unsigned)__builtin_amdgcn_readfirstlane((int)nb);   // wave-uniform: kept in scalar registers
+            const unsigned top = min(nb + (unsigned)chunk, (unsigned)n);
+            const unsigned len = nb < top ? top - nb : 0u;
+            exhausted = nb + (unsigned)chunk >= (unsigned)n;
+            if (idx >= rem && idx - rem < len) slot = (int)(nb + idx - rem);
+            wcur = nb + min(need - rem, len);
+            wend = nb + len;
+            if (len > 0) {
+              // the new range takes the slot the current range does not hold; an unfinished
+              // range still there is written out as far as it is done
+              const int k = (cur == 0 ? len0 : len1) > 0 ? 1 - cur : cur;
+              if (k == 0 && len0 > 0) flush(0, base0, len0);
+              if (k == 1 && len1 > 0) flush(1, base1, len1);
+              __builtin_amdgcn_wave_barrier();
+              for (int j = lane; j < (int)len; j += 64) res_id[k * kWaveChunk + j] = kPendingId;
+              if (k == 0) { base0 = nb; len0 = (int)len; }
+              else { base1 = nb; len1 = (int)len; }
+              cur = k;
+            }
+          }
+          if (r < 0 && slot >= 0) {
+            r = slot;
+            const float2 *R = (const float2 *)(rays + 6 * (size_t)r);
+            const float2 q0 = R[0], q1 = R[1], q2 = R[2];
+            walk_begin(T, w, v3(q0.x, q0.y, q1.x), v3(q1.y, q2.x, q2.y), exclude ? exclude[r] : -1, stk);
+          }
+          look = __popcll(__ballot(r < 0)) >= kRefillMin;
         }
       }
-      if (want) {
-        if (slot >= 0) {
-          r = slot;
-          const float2 *R = (const float2 *)(rays + 6 * (size_t)r);
-          const float2 q0 = R[0], q1 = R[1], q2 = R[2];
-          walk_begin(T, w, v3(q0.x, q0.y, q1.x), v3(q1.y, q2.x, q2.y), exclude ? exclude[r] : -1, stk);
-          if (w.state == kWalkDone) finish();
-        } else {
-          exhausted = true;
-        }
+      if (__ballot(r >= 0) == 0) {
+        if (exhausted && wcur == wend) break;
+        look = true;
+        continue;
       }
-    }
-    if (__ballot(r >= 0) == 0) {
-      if (__ballot(!exhausted) == 0) break;
-      continue;
     }
     // ---- one traversal step
-    if (r >= 0 && w.state == kWalkTrace) {
-      walk_step(T, w, stk, S, cc);
-      if (w.state == kWalkDone) finish();
-    }
+    if (r >= 0 && w.state == kWalkTrace) walk_step(T, w, stk, S, cc);
 
     // ---- castInLeaf for the pending leaves, the whole wave sharing their records
     const bool pend = r >= 0 && w.state == kWalkLeaf;
     const uint64_t pm = __ballot(pend);
-    if (pm && (__popcll(pm) >= leaf_min(__popcll(__ballot(r >= 0))) || __ballot(r >= 0 && w.state == kWalkTrace) == 0)) {
+    if (pm && (__popcll(pm) >= leaf_min(__popcll(__ballot(r >= 0))) || __ballot(r >= 0 && w.state == kWalkTrace) == 0))
       walk_leaf_wave<true>(T, w, pend, clip != 0, leaf, ins, cc);
-      if (pend && w.state == kWalkDone) finish();
-    }
   }
   // every ray of the wave has ended: the ranges still staged go out
   if (len0 > 0) flush(0, base0, len0);
@@ -214,6 +219,9 @@ static int launch_cast(dr_scene s, const float *rays, int n, unsigned flags, con
   const size_t lds = (size_t)levels * kStackWordsPerLevel * kCastBlock * sizeof(uint32_t);
   int per_cu = 0;
   DR_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_cast<false>, kCastBlock, lds));
+  // (the registers would allow five, which share the caches worse: 4M incoherent rays 1.29 against
+  // 1.24 ms, 400,000 bounce rays 935 against 893 us)
+  per_cu = std::min(per_cu, 4);
   // Rays a wave takes at a time.  A batch that the chip can hold at once is bound by its longest ray:
   // it goes one ray a lane over as many waves as give every SIMD one, then over lanes (99,991 bounce
   // rays 246 us with 128 a wave, 228 us with 32, 191 us with 64; 4,096 rays 101 us with 128, 183 us
