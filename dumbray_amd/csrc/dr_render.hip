@@ -54,27 +54,6 @@ __device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlan
 __device__ __forceinline__ uint32_t uni(uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); }
 __device__ __forceinline__ UDiv uni(UDiv D) { return {uni(D.d), uni(D.m)}; }
 __device__ __forceinline__ UDiv udiv_uniform(uint32_t d) { return uni(make_udiv(d)); }
-// frame_k(P) formed in the kernel and moved to scalar registers (the kernels otherwise take
-// the host's frame_k as an argument).
-__device__ __forceinline__ FrameK frame_k_uniform(const dr_render_params &P) {
-  FrameK K = frame_k(P);
-  K.nbw = uni(K.nbw);
-  K.fy = uni(K.fy);
-  K.hw = uni(K.hw);
-  K.hh = uni(K.hh);
-  K.ps = uni(K.ps);
-  K.pdx = uni(K.pdx);
-  K.pdy = uni(K.pdy);
-  K.jx = uni(K.jx);
-  K.ox = uni(K.ox);
-  K.jy = uni(K.jy);
-  K.oy = uni(K.oy);
-  for (int k = 0; k < 4; k++) K.zc[k] = uni(K.zc[k]);
-  K.amount = uni(K.amount);
-  K.keep = uni(K.keep);
-  K.inv_rr = uni(K.inv_rr);
-  return K;
-}
 
 // The first ray of a path: sample `samp` of pixel `pix`, kNoPixel for a pixel outside the image.
 constexpr uint32_t kNoPixel = 0xffffffffu;
@@ -170,6 +149,24 @@ struct Tables {
   const float *faces;    // per triangle: kFaceWords floats (vertices, vertex normals)
 };
 
+// What a stream reads throughout, where it lies in constant memory: the first argument of
+// k_render_stream, part of a batch's request.
+struct RenderArgs {
+  DevTree T;
+  Tables tb;
+  dr_render_params P;
+  FrameK K;
+};
+typedef const __attribute__((address_space(4))) RenderArgs *ConstArgs;
+// The arguments, to be read anew by what follows.  Kernel arguments are loaded once and kept in scalar
+// registers; these are more than there are, and what does not fit went to lanes of vector registers:
+// 559 of the 2,791 vector instructions of k_render_stream<BenchPath> moved scalars back, 15 do now
+// (1080p 16 spp 15.60 -> 15.14 ms, reference plugins 1080p 3.11 -> 2.96 ms).
+__device__ __forceinline__ const RenderArgs &again(ConstArgs A) {
+  asm volatile("" : "+s"(A));
+  return *(const RenderArgs *)A;
+}
+
 // Path updates of the benchmark plugins (DR_PLUGINS_BENCHMARK).
 struct BenchPath {
   // render_block: finished casts that trigger the path updates, idle lanes that trigger new path
@@ -177,7 +174,6 @@ struct BenchPath {
   // updates (in proportion with fewer lanes; 1080p 16 spp 16.4 / 15.9 / 15.8 ms at 16 / 24 / 32),
   // idle lanes that pop the queue (1, 4, 10: 16.2, 15.9, 15.9 ms)
   static constexpr int kShadeMin = 32, kRefillMin = 8, kStreamShadeMin = 32, kStreamRefillMin = 4;
-  static constexpr bool kStreamFrameInKernel = false;
   Path st;
   __device__ __forceinline__ bool start(const dr_render_params &P, const FrameK &K, int block, int lp, int s,
                                         uint32_t samp0) {
@@ -238,7 +234,6 @@ struct BenchPath {
 struct RefPath {
   // the same thresholds (reference plugins at 1080p, 1 spp: 3.23 / 3.12 / 3.26 ms at 32 / 44 / 52)
   static constexpr int kShadeMin = 32, kRefillMin = 8, kStreamShadeMin = 44, kStreamRefillMin = 4;
-  static constexpr bool kStreamFrameInKernel = true;
   uint32_t pix, samp;
   int layer, phase, light, lk, excl, trans;   // lk: photons of the current light still to send
   V3 o, d;                          // the next ray to cast
@@ -541,7 +536,7 @@ __device__ __forceinline__ void render_block(const DevTree &T, const Tables &tb,
       if (job >= 0 && w.state == kWalkTrace) walk_step(T, w, lds.stk, kRB, cc);
       // ---- leaf tests, batched
       const bool pend = job >= 0 && w.state == kWalkLeaf;
-      const uint64_t pm = __ballot(pend);
+      const uint64_t pm = __ballot(pend && w.state == kWalkLeaf);
       if (pm && (__popcll(pm) >= kLeafMin || __ballot(job >= 0 && w.state == kWalkTrace) == 0))
         walk_leaf_wave(T, w, pend, clip, *lds.leaf, kStats ? lds.ins : nullptr, cc);
       // ---- path updates of the finished casts, batched
@@ -654,10 +649,12 @@ struct StreamShape {
 // One stream (every lane of the workgroup calls it): tiles from the counter `next_tile` until they run out.
 // ins: this wave's inside-test counts (measurement launches only).
 template <class PathT, bool kStats>
-__device__ __forceinline__ void stream_paths(const DevTree &T, const Tables &tb, const dr_render_params &P, FrameK K,
+__device__ __forceinline__ void stream_paths(ConstArgs args,
                                              float *__restrict__ frame, int start_block, const StreamShape &S, int levels,
                                              unsigned *next_tile, int refill_min, uint32_t *lds, StreamLds &sh, int *ins,
                                              RenderCounters &rc) {
+  const DevTree T = again(args).T;
+  const dr_render_params &P = again(args).P;
   const int ntiles = S.ntiles, tile_shift = S.tile_shift, chunk = S.chunk, slot_shift = S.slot_shift;
   const int spp = P.fsaa_x * P.fsaa_y;
   const int nslots = slot_shift < 0 ? 0 : 1 << slot_shift;
@@ -676,7 +673,6 @@ __device__ __forceinline__ void stream_paths(const DevTree &T, const Tables &tb,
   CastCounters *cc = kStats ? &rc.cast : nullptr;
   const uint32_t samp0 = (uint32_t)(P.iteration > 1 ? P.iteration - 1 : 0) * (uint32_t)spp;
   const float spw = uni(1.0f / (((float)P.fsaa_x) * ((float)P.fsaa_y)));
-  if constexpr (PathT::kStreamFrameInKernel) K = frame_k_uniform(P);
   const UDiv Dspp = udiv_uniform((uint32_t)spp);
   const bool clip = P.cull_backfaces != 0;
   const int lane = (int)__lane_id();
@@ -696,7 +692,7 @@ __device__ __forceinline__ void stream_paths(const DevTree &T, const Tables &tb,
   auto tile_pixel = [&](int e, int p) {
     return ((((e >> 8) - 1) & ((1 << (7 - tile_shift)) - 1)) << tile_shift) + (p & ((1 << tile_shift) - 1));
   };
-  auto pixel_written = [&](const float a[3]) {
+  auto pixel_written = [&](const FrameK &K, const float a[3]) {
     const int kk = (u >> tile_shift) & (kStreamRing - 1);
     // (the tile's ring entry stays until every pixel of the tile is written)
     const int e = lds_get(&sh.tiles[kk]);
@@ -711,19 +707,20 @@ __device__ __forceinline__ void stream_paths(const DevTree &T, const Tables &tb,
     bool fresh = false;   // the lane has a new ray
     const uint64_t lm = __ballot(live);
     if (dm && __popcll(dm) * 64 >= __popcll(lm) * PathT::kStreamShadeMin) {
+      const RenderArgs &A = again(args);
       if (live && w.state == kWalkDone) {
         const bool outside = ps.pixel() == kNoPixel;
-        if (outside || ps.shade(P, K, tb, w)) {
+        if (outside || ps.shade(A.P, A.K, A.tb, w)) {
           // stages the sample's colour (the lens filter applied: getPixelColor, see render_block; a job
           // outside the image stages black); the lane that completes the pixel writes it out
           const float *col = ps.color();
           float c[3] = {col[0], col[1], col[2]};
           if (origins)
-            for (int k = 0; k < 3; k++) c[k] = c[k] * P.lens_p[4 + k];
+            for (int k = 0; k < 3; k++) c[k] = c[k] * A.P.lens_p[4 + k];
           if (outside) c[0] = c[1] = c[2] = 0.0f;
           if (nslots == 0) {
             const float a[3] = {0.0f + c[0] * spw, 0.0f + c[1] * spw, 0.0f + c[2] * spw};
-            pixel_written(a);
+            pixel_written(A.K, a);
           } else {
             const int slot = u & (nslots - 1);
             float *src = samp + 3 * (size_t)slot * spp;
@@ -737,7 +734,7 @@ __device__ __forceinline__ void stream_paths(const DevTree &T, const Tables &tb,
               float a[3] = {0.0f, 0.0f, 0.0f};
               for (int k = 0; k < spp; k++)
                 for (int j = 0; j < 3; j++) a[j] += src[3 * k + j] * spw;
-              pixel_written(a);
+              pixel_written(A.K, a);
               __threadfence_block();
               lds_put(&turn[slot], (((left >> 9) + 1) << 9) | spp);
             }
@@ -789,7 +786,8 @@ __device__ __forceinline__ void stream_paths(const DevTree &T, const Tables &tb,
         if (lane < chunk) {
           const int q = (int)qbase + lane;
           const int uq = (int)udiv((uint32_t)q, Dspp), s = q - uq * spp;
-          const PathStart st = path_start(P, K, tile_block(e), tile_pixel(e, uq), s, samp0);
+          const RenderArgs &A = again(args);
+          const PathStart st = path_start(A.P, A.K, tile_block(e), tile_pixel(e, uq), s, samp0);
           queue[0 * 64 + lane] = st.d.x;
           queue[1 * 64 + lane] = st.d.y;
           queue[2 * 64 + lane] = st.d.z;
@@ -824,7 +822,8 @@ __device__ __forceinline__ void stream_paths(const DevTree &T, const Tables &tb,
         st.d = v3(queue[0 * 64 + entry], queue[1 * 64 + entry], queue[2 * 64 + entry]);
         st.pix = (uint32_t)__float_as_int(queue[3 * 64 + entry]);
         st.samp = samp0 + (qbase + (uint32_t)entry - (uint32_t)uq * (uint32_t)spp);
-        st.o = v3(P.cam[0], P.cam[1], P.cam[2]);
+        const RenderArgs &A = again(args);
+        st.o = v3(A.P.cam[0], A.P.cam[1], A.P.cam[2]);
         if (origins) st.o = v3(queue[5 * 64 + entry], queue[6 * 64 + entry], queue[7 * 64 + entry]);
         u = uq;
         live = true;
@@ -839,22 +838,22 @@ __device__ __forceinline__ void stream_paths(const DevTree &T, const Tables &tb,
       continue;
     }
     if (fresh) {
-      walk_begin(T, w, ps.ray_o(), ps.ray_d(), ps.ray_excl(), stk);
+      walk_begin(again(args).T, w, ps.ray_o(), ps.ray_d(), ps.ray_excl(), stk);
       if (ps.pixel() == kNoPixel) w.state = kWalkDone;
     }
     // ---- one traversal step of every ray in flight
     if (live && w.state == kWalkTrace) walk_step(T, w, stk, kRB, cc);
     // ---- leaf tests, batched
     const bool pend = live && w.state == kWalkLeaf;
-    const uint64_t pm = __ballot(pend);
+    const uint64_t pm = __ballot(pend && w.state == kWalkLeaf);
     if (pm && (__popcll(pm) * (64 / kLeafMin) >= __popcll(__ballot(live)) || __ballot(live && w.state == kWalkTrace) == 0))
       walk_leaf_wave(T, w, pend, clip, leaf, ins, cc);
   }
 }
 
 template <class PathT, bool kStats>
-__global__ __launch_bounds__(kRB, kRenderWaves) void k_render_stream(DevTree T, Tables tb, dr_render_params P,
-                                                                      FrameK K, float *__restrict__ frame, int start_block,
+__global__ __launch_bounds__(kRB, kRenderWaves) void k_render_stream(RenderArgs by_value,
+                                                                      float *__restrict__ frame, int start_block,
                                                                       StreamShape S, int levels,
                                                                       unsigned *__restrict__ work,
                                                                       unsigned long long *__restrict__ counts) {
@@ -862,7 +861,8 @@ __global__ __launch_bounds__(kRB, kRenderWaves) void k_render_stream(DevTree T, 
   __shared__ StreamLds sh;
   __shared__ int ins_all[kStats ? kRB : 1];
   RenderCounters rc;
-  stream_paths<PathT, kStats>(T, tb, P, K, frame, start_block, S, levels, work, PathT::kStreamRefillMin, lds, sh,
+  // (by_value is the kernel's first argument)
+  stream_paths<PathT, kStats>((ConstArgs)__builtin_amdgcn_kernarg_segment_ptr(), frame, start_block, S, levels, work, PathT::kStreamRefillMin, lds, sh,
                               kStats ? ins_all + (threadIdx.x & ~63u) : nullptr, rc);
   if (kStats) flush_counters(rc, counts);
   // ---- the last wave out resets the block counter for the next launch
@@ -1178,7 +1178,7 @@ __global__ __launch_bounds__(kRB, kRenderWaves) void k_backward(DevTree T, const
     if (fresh) walk_begin(T, w, st.o, st.d, st.restrict_tri, stk);
     if (live && w.state == kWalkTrace) walk_step(T, w, stk, kRB, nullptr);
     const bool pend = live && w.state == kWalkLeaf;
-    const uint64_t pm = __ballot(pend);
+    const uint64_t pm = __ballot(pend && w.state == kWalkLeaf);
     if (pm && (__popcll(pm) * (64 / kLeafMin) >= __popcll(__ballot(live)) || __ballot(live && w.state == kWalkTrace) == 0))
       walk_leaf_wave(T, w, pend, clip, leaf, nullptr, nullptr);
   }
@@ -1188,11 +1188,7 @@ __global__ __launch_bounds__(kRB, kRenderWaves) void k_backward(DevTree T, const
 
 // ------------------------------------------------------------------ batched requests
 struct DevRequest {
-  DevTree T;
-  const float4 *shade;
-  const float *faces;            // shading records of the reference plugins
-  dr_render_params P;
-  FrameK K;                      // frame_k(P), formed on the host
+  RenderArgs A;
   float *frame;
 };
 
@@ -1228,10 +1224,9 @@ __global__ __launch_bounds__(kRB, kRenderWaves) void k_batch_stream(const DevReq
     // the requests are read-only while the kernel runs: the constant address space keeps their loads scalar
     typedef const __attribute__((address_space(4))) DevRequest *ConstRequest;
     const StreamRequest E = list[i];
-    const DevRequest &R = *(const DevRequest *)(ConstRequest)(uintptr_t)&reqs[uni(E.req)];
-    const Tables tb = {R.shade, R.faces};
+    const ConstRequest R = (ConstRequest)(uintptr_t)&reqs[uni(E.req)];
     const StreamShape S = {uni(E.S.ntiles), uni(E.S.tile_shift), uni(E.S.chunk), uni(E.S.slot_shift)};
-    stream_paths<PathT, false>(R.T, tb, R.P, R.K, R.frame, 0, S, levels, next_tile + i, refill_min, lds, sh, nullptr, rc);
+    stream_paths<PathT, false>(&R->A, R->frame, 0, S, levels, next_tile + i, refill_min, lds, sh, nullptr, rc);
     // the request with the most work left
     if (threadIdx.x < 64) {
       int best = 0, at = -1;
@@ -1273,8 +1268,7 @@ __global__ __launch_bounds__(kRB, kRenderWaves) void k_batch(const DevRequest *_
     if (it >= nitems) break;
     const int4 w = items[it];
     const DevRequest &R = reqs[w.x];
-    const Tables tb = {R.shade, R.faces};
-    for (int b = w.y; b < w.y + w.z; b++) render_block<PathT>(R.T, tb, R.P, R.K, R.frame, b, L, refill_min);
+    for (int b = w.y; b < w.y + w.z; b++) render_block<PathT>(R.A.T, R.A.tb, R.A.P, R.A.K, R.frame, b, L, refill_min);
   }
 }
 
@@ -1384,8 +1378,8 @@ static int launch_render(dr_scene s, const dr_render_params *p, float *frame, in
     const StreamShape S = stream_shape(nrange, spp, slot_shift, (double)resident);
     const long long groups = std::min<long long>(S.ntiles, resident);
     unsigned *work = (unsigned *)s->work.p + 2 * (s->work_slot.fetch_add(1) % kWorkSlots);
-    hipLaunchKernelGGL(kern, dim3((unsigned)groups), dim3(kRB), lds_s, (hipStream_t)stream, s->tree, tb, *p, frame_k(*p),
-                       frame, start_block, S, levels, work, counts);
+    hipLaunchKernelGGL(kern, dim3((unsigned)groups), dim3(kRB), lds_s, (hipStream_t)stream,
+                       RenderArgs{s->tree, tb, *p, frame_k(*p)}, frame, start_block, S, levels, work, counts);
     DR_HIP_CHECK(hipGetLastError());
     return DR_OK;
   }
@@ -1581,7 +1575,7 @@ static double pixel_cost(const dr_render_params &P) {
 static std::vector<int4> make_items(const std::vector<DevRequest> &R, int tile, int set) {
   std::vector<std::pair<double, int4>> v;
   for (int r = 0; r < (int)R.size(); r++) {
-    const dr_render_params &P = R[r].P;
+    const dr_render_params &P = R[r].A.P;
     if ((P.plugins == DR_PLUGINS_REFERENCE) != (set == 1) || request_streams(P)) continue;
     const int nb = block_count(&P);
     for (int b = 0; b < nb; b += tile)
@@ -1603,7 +1597,7 @@ static int make_streams(dr_batch b, int set) {
   std::vector<int> ids;
   double total = 0.0;
   for (int r = 0; r < (int)b->host_reqs.size(); r++) {
-    const dr_render_params &P = b->host_reqs[r].P;
+    const dr_render_params &P = b->host_reqs[r].A.P;
     if ((P.plugins == DR_PLUGINS_REFERENCE) != (set == 1) || !request_streams(P)) continue;
     ids.push_back(r);
     total += pixel_cost(P) * block_count(&P);
@@ -1615,7 +1609,7 @@ static int make_streams(dr_batch b, int set) {
   std::vector<int> first(grid);
   double before = 0.0;
   for (int i = 0, g = 0; i < st.n; i++) {
-    const dr_render_params &P = b->host_reqs[ids[i]].P;
+    const dr_render_params &P = b->host_reqs[ids[i]].A.P;
     const int spp = P.fsaa_x * P.fsaa_y;
     const bool origins = P.lens == DR_SPHERICAL_SEGMENT_LENS;
     int slot_shift, per_cu;
@@ -1673,12 +1667,7 @@ extern "C" int dr_batch_create(const dr_request *reqs, int n, const dr_batch_tun
     if (rc == DR_OK && !reqs[r].frame) rc = dr::fail(DR_ERR_ARG, "dr_batch_create: null frame");
     if (rc != DR_OK) break;
     dr::DevRequest d;
-    const dr::Tables tb = dr::tables_of(reqs[r].scene, &reqs[r].params);
-    d.T = reqs[r].scene->tree;
-    d.shade = tb.shade;
-    d.faces = tb.faces;
-    d.P = reqs[r].params;
-    d.K = dr::frame_k(d.P);
+    d.A = {reqs[r].scene->tree, dr::tables_of(reqs[r].scene, &reqs[r].params), reqs[r].params, dr::frame_k(reqs[r].params)};
     dr::scene_retain(reqs[r].scene);
     b->scenes.push_back(reqs[r].scene);
     if (reqs[r].params.shading) {
