@@ -70,7 +70,7 @@ __global__ __launch_bounds__(kCastBlock, 4) void k_cast(DevTree T, const float *
   int r = -1;
   bool exhausted = false;
   Walk w;
-  w.state = kWalkDone;
+  w.state = kWalkIdle;          // the lane has no ray
   CastCounters cnt_local = {0, 0, 0, 0, 0, 0};
   CastCounters *cc = kStats ? &cnt_local : nullptr;
   auto finish = [&]() {
@@ -103,6 +103,7 @@ __global__ __launch_bounds__(kCastBlock, 4) void k_cast(DevTree T, const float *
       cnt_local = {0, 0, 0, 0, 0, 0};
     }
     r = -1;
+    w.state = kWalkIdle;
   };
   // writes the finished entries of slot k (range base, len) as whole lines (wave-uniform)
   auto flush = [&](int k, unsigned base, int len) {
@@ -131,13 +132,13 @@ __global__ __launch_bounds__(kCastBlock, 4) void k_cast(DevTree T, const float *
   // batch, to let the waves end together, cost more than they gave (1M rays 452 -> 499 us).
   bool look = true;
   for (;;) {
-    const bool done = r >= 0 && w.state == kWalkDone;
+    const bool done = w.state == kWalkDone;
     if (look || __ballot(done) != 0) {
       if (done) finish();
       retire(0, base0, len0);
       retire(1, base1, len1);
       // ---- refill idle lanes
-      const uint64_t wmask = __ballot(r < 0);
+      const uint64_t wmask = __ballot(w.state == kWalkIdle);
       const unsigned need = (unsigned)__popcll(wmask);
       const unsigned rem = wend - wcur;
       look = false;
@@ -172,29 +173,28 @@ __global__ __launch_bounds__(kCastBlock, 4) void k_cast(DevTree T, const float *
               cur = k;
             }
           }
-          if (r < 0 && slot >= 0) {
+          if (w.state == kWalkIdle && slot >= 0) {
             r = slot;
             const float2 *R = (const float2 *)(rays + 6 * (size_t)r);
             const float2 q0 = R[0], q1 = R[1], q2 = R[2];
             walk_begin(T, w, v3(q0.x, q0.y, q1.x), v3(q1.y, q2.x, q2.y), exclude ? exclude[r] : -1, stk);
           }
-          look = __popcll(__ballot(r < 0)) >= kRefillMin;
+          look = __popcll(__ballot(w.state == kWalkIdle)) >= kRefillMin;
         }
       }
-      if (__ballot(r >= 0) == 0) {
+      if (__ballot(w.state != kWalkIdle) == 0) {
         if (exhausted && wcur == wend) break;
         look = true;
         continue;
       }
     }
     // ---- one traversal step
-    if (r >= 0 && w.state == kWalkTrace) walk_step(T, w, stk, S, cc);
+    if (w.state == kWalkTrace) walk_step(T, w, stk, S, cc);
 
     // ---- castInLeaf for the pending leaves, the whole wave sharing their records
-    const bool pend = r >= 0 && w.state == kWalkLeaf;
-    const uint64_t pm = __ballot(pend);
-    if (pm && (__popcll(pm) >= leaf_min(__popcll(__ballot(r >= 0))) || __ballot(r >= 0 && w.state == kWalkTrace) == 0))
-      walk_leaf_wave<true>(T, w, pend, clip != 0, leaf, ins, cc);
+    const uint64_t pm = __ballot(w.state == kWalkLeaf);
+    if (pm && (__popcll(pm) >= leaf_min(__popcll(__ballot(w.state != kWalkIdle))) || __ballot(w.state == kWalkTrace) == 0))
+      walk_leaf_wave<true>(T, w, w.state == kWalkLeaf, clip != 0, leaf, ins, cc);
   }
   // every ray of the wave has ended: the ranges still staged go out
   if (len0 > 0) flush(0, base0, len0);

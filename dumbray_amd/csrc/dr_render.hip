@@ -536,7 +536,7 @@ __device__ __forceinline__ void render_block(const DevTree &T, const Tables &tb,
       if (job >= 0 && w.state == kWalkTrace) walk_step(T, w, lds.stk, kRB, cc);
       // ---- leaf tests, batched
       const bool pend = job >= 0 && w.state == kWalkLeaf;
-      const uint64_t pm = __ballot(pend && w.state == kWalkLeaf);
+      const uint64_t pm = __ballot(pend);
       if (pm && (__popcll(pm) >= kLeafMin || __ballot(job >= 0 && w.state == kWalkTrace) == 0))
         walk_leaf_wave(T, w, pend, clip, *lds.leaf, kStats ? lds.ins : nullptr, cc);
       // ---- path updates of the finished casts, batched
@@ -678,10 +678,9 @@ __device__ __forceinline__ void stream_paths(ConstArgs args,
   const int lane = (int)__lane_id();
   const uint64_t below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
   PathT ps;
-  Walk w;
-  w.state = kWalkDone;
+  Walk w;                 // (kWalkIdle: the lane has no path)
+  w.state = kWalkIdle;
   int u = 0;              // stream pixel of this lane's path
-  bool live = false;      // the lane has a path
   // the wave's queue (wave-uniform): entries [qpos, qlen) of the jobs from qbase on
   unsigned qbase = 0;
   int qpos = 0, qlen = 0;
@@ -703,12 +702,12 @@ __device__ __forceinline__ void stream_paths(ConstArgs args,
     // ---- path updates of the finished casts, batched.  The thresholds here and of the leaf tests are
     // shares of the lanes that have a path: a wave near the end of the frame, with few, would otherwise
     // hold each finished cast until its slowest ray (517x389 at 1 spp: 1067 -> 968 us)
-    const uint64_t dm = __ballot(live && w.state == kWalkDone);
+    const uint64_t dm = __ballot(w.state == kWalkDone);
     bool fresh = false;   // the lane has a new ray
-    const uint64_t lm = __ballot(live);
+    const uint64_t lm = __ballot(w.state != kWalkIdle);
     if (dm && __popcll(dm) * 64 >= __popcll(lm) * PathT::kStreamShadeMin) {
       const RenderArgs &A = again(args);
-      if (live && w.state == kWalkDone) {
+      if (w.state == kWalkDone) {
         const bool outside = ps.pixel() == kNoPixel;
         if (outside || ps.shade(A.P, A.K, A.tb, w)) {
           // stages the sample's colour (the lens filter applied: getPixelColor, see render_block; a job
@@ -739,7 +738,7 @@ __device__ __forceinline__ void stream_paths(ConstArgs args,
               lds_put(&turn[slot], (((left >> 9) + 1) << 9) | spp);
             }
           }
-          live = false;
+          w.state = kWalkIdle;
         } else {
           fresh = true;
           if (kStats) { rc.segments++; rc.photons += ps.photon() ? 1 : 0; }
@@ -803,10 +802,10 @@ __device__ __forceinline__ void stream_paths(ConstArgs args,
       }
     }
     // ---- idle lanes pop the next entries whose pixel slot is free
-    const uint64_t idle = __ballot(!live);
+    const uint64_t idle = __ballot(w.state == kWalkIdle);
     if (qpos < qlen && idle && (__popcll(idle) >= refill_min || idle == ~0ull)) {
       const int entry = qpos + __popcll(idle & below);
-      const bool some = !live && entry < qlen;
+      const bool some = w.state == kWalkIdle && entry < qlen;
       int uq = 0;
       bool free = false;
       if (some) {
@@ -826,13 +825,13 @@ __device__ __forceinline__ void stream_paths(ConstArgs args,
         st.o = v3(A.P.cam[0], A.P.cam[1], A.P.cam[2]);
         if (origins) st.o = v3(queue[5 * 64 + entry], queue[6 * 64 + entry], queue[7 * 64 + entry]);
         u = uq;
-        live = true;
+        w.state = kWalkTrace;
         ps.begin(st);
         fresh = true;
         if (kStats && st.pix != kNoPixel) { rc.paths++; rc.segments++; }
       }
     }
-    if (__ballot(live) == 0) {
+    if (__ballot(w.state != kWalkIdle) == 0) {
       if (qpos == qlen && ended) break;
       __builtin_amdgcn_s_sleep(1);   // the next jobs wait for a slot or a tile id
       continue;
@@ -842,12 +841,12 @@ __device__ __forceinline__ void stream_paths(ConstArgs args,
       if (ps.pixel() == kNoPixel) w.state = kWalkDone;
     }
     // ---- one traversal step of every ray in flight
-    if (live && w.state == kWalkTrace) walk_step(T, w, stk, kRB, cc);
+    if (w.state == kWalkTrace) walk_step(T, w, stk, kRB, cc);
     // ---- leaf tests, batched
-    const bool pend = live && w.state == kWalkLeaf;
-    const uint64_t pm = __ballot(pend && w.state == kWalkLeaf);
-    if (pm && (__popcll(pm) * (64 / kLeafMin) >= __popcll(__ballot(live)) || __ballot(live && w.state == kWalkTrace) == 0))
-      walk_leaf_wave(T, w, pend, clip, leaf, ins, cc);
+    const uint64_t pm = __ballot(w.state == kWalkLeaf);
+    if (pm && (__popcll(pm) * (64 / kLeafMin) >= __popcll(__ballot(w.state != kWalkIdle)) ||
+               __ballot(w.state == kWalkTrace) == 0))
+      walk_leaf_wave(T, w, w.state == kWalkLeaf, clip, leaf, ins, cc);
   }
 }
 
@@ -1014,9 +1013,8 @@ __global__ __launch_bounds__(kRB, kRenderWaves) void k_backward(DevTree T, const
 
   Path st;
   Walk w;
-  w.state = kWalkDone;
+  w.state = kWalkIdle;            // the lane has no path
   int K = 0;                      // vertices recorded for the current path
-  bool live = false;              // the lane has a path
   bool fin = false;               // the current path has ended; its albedo terms are pending
   float wdl[3] = {0, 0, 0};       // spw * dL/dI (* lens filter) of the current pixel
   // the wave's queue (wave-uniform): entries [qpos, qlen); the unit's next chunks [cnext, cend) of block `block`
@@ -1043,12 +1041,12 @@ __global__ __launch_bounds__(kRB, kRenderWaves) void k_backward(DevTree T, const
     // ---- path updates of the finished casts, batched (the threshold in proportion to the busy
     // lanes, as in k_render_stream)
     bool fresh = false;           // the lane has a new ray
-    const uint64_t dm = __ballot(live && w.state == kWalkDone);
-    if (dm && __popcll(dm) * 64 >= __popcll(__ballot(live)) * kShadeMin) {
+    const uint64_t dm = __ballot(w.state == kWalkDone);
+    if (dm && __popcll(dm) * 64 >= __popcll(__ballot(w.state != kWalkIdle)) * kShadeMin) {
       bool lit = false;
       float ev[3] = {0.0f, 0.0f, 0.0f};
       int lkey = 0;
-      if (live && w.state == kWalkDone) {
+      if (w.state == kWalkDone) {
         bool photons = false;
         if (st.phase == 0) {
           if (!w.hit) fin = true;
@@ -1108,7 +1106,7 @@ __global__ __launch_bounds__(kRB, kRenderWaves) void k_backward(DevTree T, const
           }
           wave_add3(add, has, m, av);
         }
-        if (fin) { live = false; fin = false; }
+        if (fin) { w.state = kWalkIdle; fin = false; }
       }
     }
     // ---- the queue is empty: the next chunk of the unit, or the next unit
@@ -1153,10 +1151,10 @@ __global__ __launch_bounds__(kRB, kRenderWaves) void k_backward(DevTree T, const
       }
     }
     // ---- idle lanes pop the next entries
-    const uint64_t idle = __ballot(!live);
+    const uint64_t idle = __ballot(w.state == kWalkIdle);
     if (qpos < qlen && idle && (__popcll(idle) >= kAdjointRefillMin || idle == ~0ull)) {
       const int entry = qpos + __popcll(idle & below);
-      const bool take = !live && entry < qlen;
+      const bool take = w.state == kWalkIdle && entry < qlen;
       qpos += __popcll(__ballot(take));
       if (take) {
         PathStart ps;
@@ -1166,21 +1164,22 @@ __global__ __launch_bounds__(kRB, kRenderWaves) void k_backward(DevTree T, const
         for (int c = 0; c < 3; c++) wdl[c] = queue[(5 + c) * 64 + entry];
         ps.o = v3(P.cam[0], P.cam[1], P.cam[2]);
         if (origins) ps.o = v3(queue[8 * 64 + entry], queue[9 * 64 + entry], queue[10 * 64 + entry]);
-        live = fresh = ps.pix != kNoPixel;     // (a pixel outside the image has no paths)
+        fresh = ps.pix != kNoPixel;            // (a pixel outside the image has no paths)
+        if (fresh) w.state = kWalkTrace;
         begin_path(st, ps);
         K = 0;
       }
     }
-    if (__ballot(live) == 0) {
+    if (__ballot(w.state != kWalkIdle) == 0) {
       if (qpos == qlen && ended) break;
       continue;
     }
     if (fresh) walk_begin(T, w, st.o, st.d, st.restrict_tri, stk);
-    if (live && w.state == kWalkTrace) walk_step(T, w, stk, kRB, nullptr);
-    const bool pend = live && w.state == kWalkLeaf;
-    const uint64_t pm = __ballot(pend && w.state == kWalkLeaf);
-    if (pm && (__popcll(pm) * (64 / kLeafMin) >= __popcll(__ballot(live)) || __ballot(live && w.state == kWalkTrace) == 0))
-      walk_leaf_wave(T, w, pend, clip, leaf, nullptr, nullptr);
+    if (w.state == kWalkTrace) walk_step(T, w, stk, kRB, nullptr);
+    const uint64_t pm = __ballot(w.state == kWalkLeaf);
+    if (pm && (__popcll(pm) * (64 / kLeafMin) >= __popcll(__ballot(w.state != kWalkIdle)) ||
+               __ballot(w.state == kWalkTrace) == 0))
+      walk_leaf_wave(T, w, w.state == kWalkLeaf, clip, leaf, nullptr, nullptr);
   }
   __syncthreads();
   if (kSums != kSumsGlobal) flush(threadIdx.x, kRB);
