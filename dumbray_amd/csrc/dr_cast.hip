@@ -16,7 +16,9 @@ constexpr int kWaveChunk = 128;       // most rays a wave takes from the global 
 // idle lanes that trigger a refill (incoherent batch: 12, 16, 20, 24, 28, 32 measured 2.16,
 // 2.11-2.12, 2.09, 2.07-2.08, 2.09, 2.11 ms)
 constexpr int kRefillMin = 24;
-constexpr int kLeafMin = 16;          // pending leaves that trigger the (wave-shared) leaf tests
+// lanes waiting at a leaf that trigger the (wave-shared) leaf tests (1080p primary rays 731, 721, 718,
+// 729 us with 4, 8, 10, 16; 4M incoherent rays 1215, 1227, 1231, 1238 us)
+constexpr int kLeafMin = 4;
 // ... and fewer in a wave with few rays left, which would otherwise hold each leaf until its slowest ray
 __device__ __forceinline__ int leaf_min(int rays) { return min(kLeafMin, (5 * rays + 15) >> 4); }
 
@@ -71,6 +73,7 @@ __global__ __launch_bounds__(kCastBlock, 4) void k_cast(DevTree T, const float *
   bool exhausted = false;
   Walk w;
   w.state = kWalkIdle;          // the lane has no ray
+  w.leaf = kNoLeaf;
   CastCounters cnt_local = {0, 0, 0, 0, 0, 0};
   CastCounters *cc = kStats ? &cnt_local : nullptr;
   auto finish = [&]() {
@@ -194,7 +197,7 @@ __global__ __launch_bounds__(kCastBlock, 4) void k_cast(DevTree T, const float *
     // ---- castInLeaf for the pending leaves, the whole wave sharing their records
     const uint64_t pm = __ballot(w.state == kWalkLeaf);
     if (pm && (__popcll(pm) >= leaf_min(__popcll(__ballot(w.state != kWalkIdle))) || __ballot(w.state == kWalkTrace) == 0))
-      walk_leaf_wave<true>(T, w, w.state == kWalkLeaf, clip != 0, leaf, ins, cc);
+      walk_leaf_wave<true>(T, w, w.leaf != kNoLeaf, clip != 0, leaf, ins, cc);
   }
   // every ray of the wave has ended: the ranges still staged go out
   if (len0 > 0) flush(0, base0, len0);

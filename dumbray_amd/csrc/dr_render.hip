@@ -172,8 +172,10 @@ struct BenchPath {
   // render_block: finished casts that trigger the path updates, idle lanes that trigger new path
   // jobs.  k_render_stream: finished casts of a wave with all lanes busy that trigger the path
   // updates (in proportion with fewer lanes; 1080p 16 spp 16.4 / 15.9 / 15.8 ms at 16 / 24 / 32),
-  // idle lanes that pop the queue (1, 4, 10: 16.2, 15.9, 15.9 ms)
-  static constexpr int kShadeMin = 32, kRefillMin = 8, kStreamShadeMin = 32, kStreamRefillMin = 4;
+  // idle lanes that pop the queue (1, 4, 10: 16.2, 15.9, 15.9 ms), lanes that wait at a leaf for the
+  // leaf tests (8, 12, 16, 20: 13.50, 13.33, 13.29, 13.32 ms)
+  static constexpr int kShadeMin = 32, kRefillMin = 8, kStreamShadeMin = 32, kStreamRefillMin = 4,
+                       kStreamLeafMin = 16;
   Path st;
   __device__ __forceinline__ bool start(const dr_render_params &P, const FrameK &K, int block, int lp, int s,
                                         uint32_t samp0) {
@@ -232,8 +234,10 @@ struct BenchPath {
 // sample are computed again where they are used; both are functions of the vertex and
 // of counter-based random numbers, so the order of evaluation does not change them.
 struct RefPath {
-  // the same thresholds (reference plugins at 1080p, 1 spp: 3.23 / 3.12 / 3.26 ms at 32 / 44 / 52)
-  static constexpr int kShadeMin = 32, kRefillMin = 8, kStreamShadeMin = 44, kStreamRefillMin = 4;
+  // the same thresholds (reference plugins at 1080p, 1 spp: 3.23 / 3.12 / 3.26 ms at 32 / 44 / 52; leaf
+  // tests 2.78 / 2.76 / 2.75 / 2.84 ms at 4 / 6 / 8 / 16)
+  static constexpr int kShadeMin = 32, kRefillMin = 8, kStreamShadeMin = 44, kStreamRefillMin = 4,
+                       kStreamLeafMin = 8;
   uint32_t pix, samp;
   int layer, phase, light, lk, excl, trans;   // lk: photons of the current light still to send
   V3 o, d;                          // the next ray to cast
@@ -535,8 +539,8 @@ __device__ __forceinline__ void render_block(const DevTree &T, const Tables &tb,
       // ---- one traversal step of every ray in flight
       if (job >= 0 && w.state == kWalkTrace) walk_step(T, w, lds.stk, kRB, cc);
       // ---- leaf tests, batched
-      const bool pend = job >= 0 && w.state == kWalkLeaf;
-      const uint64_t pm = __ballot(pend);
+      const bool pend = job >= 0 && w.leaf != kNoLeaf;
+      const uint64_t pm = __ballot(pend && w.state == kWalkLeaf);
       if (pm && (__popcll(pm) >= kLeafMin || __ballot(job >= 0 && w.state == kWalkTrace) == 0))
         walk_leaf_wave(T, w, pend, clip, *lds.leaf, kStats ? lds.ins : nullptr, cc);
       // ---- path updates of the finished casts, batched
@@ -680,6 +684,7 @@ __device__ __forceinline__ void stream_paths(ConstArgs args,
   PathT ps;
   Walk w;                 // (kWalkIdle: the lane has no path)
   w.state = kWalkIdle;
+  w.leaf = kNoLeaf;
   int u = 0;              // stream pixel of this lane's path
   // the wave's queue (wave-uniform): entries [qpos, qlen) of the jobs from qbase on
   unsigned qbase = 0;
@@ -838,15 +843,18 @@ __device__ __forceinline__ void stream_paths(ConstArgs args,
     }
     if (fresh) {
       walk_begin(again(args).T, w, ps.ray_o(), ps.ray_d(), ps.ray_excl(), stk);
-      if (ps.pixel() == kNoPixel) w.state = kWalkDone;
+      if (ps.pixel() == kNoPixel) {
+        w.state = kWalkDone;
+        w.leaf = kNoLeaf;
+      }
     }
     // ---- one traversal step of every ray in flight
     if (w.state == kWalkTrace) walk_step(T, w, stk, kRB, cc);
     // ---- leaf tests, batched
     const uint64_t pm = __ballot(w.state == kWalkLeaf);
-    if (pm && (__popcll(pm) * (64 / kLeafMin) >= __popcll(__ballot(w.state != kWalkIdle)) ||
+    if (pm && (__popcll(pm) * 64 >= __popcll(__ballot(w.state != kWalkIdle)) * PathT::kStreamLeafMin ||
                __ballot(w.state == kWalkTrace) == 0))
-      walk_leaf_wave(T, w, w.state == kWalkLeaf, clip, leaf, ins, cc);
+      walk_leaf_wave(T, w, w.leaf != kNoLeaf, clip, leaf, ins, cc);
   }
 }
 
@@ -1014,6 +1022,7 @@ __global__ __launch_bounds__(kRB, kRenderWaves) void k_backward(DevTree T, const
   Path st;
   Walk w;
   w.state = kWalkIdle;            // the lane has no path
+  w.leaf = kNoLeaf;
   int K = 0;                      // vertices recorded for the current path
   bool fin = false;               // the current path has ended; its albedo terms are pending
   float wdl[3] = {0, 0, 0};       // spw * dL/dI (* lens filter) of the current pixel
@@ -1177,9 +1186,9 @@ __global__ __launch_bounds__(kRB, kRenderWaves) void k_backward(DevTree T, const
     if (fresh) walk_begin(T, w, st.o, st.d, st.restrict_tri, stk);
     if (w.state == kWalkTrace) walk_step(T, w, stk, kRB, nullptr);
     const uint64_t pm = __ballot(w.state == kWalkLeaf);
-    if (pm && (__popcll(pm) * (64 / kLeafMin) >= __popcll(__ballot(w.state != kWalkIdle)) ||
+    if (pm && (__popcll(pm) * 64 >= __popcll(__ballot(w.state != kWalkIdle)) * kLeafMin ||
                __ballot(w.state == kWalkTrace) == 0))
-      walk_leaf_wave(T, w, w.state == kWalkLeaf, clip, leaf, nullptr, nullptr);
+      walk_leaf_wave(T, w, w.leaf != kNoLeaf, clip, leaf, nullptr, nullptr);
   }
   __syncthreads();
   if (kSums != kSumsGlobal) flush(threadIdx.x, kRB);

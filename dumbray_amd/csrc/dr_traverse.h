@@ -139,12 +139,13 @@ __device__ __forceinline__ void group_entry(const float4 *__restrict__ G, int g,
 // without work.  With it in the state, a ballot over lanes to trace, to test, to finish or to refill is
 // one comparison; of two conditions it was three instructions, in five places of every iteration.
 enum : int { kWalkIdle = 0, kWalkTrace = 1, kWalkLeaf = 2, kWalkDone = 3 };
+constexpr int kNoLeaf = -2;
 struct Walk {
   V3 o, d;
   BoxRay box;
   int ex;              // validateNotSameAsObject's object, or -1
   int sp, state;
-  int leaf, llink, lcnt;   // pending leaf: its node (-1: the root), first leaf entry and entry count
+  int leaf, llink, lend;   // held leaf: its node (-1: the root, kNoLeaf: none held), first leaf entry and their end
   bool hit;            // result once state == kWalkDone
   Hit h;
 };
@@ -155,10 +156,11 @@ __device__ __forceinline__ void walk_begin(const DevTree &T, Walk &w, V3 o, V3 d
   w.ex = exclude;
   w.hit = false;
   w.sp = -1;
-  w.leaf = -1;
+  w.leaf = kNoLeaf;
   if (T.root_is_leaf) {
+    w.leaf = -1;
     w.llink = T.root_start;
-    w.lcnt = T.root_count;
+    w.lend = T.root_start + T.root_count;
     w.state = kWalkLeaf;
     return;
   }
@@ -170,22 +172,36 @@ __device__ __forceinline__ void walk_begin(const DevTree &T, Walk &w, V3 o, V3 d
   stk[0] = make_uint2(1u, 1u << w.box.canon);
 }
 
-// Pops one child: expands an interior child, or holds a leaf child as pending.
+// Pops one child: expands an interior child, or holds a leaf child until the wave's next leaf batch.
+// A lane that holds a leaf walks on: the children after it are expanded as if the leaf held no hit,
+// and the lane waits (kWalkLeaf) only at its next leaf, which stays on the stack, or at the walk's end.
+// Lanes waiting for a batch were idle in the expansions, most of the work; a batch's leaves are those of
+// the waiting and of the walking lanes.  The next child is popped in the same step: a lane that only took
+// its leaf sat out the expansion (that form: 1080p 16 spp 16.2 ms against 15.9 without walking on).
+// Measured, before -> after: 1080p 16 spp 14.00 -> 13.28 ms, 512x512 adjoint 6.10 -> 5.87 ms, 99,991
+// bounce rays 184 -> 174 us, 1080p primary rays 743 -> 731 us, batch of 24 5.78 -> 5.50 ms; 4M
+// incoherent rays, whose waves wait for memory, 1.218 -> 1.215 ms.
 __device__ __forceinline__ void walk_step(const DevTree &T, Walk &w, uint2 *stk, int stride, CastCounters *cc) {
-  const uint2 f = stk[w.sp * stride];
-  const int k = w.box.canon ^ __builtin_ctz(f.x);
-  const uint32_t rest = f.x & (f.x - 1);
-  stk[w.sp * stride].x = rest;
-  w.sp -= (rest & 0xffu) ? 0 : 1;
-  const uint32_t im = f.y & 0xffu;
-  if (!((im >> k) & 1u)) {
+  uint2 f = stk[w.sp * stride];
+  int k = w.box.canon ^ __builtin_ctz(f.x);
+  if (!((f.y >> k) & 1u) && w.leaf == kNoLeaf) {
     const int *E = (const int *)T.groups + kGroupWords * (size_t)(f.x >> 8) + kGroupEntry + k;
     w.leaf = (int)(f.x >> 8) * 8 + k;
     w.llink = E[0];
-    w.lcnt = E[1] - E[0];
-    w.state = kWalkLeaf;
-    return;
+    w.lend = E[1];
+    const uint32_t rest = f.x & (f.x - 1);
+    stk[w.sp * stride].x = rest;
+    w.sp -= (rest & 0xffu) ? 0 : 1;
+    // (a measurement launch counts the work of a walk that waits at every leaf)
+    if (cc || w.sp < 0) { w.state = kWalkLeaf; return; }
+    f = stk[w.sp * stride];
+    k = w.box.canon ^ __builtin_ctz(f.x);
   }
+  const uint32_t im = f.y & 0xffu;
+  if (!((im >> k) & 1u)) { w.state = kWalkLeaf; return; }
+  const uint32_t rest = f.x & (f.x - 1);
+  stk[w.sp * stride].x = rest;
+  w.sp -= (rest & 0xffu) ? 0 : 1;
   const int child = (int)(f.y >> 8) + __builtin_popcount(im & ((1u << k) - 1u));
   uint2 e;
   group_entry(T.groups, child, w.box, e.x, e.y, cc);
@@ -196,7 +212,7 @@ __device__ __forceinline__ void walk_step(const DevTree &T, Walk &w, uint2 *stk,
   // 1080p primary rays 785 -> 743 us, 512x512 adjoint 6.40 -> 6.10 ms).
   stk[(w.sp + 1) * stride] = e;
   w.sp += (e.x & 0xffu) ? 1 : 0;
-  w.state = w.sp < 0 ? kWalkDone : kWalkTrace;
+  if (w.sp < 0) w.state = w.leaf != kNoLeaf ? kWalkLeaf : kWalkDone;
 }
 
 // Inclusive prefix sum and maximum over the 64 lanes of the wave (every lane active): DPP row
@@ -264,7 +280,7 @@ template <bool kIndexed = false>
 __device__ __forceinline__ void walk_leaf_wave(const DevTree &T, Walk &w, bool pending, bool clip, LeafLds &lds,
                                                int *ins, CastCounters *cc) {
   const int lane = (int)__lane_id();
-  const int cnt = pending ? w.lcnt : 0;
+  const int cnt = pending ? w.lend - w.llink : 0;
   int total;
   const int incl = wave_incl_scan(cnt, total);
   const int start = incl - cnt;
@@ -350,6 +366,7 @@ __device__ __forceinline__ void walk_leaf_wave(const DevTree &T, Walk &w, bool p
     }
   }
   w.hit = hit;
+  w.leaf = kNoLeaf;
   w.state = (hit || w.sp < 0) ? kWalkDone : kWalkTrace;
 }
 
