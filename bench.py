@@ -37,11 +37,11 @@ OPS_RAY, OPS_BOX, OPS_TRI = 6, 24, 155
 # every leaf); a plane test reads the 4-B record index of the leaf entry and 32 B of the record,
 # an inside test 32 B more.
 # ops: 30 per ray (3 reciprocals, 3 slacks, the root's box) + 27 per group (grid planes and their
-#      near / far order) + 17 per box test (the children of an expanded group with a non-empty
-#      leaf below: 6 conversions, 6 fused products, 5 to combine) + 25 per plane test
+#      near / far order) + 16 per box test (the children of an expanded group with a non-empty
+#      leaf below: 6 conversions, 6 fused products, 4 to combine) + 25 per plane test
 #      + 140 per inside test (6 edge vectors, 3 dots, 3 square roots, 3 divisions).
 K_RAY, K_OUT, K_GROUP, K_POP, K_LEAF, K_PLANE, K_INSIDE = 24, 8, 80, 8, 32, 36, 32
-KOPS_RAY, KOPS_GROUP, KOPS_CHILD, KOPS_PLANE, KOPS_INSIDE = 30, 27, 17, 25, 140
+KOPS_RAY, KOPS_GROUP, KOPS_CHILD, KOPS_PLANE, KOPS_INSIDE = 30, 27, 16, 25, 140
 
 
 # host threads of the CPU legs: the cores this process may run on (the lease's share of the host)
