@@ -134,6 +134,12 @@ __global__ __launch_bounds__(kCastBlock, 4) void k_cast(DevTree T, const float *
   // bounce rays 186 -> 177 us, 4M incoherent rays 1.26 -> 1.24 ms).  Smaller ranges near the end of the
   // batch, to let the waves end together, cost more than they gave (1M rays 452 -> 499 us).
   bool look = true;
+  // Lanes that take rays: of a short range no more than it holds.  (With all lanes taking, the waves that
+  // start first found idle lanes and took the ranges of those still to start: 1,000 bounce rays 79 ->
+  // 69 us, 16,000 111 -> 99 us, 1,000 rays of a view 46.4 -> 42 us.)
+  const int width = min(chunk, 64);
+  const uint64_t wide = ~0ull >> (64 - width);
+  const unsigned refill_min = (unsigned)min(kRefillMin, max(1, (3 * width) >> 3));
   for (;;) {
     const bool done = w.state == kWalkDone;
     if (look || __ballot(done) != 0) {
@@ -141,12 +147,12 @@ __global__ __launch_bounds__(kCastBlock, 4) void k_cast(DevTree T, const float *
       retire(0, base0, len0);
       retire(1, base1, len1);
       // ---- refill idle lanes
-      const uint64_t wmask = __ballot(w.state == kWalkIdle);
+      const uint64_t wmask = __ballot(w.state == kWalkIdle) & wide;
       const unsigned need = (unsigned)__popcll(wmask);
       const unsigned rem = wend - wcur;
       look = false;
       if (rem > 0 || !exhausted) {
-        if (need >= kRefillMin || need == 64) {
+        if (need >= refill_min) {
           const unsigned idx = (unsigned)__popcll(wmask & below);
           int slot = idx < rem ? (int)(wcur + idx) : -1;
           if (rem >= need) {
@@ -176,13 +182,13 @@ __global__ __launch_bounds__(kCastBlock, 4) void k_cast(DevTree T, const float *
               cur = k;
             }
           }
-          if (w.state == kWalkIdle && slot >= 0) {
+          if (w.state == kWalkIdle && lane < width && slot >= 0) {
             r = slot;
             const float2 *R = (const float2 *)(rays + 6 * (size_t)r);
             const float2 q0 = R[0], q1 = R[1], q2 = R[2];
             walk_begin(T, w, v3(q0.x, q0.y, q1.x), v3(q1.y, q2.x, q2.y), exclude ? exclude[r] : -1, stk);
           }
-          look = __popcll(__ballot(w.state == kWalkIdle)) >= kRefillMin;
+          look = (unsigned)__popcll(__ballot(w.state == kWalkIdle) & wide) >= refill_min;
         }
       }
       if (__ballot(w.state != kWalkIdle) == 0) {
@@ -228,7 +234,8 @@ static int launch_cast(dr_scene s, const float *rays, int n, unsigned flags, con
   // Rays a wave takes at a time.  A batch that the chip can hold at once is bound by its longest ray:
   // it goes one ray a lane over as many waves as give every SIMD one, then over lanes (99,991 bounce
   // rays 246 us with 128 a wave, 228 us with 32, 191 us with 64; 4,096 rays 101 us with 128, 183 us
-  // with 1 on four waves a SIMD, 81 us with 4 on one; 64 rays 46 -> 24 us).  A larger one takes
+  // with 1 on four waves a SIMD, 81 us with 4 on one; 64 rays 46 -> 24 us; two or four waves a SIMD, with
+  // as many lanes of each as the range holds: 4,096 bounce rays 112 and 177 us).  A larger one takes
   // whole ranges, with two of them staged.
   int chunk = 1;
   while (chunk < 64 && (long long)chunk * s->num_cu * 4 < n) chunk *= 2;
