@@ -23,9 +23,9 @@ constexpr int kLeafMin = 4;
 __device__ __forceinline__ int leaf_min(int rays) { return min(kLeafMin, (5 * rays + 15) >> 4); }
 
 // One bounded step per loop iteration.  A lane that is traversing pops one child:
-// an interior child is expanded and pushed, a leaf child is held as pending.
-// Pending leaves are tested together once at least kLeafMin lanes hold one (or
-// no lane is still traversing), and idle lanes take new rays once kRefillMin of
+// an interior child is expanded and pushed, a leaf child is held and the walk goes on to
+// the next leaf.  Held leaves are tested together once at least kLeafMin lanes wait at
+// their next one (or no lane is still traversing), and idle lanes take new rays once kRefillMin of
 // them are idle (or no lane is busy), so the node expansions, which dominate the
 // work, run with most lanes of the wave active.
 //

@@ -383,7 +383,8 @@ int dr_png_read(const char *path, uint8_t *rgba, int width, int height);
  * device int32[n*6] receiving, per ray, the groups expanded (80 B read each), leaves
  * tested, triangle plane tests (32 B record reads), inside tests (a further 32 B each),
  * children of the expanded groups with a non-empty leaf below (box tests) and children
- * that the box test kept.  Same results as dr_cast. */
+ * that the box test kept.  Counting walks wait at every leaf (dr_cast's go on past one), so the
+ * counts do not depend on which rays share a wave.  Same results as dr_cast. */
 int dr_cast_stats(dr_scene s, const float *rays, int n, unsigned flags, const int32_t *exclude, int32_t *out_id,
                   float *out_t, int32_t *out_counts, void *stream);
 
@@ -392,7 +393,8 @@ int dr_cast_stats(dr_scene s, const float *rays, int n, unsigned flags, const in
  * it): casts (camera, bounce and photon rays), of which light photons, group expansions (80 B
  * read each), leaves tested, triangle plane tests and inside tests (32 B of a record each), path
  * jobs started, children of expanded groups with a non-empty leaf below (box tests) and
- * children that the box test kept.  Same frame as dr_render_blocks. */
+ * children that the box test kept, by walks that wait at every leaf (see dr_cast_stats).  Same
+ * frame as dr_render_blocks. */
 int dr_render_stats(dr_scene s, const dr_render_params *p, float *frame, int start_block, int end_block,
                     uint64_t *counts, void *stream);
 
