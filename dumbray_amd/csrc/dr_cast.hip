@@ -22,6 +22,8 @@ constexpr int kLeafMin = 4;
 // ... and fewer in a wave with few rays left, which would otherwise hold each leaf until its slowest ray
 __device__ __forceinline__ int leaf_min(int rays) { return min(kLeafMin, (5 * rays + 15) >> 4); }
 
+constexpr int kLongLeaf = 2048;       // records of a leaf from which small batches go out over more waves
+
 // One bounded step per loop iteration.  A lane that is traversing pops one child:
 // an interior child is expanded and pushed, a leaf child is held and the walk goes on to
 // the next leaf.  Held leaves are tested together once at least kLeafMin lanes wait at
@@ -237,8 +239,13 @@ static int launch_cast(dr_scene s, const float *rays, int n, unsigned flags, con
   // with 1 on four waves a SIMD, 81 us with 4 on one; 64 rays 46 -> 24 us; two or four waves a SIMD, with
   // as many lanes of each as the range holds: 4,096 bounce rays 112 and 177 us).  A larger one takes
   // whole ranges, with two of them staged.
+  // Where leaves hold thousands of records (the reference's build stops at some grids), a wave spends its
+  // time in their rounds, each a trip to memory that other waves of the SIMD hide: four waves a SIMD
+  // (524,288-triangle heightfield, leaves of up to 87,368 records: 4,096 rays 7.1 -> 3.0 ms,
+  // 40,000 rays 57 -> 22 ms).
+  const int waves = s->max_leaf >= kLongLeaf ? 16 : 4;
   int chunk = 1;
-  while (chunk < 64 && (long long)chunk * s->num_cu * 4 < n) chunk *= 2;
+  while (chunk < 64 && (long long)chunk * s->num_cu * waves < n) chunk *= 2;
   if ((long long)n > 2LL * 64 * kWavesPerBlock * s->num_cu * std::max(per_cu, 1)) chunk = kWaveChunk;
   // persistent grid: at most one block per resident slot, fewer for small batches
   const long long need = ((long long)n + kWavesPerBlock * chunk - 1) / (kWavesPerBlock * chunk);

@@ -572,6 +572,7 @@ int flatten_octree(const OctreeHost &t, OctreeFlat &out) {
       out.lref.push_back(urec_of[id]);
       count++;
     }
+    out.max_leaf = std::max(out.max_leaf, (int)count);
   };
   if (t.children[0] < 0) {
     out.root_is_leaf = 1;

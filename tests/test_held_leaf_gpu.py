@@ -10,7 +10,8 @@ from dumbray_amd import scenes as S
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("ntris,split,depth", [(1, 8, 24), (8, 8, 24), (9, 8, 6), (60, 1, 4), (2000, 1, 3), (2000, 2, 5)])
+@pytest.mark.parametrize("ntris,split,depth", [(1, 8, 24), (8, 8, 24), (9, 8, 6), (60, 1, 4), (2000, 1, 3), (2000, 2, 5),
+                                               (3000, 5000, 4), (20000, 1, 1)])    # leaves of thousands of records
 def test_batches_of_every_size(oracle, ntris, split, depth):
     import torch
 
