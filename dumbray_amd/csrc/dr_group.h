@@ -78,9 +78,11 @@ DR_HD bool box_ray(V3 o, V3 d, float reach, BoxRay &r) {
   const float ax = __builtin_fabsf(d.x), ay = __builtin_fabsf(d.y), az = __builtin_fabsf(d.z);
   const float dm = max3(ax, ay, az);
   const float om = max3(__builtin_fabsf(o.x), __builtin_fabsf(o.y), __builtin_fabsf(o.z));
-  // (a sum, unlike a maximum, keeps a NaN)
-  const bool able = ((ax + ay) + az) + ((__builtin_fabsf(o.x) + __builtin_fabsf(o.y)) + __builtin_fabsf(o.z)) < __builtin_inff() &&
-                    dm > 0.0f;
+  // (a sum, unlike a maximum, keeps a NaN; of eighths, so that six finite components stay below infinity)
+  const float sum = __builtin_fmaf(ax, 0.125f, __builtin_fmaf(ay, 0.125f, __builtin_fmaf(az, 0.125f,
+                    __builtin_fmaf(__builtin_fabsf(o.x), 0.125f, __builtin_fmaf(__builtin_fabsf(o.y), 0.125f,
+                                   __builtin_fabsf(o.z) * 0.125f)))));
+  const bool able = sum < __builtin_inff() && dm > 0.0f;
   int c = (d.z < 0) ? 1 : 0;
   if (d.y < 0) c += 2;
   if (d.x < 0) c += 4;
