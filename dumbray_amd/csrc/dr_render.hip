@@ -977,7 +977,7 @@ __global__ __launch_bounds__(kRB, kRenderWaves) void k_backward(DevTree T, const
                                                                  double *__restrict__ g_emission,
                                                                  float *__restrict__ vtx_all,
                                                                  int *__restrict__ next_unit, int nblocks, int chunk,
-                                                                 int unit_chunks, int levels, int maxv) {
+                                                                 uint32_t unit_chunks, int levels, int maxv) {
   extern __shared__ __align__(16) uint32_t lds[];
   __shared__ LeafLds leaf_all[kRB / 64];
   LeafLds &leaf = leaf_all[threadIdx.x >> 6];
@@ -1003,8 +1003,8 @@ __global__ __launch_bounds__(kRB, kRenderWaves) void k_backward(DevTree T, const
     if constexpr (kSums != kSumsGlobal) atomicAdd(&gacc[i], (Acc)v);
     else atomicAdd(i < 3 * P.nmat ? &g_albedo[i] : &g_emission[i - 3 * P.nmat], (double)v);
   };
-  // units of unit_chunks chunks, numbered block by block
-  const int nchunks = kBlockPixels * spp / chunk, parts = (nchunks + unit_chunks - 1) / unit_chunks;
+  // units of unit_chunks chunks, numbered block by block (a block has up to 2^38 jobs, in fewer than 2^32 chunks)
+  const uint32_t nchunks = (uint32_t)spp * (uint32_t)(kBlockPixels / chunk), parts = (nchunks - 1) / unit_chunks + 1;
   auto V_ = [&](int k, int w) -> float & { return vtx[((size_t)k * kVtxWords + w) * kRB + threadIdx.x]; };
   // sums t, t + step, ... into the FP64 gradients
   auto flush = [&](int t0, int step) {
@@ -1027,7 +1027,8 @@ __global__ __launch_bounds__(kRB, kRenderWaves) void k_backward(DevTree T, const
   bool fin = false;               // the current path has ended; its albedo terms are pending
   float wdl[3] = {0, 0, 0};       // spw * dL/dI (* lens filter) of the current pixel
   // the wave's queue (wave-uniform): entries [qpos, qlen); the unit's next chunks [cnext, cend) of block `block`
-  int qpos = 0, qlen = 0, block = 0, cnext = 0, cend = 0, jobs = 0;
+  int qpos = 0, qlen = 0, block = 0, jobs = 0;
+  uint32_t cnext = 0, cend = 0;
   bool ended = false;
   // the vertex's reflection factor and dA/dalbedo, then the next bounce (or the path's end)
   auto advance = [&]() {
@@ -1121,12 +1122,12 @@ __global__ __launch_bounds__(kRB, kRenderWaves) void k_backward(DevTree T, const
     // ---- the queue is empty: the next chunk of the unit, or the next unit
     if (qpos == qlen && !ended) {
       if (cnext == cend) {
-        int unit = 0;
-        if (lane == 0) unit = atomicAdd(next_unit, 1);
+        uint32_t unit = 0;
+        if (lane == 0) unit = (uint32_t)atomicAdd(next_unit, 1);
         unit = uni(unit);
-        block = unit / parts;
-        cnext = (unit - block * parts) * unit_chunks;
-        cend = min(cnext + unit_chunks, nchunks);
+        block = (int)(unit / parts);
+        cnext = (unit - (uint32_t)block * parts) * unit_chunks;
+        cend = cnext + min(unit_chunks, nchunks - cnext);
         ended = block >= nblocks;
         if (kSums == kSumsFp32 && !ended && jobs >= kFlushJobs) {
           flush(lane, 64);
@@ -1135,9 +1136,17 @@ __global__ __launch_bounds__(kRB, kRenderWaves) void k_backward(DevTree T, const
       }
       if (!ended) {
         if (lane < chunk) {
-          const int q = cnext * chunk + lane;
-          const int lp = (int)udiv((uint32_t)q, Dspp);
-          const PathStart ps = path_start(P, FK, block, lp, q - lp * spp, samp0);
+          int lp, s;
+          if (spp < (1 << 24)) {
+            const uint32_t q = cnext * (uint32_t)chunk + (uint32_t)lane;
+            lp = (int)udiv(q, Dspp);
+            s = (int)(q - (uint32_t)lp * (uint32_t)spp);
+          } else {                               // 128 pixels' jobs are 2^31 or more
+            const uint64_t q = (uint64_t)cnext * (uint32_t)chunk + (uint32_t)lane;
+            lp = (int)(q / (uint32_t)spp);
+            s = (int)(q - (uint64_t)lp * (uint32_t)spp);
+          }
+          const PathStart ps = path_start(P, FK, block, lp, s, samp0);
           const float *g = dl + 4 * ((size_t)kBlockPixels * block + lp);
           queue[0 * 64 + lane] = ps.d.x;
           queue[1 * 64 + lane] = ps.d.y;
@@ -1288,6 +1297,7 @@ static int check_params(dr_scene s, const dr_render_params *p) {
   const int max_mat = p->shading ? p->shading->max_mat : s->max_mat;
   if (p->width < 1 || p->height < 1 || p->fsaa_x < 1 || p->fsaa_y < 1 || p->max_bounces < 0 || p->max_bounces > 64)
     return fail(DR_ERR_ARG, "render: bad image size, subpixel grid or max_bounces");
+  if ((int64_t)p->fsaa_x * p->fsaa_y > INT32_MAX) return fail(DR_ERR_ARG, "render: more than 2^31 - 1 samples a pixel");
   if (p->nlights < 0 || p->nlights > kMaxLights || (p->nlights > 0 && !p->lights))
     return fail(DR_ERR_ARG, "render: 0 <= nlights <= 16 with a light table required");
   if (!p->materials || p->nmat <= max_mat) return fail(DR_ERR_ARG, "render: material table smaller than the ids in use");
@@ -1424,7 +1434,8 @@ struct BackwardShape {
   int sums;               // kSums* of k_backward
   int levels, maxv;
   size_t lds, slice;      // LDS bytes, and bytes of one workgroup's vertex records
-  int nblocks, groups, chunk, unit_chunks;
+  int nblocks, groups, chunk;
+  uint32_t unit_chunks;
 };
 // Workgroups of the persistent grid: one per resident slot, at most one per 256 paths, and at
 // most as many as `vtx_bytes` of vertex records hold.

@@ -187,7 +187,7 @@ enum {
  * DumbRenderer.cuh:80-101, plus the estimator's seeds). */
 typedef struct {
   int32_t width, height;          /* image size in pixels */
-  int32_t fsaa_x, fsaa_y;         /* subpixel grid = samples per pixel per iteration */
+  int32_t fsaa_x, fsaa_y;         /* subpixel grid = samples per pixel per iteration (at most 2^31 - 1) */
   int32_t max_bounces;            /* DumbRenderer maxBounces (<= 64, DumbRenderer.cuh:7) */
   int32_t rr_start;               /* Russian roulette at layers >= rr_start */
   float rr_survive;               /* survival probability (1 disables) */
