@@ -66,6 +66,17 @@ static int fill_shade(const dr_scene_s &s, const int32_t *mat_id, std::vector<fl
 }
 
 void scene_retain(dr_scene s) { s->refs.fetch_add(1); }
+
+unsigned *scene_work(dr_scene s, hipStream_t stream) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(stream, &status) != hipSuccess) {
+    (void)hipGetLastError();                 // (the null stream while another stream captures)
+    status = hipStreamCaptureStatusNone;
+  }
+  const int slot = status == hipStreamCaptureStatusActive ? s->work_slots.captured() : s->work_slots.eager();
+  return slot < 0 ? nullptr : (unsigned *)s->work.p + 2 * (size_t)slot;
+}
+
 void scene_release(dr_scene s) {
   if (s->refs.fetch_sub(1) != 1) return;
   dev_free(s->groups);

@@ -250,7 +250,8 @@ static int launch_cast(dr_scene s, const float *rays, int n, unsigned flags, con
   // persistent grid: at most one block per resident slot, fewer for small batches
   const long long need = ((long long)n + kWavesPerBlock * chunk - 1) / (kWavesPerBlock * chunk);
   const int blocks = (int)std::max(1LL, std::min<long long>(need, (long long)s->num_cu * std::max(per_cu, 1)));
-  unsigned *work = (unsigned *)s->work.p + 2 * (s->work_slot.fetch_add(1) % kWorkSlots);
+  unsigned *work = scene_work(s, (hipStream_t)stream);
+  if (!work) work = (unsigned *)s->work.p + 2 * s->work_slots.eager();   // (casts have no kernel without counters)
   if (stats)
     hipLaunchKernelGGL(k_cast<true>, dim3(blocks), dim3(kCastBlock), lds, (hipStream_t)stream, s->tree, rays, n, clip,
                        (const int *)exclude, (int *)out_id, out_t, out_point, (int *)stats, work, chunk);

@@ -8,10 +8,9 @@
 #include "../../include/dumbray.h"
 #include "dr_octree_build.h"
 #include "dr_traverse.h"
+#include "dr_work_slots.h"
 
 namespace dr {
-
-constexpr int kWorkSlots = 1024;         // cast work-counter pairs per scene
 
 void set_error(const std::string &msg);
 int fail(int code, const std::string &msg);
@@ -53,11 +52,10 @@ struct dr_scene_s {
   // from the unnormalized one per hit, its square root and division were 38 of a path update's 800
   // vector instructions.)
   std::vector<float4> shade_host;
-  // Work counters of the cast kernels: kWorkSlots pairs (next ray, waves done), zero
-  // between launches; each launch takes the next pair, so launches in flight at the
-  // same time (up to kWorkSlots of them) use distinct counters.
+  // Work counters of the cast and stream kernels: kWorkSlots pairs (next ray or tile, waves done),
+  // zero between launches, handed out by work_slots.
   dr::DevBuf work;
-  std::atomic<uint32_t> work_slot{0};
+  dr::WorkSlots work_slots;
   int num_cu = 1;
   // Adjoint vertex records, one buffer per stream that has run dr_backward on this scene
   // (grown when a call needs more; calls on one stream are ordered, so they share it).
@@ -83,6 +81,9 @@ void scene_retain(dr_scene s);
 void scene_release(dr_scene s);
 void shading_retain(dr_shading h);
 void shading_release(dr_shading h);
+// The work counters for a launch on `stream`; nullptr for one under graph capture when the pairs of
+// captured launches are used up.
+unsigned *scene_work(dr_scene s, hipStream_t stream);
 // The scene's vertex-record buffer for `stream`, at least `bytes` long.
 int scene_scratch(dr_scene s, hipStream_t stream, size_t bytes, void **out);
 // Device address of dr_backward_noalloc's scratch array on `device` (resolved once per device).

@@ -1382,10 +1382,11 @@ static int launch_render(dr_scene s, const dr_render_params *p, float *frame, in
   const Tables tb = tables_of(s, p);
   const bool ref = p->plugins == DR_PLUGINS_REFERENCE;
   const int spp = p->fsaa_x * p->fsaa_y;
-  // streamed tiles (k_render_stream) unless the sample count or the stream length is too large; one
-  // block per workgroup otherwise
+  // streamed tiles (k_render_stream) unless the sample count or the stream length is too large or no
+  // work counters are left for a captured launch; one block per workgroup otherwise
   const long long nrange = end_block - start_block;
-  if (streams(nrange, end_block, spp)) {
+  unsigned *work = nullptr;
+  if (streams(nrange, end_block, spp) && (work = scene_work(s, (hipStream_t)stream)) != nullptr) {
     const bool origins = p->lens == DR_SPHERICAL_SEGMENT_LENS;
     auto kern = counts ? (ref ? k_render_stream<RefPath, true> : k_render_stream<BenchPath, true>)
                        : (ref ? k_render_stream<RefPath, false> : k_render_stream<BenchPath, false>);
@@ -1395,7 +1396,6 @@ static int launch_render(dr_scene s, const dr_render_params *p, float *frame, in
     const long long resident = (long long)s->num_cu * std::max(per_cu, 1);
     const StreamShape S = stream_shape(nrange, spp, slot_shift, (double)resident);
     const long long groups = std::min<long long>(S.ntiles, resident);
-    unsigned *work = (unsigned *)s->work.p + 2 * (s->work_slot.fetch_add(1) % kWorkSlots);
     hipLaunchKernelGGL(kern, dim3((unsigned)groups), dim3(kRB), lds_s, (hipStream_t)stream,
                        RenderArgs{s->tree, tb, *p, frame_k(*p)}, frame, start_block, S, levels, work, counts);
     DR_HIP_CHECK(hipGetLastError());
