@@ -85,16 +85,22 @@ class BlockBasedFrameBuffer:
         """Row of `data` for every row-major pixel, made when an image is first converted: a frame
         that is only rendered into needs none, and its upload makes the host wait for the device.
         A first conversion under graph capture, where nothing can be uploaded, forms the rows in
-        the graph and keeps none."""
+        the graph and keeps none.  Kept rows serve later calls of any kind: they are no inference
+        tensor, whose use autograd refuses, and a stream that reads them is recorded, so that their
+        memory is not given to the stream of the first call while it does."""
         import torch
 
+        capturing = self.data.is_cuda and torch.cuda.is_current_stream_capturing()
         if self._rows is None:
-            if self.data.is_cuda and torch.cuda.is_current_stream_capturing():
+            if capturing:
                 y = torch.arange(self.height, device=self.data.device).unsqueeze(1)
                 x = torch.arange(self.width, device=self.data.device)
                 block = (y // BLOCK_H) * ((self.width + BLOCK_W - 1) // BLOCK_W) + x // BLOCK_W
                 return (block * BLOCK_SIZE + (y % BLOCK_H) * BLOCK_W + x % BLOCK_W).reshape(-1)
-            self._rows = torch.from_numpy(block_to_image_index(self.width, self.height)).to(self.data.device)
+            with torch.inference_mode(False):
+                self._rows = torch.from_numpy(block_to_image_index(self.width, self.height)).to(self.data.device)
+        if self._rows.is_cuda and not capturing:
+            self._rows.record_stream(torch.cuda.current_stream(self._rows.device))
         return self._rows
 
     def getBlockSize(self) -> int:
