@@ -22,6 +22,7 @@
 namespace dr {
 
 constexpr int kRB = 256;               // lanes per workgroup
+constexpr int kLdsBytes = 160 * 1024;  // LDS of a CU
 constexpr int kRoundSamples = 16;      // samples per pixel staged in LDS per round
 constexpr int kBlockPixels = 128;      // BlockBasedFrameBuffer<8,16>
 constexpr int kLeafMin = 16;           // pending leaves that trigger the (wave-shared) leaf tests
@@ -1323,6 +1324,17 @@ static Tables tables_of(dr_scene s, const dr_render_params *p) {
 }  // namespace dr
 
 namespace dr {
+// Allows launches of `kern` with `bytes` of dynamic LDS.  The limit belongs to the kernel, not to a launch:
+// it is always set to all that the kernel's own arrays leave, never to one caller's size, which a launch
+// from another thread, or a batch's launch for its largest request, could exceed.
+static int allow_lds(const void *kern, size_t bytes) {
+  if (bytes <= 64 * 1024) return DR_OK;
+  hipFuncAttributes a;
+  DR_HIP_CHECK(hipFuncGetAttributes(&a, kern));
+  DR_HIP_CHECK(hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes - (int)a.sharedSizeBytes));
+  return DR_OK;
+}
+
 // Pixel slots of a stream, and the workgroups per CU of kernel `kern` with them.  Deep trees, whose
 // stacks leave no room for all the slots beside the registers' three workgroups a CU, get half the
 // slots if that gives a workgroup more (1080p 16 spp: 15.8 ms with 2,048 samples staged and three,
@@ -1330,8 +1342,8 @@ namespace dr {
 static int stream_slots(const void *kern, int levels, int spp, bool origins, int &slot_shift, int &per_cu) {
   slot_shift = stream_slot_shift(spp, kStreamSamples);
   const size_t all = stream_lds(levels, spp, slot_shift, origins);
-  if (all > 64 * 1024)
-    DR_HIP_CHECK(hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)all));
+  const int rc = allow_lds(kern, all);
+  if (rc != DR_OK) return rc;
   DR_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, kRB, all));
   if (per_cu < kRenderWaves && slot_shift > 3) {
     int more = 0;
@@ -1404,8 +1416,7 @@ static int launch_render(dr_scene s, const dr_render_params *p, float *frame, in
   const size_t lds = ((size_t)levels * kStackWordsPerLevel * kRB + (size_t)kBlockPixels * kRoundSamples * 3) * 4;
   auto kernel = counts ? (ref ? k_render<RefPath, true> : k_render<BenchPath, true>)
                        : (ref ? k_render<RefPath, false> : k_render<BenchPath, false>);
-  if (lds > 64 * 1024)
-    DR_HIP_CHECK(hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  if ((rc = allow_lds((const void *)kernel, lds)) != DR_OK) return rc;
   hipLaunchKernelGGL(kernel, dim3(end_block - start_block), dim3(kRB), lds, (hipStream_t)stream, s->tree, tb, *p,
                      frame_k(*p), frame, start_block, levels, counts);
   DR_HIP_CHECK(hipGetLastError());
@@ -1452,7 +1463,8 @@ static int backward_shape(dr_scene s, const dr_render_params *p, size_t vtx_byte
   B.sums = fixed + 8 * ngrad <= 160 * 1024 / kRenderWaves ? kSumsFp64 : (fixed + 4 * ngrad <= 160 * 1024 ? kSumsFp32 : kSumsGlobal);
   B.lds = stacks + queues + (B.sums == kSumsFp64 ? 8 : (B.sums == kSumsFp32 ? 4 : 0)) * ngrad;
   const void *kern = (const void *)backward_kernel(B.sums);
-  if (B.lds > 64 * 1024) DR_HIP_CHECK(hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)B.lds));
+  const int rc = allow_lds(kern, B.lds);
+  if (rc != DR_OK) return rc;
   int per_cu = 0;
   DR_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, kRB, B.lds));
   const long long resident = (long long)s->num_cu * std::max(per_cu, 1);
@@ -1666,6 +1678,8 @@ static int launch_batch(dr_batch b, hipStream_t stream) {
   for (int set = 0; set < 2; set++) {
     const dr_batch_s::Items &it = b->items[set];
     if (it.n == 0) continue;
+    const int rc = allow_lds(set == 0 ? (const void *)k_batch<BenchPath> : (const void *)k_batch<RefPath>, batch_lds(b->levels));
+    if (rc != DR_OK) return rc;
     hipLaunchKernelGGL(set == 0 ? k_batch<BenchPath> : k_batch<RefPath>, grid, dim3(kRB), batch_lds(b->levels), stream, reqs,
                        (const int4 *)it.list.p, it.n, counters + ncounters - 2 + set, b->levels, b->tuning.refill_min);
   }
