@@ -901,13 +901,21 @@ __global__ __launch_bounds__(kRB, kRenderWaves) void k_render_stream(RenderArgs 
 // Reductions: the lanes of a wave that add to the same parameter in the same path
 // update are summed across the wave first (one LDS atomic per distinct material or
 // light and channel), and the workgroup's LDS sums go to the FP64 outputs with one global atomic
-// per parameter.  The LDS sums are FP64 and go out once, at the end; where FP64 sums would take
-// LDS from a workgroup per CU (about 900 materials) they are FP32 and every wave moves them out
-// after kFlushJobs of its jobs, and where LDS has no room for those (about 12,000) the terms go to
-// the outputs.
+// per parameter.  Three forms, by the materials and lights and by the stacks beside the sums:
+//   kSumsFp64   the LDS sums are FP64 and go out once, at the end.  Taken unless FP32 sums leave room for
+//               more workgroups a CU (10 levels: from 857 materials and lights on): 512x512 at
+//               16 spp 6.2 ms in FP64 with three a CU (600 materials), and 7.7 ms with two against 6.9 ms in
+//               FP32 with three (1,500), 13.8 ms with one against 8.6 ms with two (2,500).
+//   kSumsFp32   FP32 sums.  A wave moves all of them out whenever flush_paths(spp) of its paths have ended,
+//               so that what adds up in FP32 is the paths of one framebuffer block (128 spp), and no more
+//               than 2,048.
+//   kSumsTight  LDS holds the stacks and as many FP32 sums as fit (the lights' always): the queues lie
+//               beside the vertex records, and the few parameters left over (sizes a whisker below the
+//               limit) are added to the outputs.  (All terms added to the outputs, with FP64 atomics on
+//               few addresses: 80 ms against 15.6 ms, 12,620 materials.)
 constexpr int kVtxWords = 9;
-enum : int { kSumsGlobal, kSumsFp32, kSumsFp64 };
-constexpr int kFlushJobs = 2048;
+enum : int { kSumsTight, kSumsFp32, kSumsFp64 };
+__device__ __forceinline__ int flush_paths(int spp) { return min(spp, 16) * (kBlockPixels / (kRB / 64)); }
 constexpr int kAdjointQueueWords = 64 * 11;   // direction, pixel, sample, loss gradient, origin
 
 // Sum of v over the 64 lanes of the wave, returned to every lane: an inclusive scan within
@@ -978,17 +986,24 @@ __global__ __launch_bounds__(kRB, kRenderWaves) void k_backward(DevTree T, const
                                                                  double *__restrict__ g_emission,
                                                                  float *__restrict__ vtx_all,
                                                                  int *__restrict__ next_unit, int nblocks, int chunk,
-                                                                 uint32_t unit_chunks, int levels, int maxv) {
+                                                                 uint32_t unit_chunks, int levels, int maxv, int nlds) {
   extern __shared__ __align__(16) uint32_t lds[];
   __shared__ LeafLds leaf_all[kRB / 64];
   LeafLds &leaf = leaf_all[threadIdx.x >> 6];
   leaf_lds_init(leaf);
   uint2 *stk = (uint2 *)lds + threadIdx.x;
-  float *queue = (float *)(lds + levels * kStackWordsPerLevel * kRB) + (threadIdx.x >> 6) * kAdjointQueueWords;   // [word][entry]
+  // this workgroup's slice of the scratch buffer: vertex records (and kSumsTight's queues)
+  constexpr int kQueues = (kRB / 64) * kAdjointQueueWords;
+  float *vtx = vtx_all + (size_t)blockIdx.x * ((size_t)maxv * kVtxWords * kRB + (kSums == kSumsTight ? kQueues : 0));
+  uint32_t *beside = lds + levels * kStackWordsPerLevel * kRB;
+  float *queues;
+  if constexpr (kSums == kSumsTight) queues = vtx + (size_t)maxv * kVtxWords * kRB;
+  else queues = (float *)beside;
+  float *queue = queues + (threadIdx.x >> 6) * kAdjointQueueWords;   // [word][entry]
+  // sums of the last nlds parameters of nmat*3 albedo, then nlights*3 emission
   using Acc = std::conditional_t<kSums == kSumsFp64, double, float>;
-  Acc *gacc = (Acc *)(lds + levels * kStackWordsPerLevel * kRB + (kRB / 64) * kAdjointQueueWords);   // nmat*3 albedo, then nlights*3 emission
-  float *vtx = vtx_all + (size_t)blockIdx.x * maxv * kVtxWords * kRB;
-  const int ngrad = 3 * (P.nmat + P.nlights);
+  Acc *gacc = (Acc *)(kSums == kSumsTight ? beside : beside + kQueues);
+  const int first = 3 * (P.nmat + P.nlights) - nlds;
   const int spp = P.fsaa_x * P.fsaa_y;
   const uint32_t samp0 = (uint32_t)(P.iteration > 1 ? P.iteration - 1 : 0) * (uint32_t)spp;
   const float spw = uni(1.0f / (((float)P.fsaa_x) * ((float)P.fsaa_y)));
@@ -997,11 +1012,10 @@ __global__ __launch_bounds__(kRB, kRenderWaves) void k_backward(DevTree T, const
   const bool origins = P.lens == DR_SPHERICAL_SEGMENT_LENS;
   const int lane = (int)__lane_id();
   const uint64_t below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-  if (kSums != kSumsGlobal)
-    for (int t = threadIdx.x; t < ngrad; t += kRB) gacc[t] = (Acc)0;
+  for (int t = threadIdx.x; t < nlds; t += kRB) gacc[t] = (Acc)0;
   __syncthreads();
   auto add = [&](int i, float v) {
-    if constexpr (kSums != kSumsGlobal) atomicAdd(&gacc[i], (Acc)v);
+    if (kSums != kSumsTight || i >= first) atomicAdd(&gacc[kSums == kSumsTight ? i - first : i], (Acc)v);
     else atomicAdd(i < 3 * P.nmat ? &g_albedo[i] : &g_emission[i - 3 * P.nmat], (double)v);
   };
   // units of unit_chunks chunks, numbered block by block (a block has up to 2^38 jobs, in fewer than 2^32 chunks)
@@ -1009,13 +1023,14 @@ __global__ __launch_bounds__(kRB, kRenderWaves) void k_backward(DevTree T, const
   auto V_ = [&](int k, int w) -> float & { return vtx[((size_t)k * kVtxWords + w) * kRB + threadIdx.x]; };
   // sums t, t + step, ... into the FP64 gradients
   auto flush = [&](int t0, int step) {
-    for (int t = t0; t < ngrad; t += step) {
+    for (int t = t0; t < nlds; t += step) {
       Acc v;
-      if constexpr (kSums == kSumsFp32) v = atomicExch(&gacc[t], (Acc)0);
+      if constexpr (kSums != kSumsFp64) v = atomicExch(&gacc[t], (Acc)0);
       else v = gacc[t];
       if (v != (Acc)0) {
-        if (t < 3 * P.nmat) atomicAdd(&g_albedo[t], (double)v);
-        else atomicAdd(&g_emission[t - 3 * P.nmat], (double)v);
+        const int i = first + t;
+        if (i < 3 * P.nmat) atomicAdd(&g_albedo[i], (double)v);
+        else atomicAdd(&g_emission[i - 3 * P.nmat], (double)v);
       }
     }
   };
@@ -1028,7 +1043,8 @@ __global__ __launch_bounds__(kRB, kRenderWaves) void k_backward(DevTree T, const
   bool fin = false;               // the current path has ended; its albedo terms are pending
   float wdl[3] = {0, 0, 0};       // spw * dL/dI (* lens filter) of the current pixel
   // the wave's queue (wave-uniform): entries [qpos, qlen); the unit's next chunks [cnext, cend) of block `block`
-  int qpos = 0, qlen = 0, block = 0, jobs = 0;
+  int qpos = 0, qlen = 0, block = 0;
+  int paths = 0;                  // ended since the wave last moved the FP32 sums out
   uint32_t cnext = 0, cend = 0;
   bool ended = false;
   // the vertex's reflection factor and dA/dalbedo, then the next bounce (or the path's end)
@@ -1089,7 +1105,8 @@ __global__ __launch_bounds__(kRB, kRenderWaves) void k_backward(DevTree T, const
       // dL/demission of this update's lit photons
       wave_add3(add, lit, lkey, ev);
       // dL/dalbedo of the paths that ended: S_k backwards, then beta_k forwards
-      if (__ballot(fin)) {
+      const uint64_t fm = __ballot(fin);
+      if (fm) {
         if (fin) {
           float Ln[3] = {0, 0, 0};
           for (int k = K - 1; k >= 0; k--)
@@ -1118,6 +1135,10 @@ __global__ __launch_bounds__(kRB, kRenderWaves) void k_backward(DevTree T, const
           wave_add3(add, has, m, av);
         }
         if (fin) { w.state = kWalkIdle; fin = false; }
+        if (kSums != kSumsFp64 && (paths += __popcll(fm)) >= flush_paths(spp)) {
+          flush(lane, 64);
+          paths = 0;
+        }
       }
     }
     // ---- the queue is empty: the next chunk of the unit, or the next unit
@@ -1130,10 +1151,6 @@ __global__ __launch_bounds__(kRB, kRenderWaves) void k_backward(DevTree T, const
         cnext = (unit - (uint32_t)block * parts) * unit_chunks;
         cend = cnext + min(unit_chunks, nchunks - cnext);
         ended = block >= nblocks;
-        if (kSums == kSumsFp32 && !ended && jobs >= kFlushJobs) {
-          flush(lane, 64);
-          jobs = 0;
-        }
       }
       if (!ended) {
         if (lane < chunk) {
@@ -1166,7 +1183,6 @@ __global__ __launch_bounds__(kRB, kRenderWaves) void k_backward(DevTree T, const
         qpos = 0;
         qlen = chunk;
         cnext++;
-        jobs += chunk;
       }
     }
     // ---- idle lanes pop the next entries
@@ -1201,7 +1217,7 @@ __global__ __launch_bounds__(kRB, kRenderWaves) void k_backward(DevTree T, const
       walk_leaf_wave(T, w, w.leaf != kNoLeaf, clip, leaf, nullptr, nullptr);
   }
   __syncthreads();
-  if (kSums != kSumsGlobal) flush(threadIdx.x, kRB);
+  flush(threadIdx.x, kRB);
 }
 
 // ------------------------------------------------------------------ batched requests
@@ -1438,13 +1454,13 @@ extern "C" int dr_render_stats(dr_scene s, const dr_render_params *p, float *fra
 namespace dr {
 
 static decltype(&k_backward<kSumsFp64>) backward_kernel(int sums) {
-  return sums == kSumsFp64 ? k_backward<kSumsFp64> : (sums == kSumsFp32 ? k_backward<kSumsFp32> : k_backward<kSumsGlobal>);
+  return sums == kSumsFp64 ? k_backward<kSumsFp64> : (sums == kSumsFp32 ? k_backward<kSumsFp32> : k_backward<kSumsTight>);
 }
 // Launch shape of the adjoint.
 struct BackwardShape {
-  int sums;               // kSums* of k_backward
+  int sums, nlds;         // kSums* of k_backward, and the sums it holds in LDS
   int levels, maxv;
-  size_t lds, slice;      // LDS bytes, and bytes of one workgroup's vertex records
+  size_t lds, slice;      // LDS bytes, and bytes of one workgroup's slice of the scratch buffer
   int nblocks, groups, chunk;
   uint32_t unit_chunks;
 };
@@ -1457,11 +1473,18 @@ static int backward_shape(dr_scene s, const dr_render_params *p, size_t vtx_byte
   B.slice = (size_t)B.maxv * kVtxWords * kRB * sizeof(float);
   const size_t stacks = (size_t)B.levels * kStackWordsPerLevel * kRB * 4, queues = (kRB / 64) * (size_t)kAdjointQueueWords * 4;
   const size_t ngrad = 3 * (size_t)(p->nmat + p->nlights);
-  if (stacks + 4 * ngrad > 160 * 1024) return fail(DR_ERR_ARG, "dr_backward: too many materials and lights for LDS");
-  // (LeafLds of the four waves beside them)
-  const size_t fixed = stacks + queues + (kRB / 64) * sizeof(LeafLds);
-  B.sums = fixed + 8 * ngrad <= 160 * 1024 / kRenderWaves ? kSumsFp64 : (fixed + 4 * ngrad <= 160 * 1024 ? kSumsFp32 : kSumsGlobal);
-  B.lds = stacks + queues + (B.sums == kSumsFp64 ? 8 : (B.sums == kSumsFp32 ? 4 : 0)) * ngrad;
+  if (stacks + 4 * ngrad > kLdsBytes) return fail(DR_ERR_ARG, "dr_backward: too many materials and lights for LDS");
+  const size_t leaf = (kRB / 64) * sizeof(LeafLds), fixed = stacks + queues + leaf;
+  auto per_cu_with = [&](size_t sums) { return std::min<size_t>(kRenderWaves, kLdsBytes / (fixed + sums)); };
+  if (per_cu_with(8 * ngrad) > 0 && per_cu_with(8 * ngrad) >= per_cu_with(4 * ngrad)) B.sums = kSumsFp64;
+  else B.sums = per_cu_with(4 * ngrad) > 0 ? kSumsFp32 : kSumsTight;
+  B.nlds = (int)ngrad;
+  B.lds = stacks + queues + (B.sums == kSumsFp64 ? 8 : 4) * ngrad;
+  if (B.sums == kSumsTight) {
+    B.nlds = (int)std::min(ngrad, (kLdsBytes - stacks - leaf) / 4);
+    B.lds = stacks + 4 * (size_t)B.nlds;
+    B.slice += queues;
+  }
   const void *kern = (const void *)backward_kernel(B.sums);
   const int rc = allow_lds(kern, B.lds);
   if (rc != DR_OK) return rc;
@@ -1497,7 +1520,7 @@ static void launch_backward(dr_scene s, const dr_render_params *p, const float *
   float *vtx = (float *)((char *)scratch_mem + kCounterBytes);
   hipLaunchKernelGGL(k_zero, dim3(1), dim3(64), 0, stream, counter, 1);
   hipLaunchKernelGGL(backward_kernel(B.sums), dim3(B.groups), dim3(kRB), B.lds, stream, s->tree, tables_of(s, p).shade,
-                     *p, frame_k(*p), dl, ga, ge, vtx, counter, B.nblocks, B.chunk, B.unit_chunks, B.levels, B.maxv);
+                     *p, frame_k(*p), dl, ga, ge, vtx, counter, B.nblocks, B.chunk, B.unit_chunks, B.levels, B.maxv, B.nlds);
 }
 
 }  // namespace dr

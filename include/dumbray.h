@@ -258,8 +258,9 @@ int dr_render_blocks(dr_scene s, const dr_render_params *p, float *frame, int st
  * by path replay (each path is re-traced from its Philox key, nothing is stored
  * between passes).  dl_dframe: device, same block layout as `frame` (alpha ignored).
  * Adds dL/dalbedo (Lambert albedo and mirror reflectance; device double[nmat*3]) and
- * dL/demission (device double[nlights*3]); the caller zeroes them.  FP64
- * sums in LDS precede one FP64 atomic per workgroup and parameter.  The benchmark
+ * dL/demission (device double[nlights*3]); the caller zeroes them.  Sums in LDS
+ * precede the FP64 atomics: FP64 sums, or with large material tables FP32 sums
+ * over the paths of at most one framebuffer block.  The benchmark
  * plugin set only; every lens (the spherical segment lens's filter scales dL/dI). */
 int dr_backward(dr_scene s, const dr_render_params *p, const float *dl_dframe, double *g_albedo, double *g_emission,
                 void *stream);
