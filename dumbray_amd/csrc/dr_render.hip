@@ -736,6 +736,7 @@ __device__ __forceinline__ void stream_paths(ConstArgs args,
             __threadfence_block();
             const int left = atomicSub(&turn[slot], 1);
             if ((left & 511) == 1) {
+              __threadfence_block();   // the other samples' colours, staged before their lanes' subtractions
               float a[3] = {0.0f, 0.0f, 0.0f};
               for (int k = 0; k < spp; k++)
                 for (int j = 0; j < 3; j++) a[j] += src[3 * k + j] * spw;
