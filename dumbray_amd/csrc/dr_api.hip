@@ -226,7 +226,7 @@ int dr_scene_create(dr_octree t, dr_scene *out) {
   T.root_count = flat.root_count;
   T.reach = flat.reach;
   s->max_depth = flat.max_depth;
-  s->max_leaf = flat.max_leaf;
+  s->ray_records = flat.ray_records;
   s->ntris = (int)t->host.tris.size();
   s->shade_host.resize(s->ntris);
   s->faces_host.assign((size_t)s->ntris * dr::kFaceWords, 0.0f);   // texture coordinates start at 0

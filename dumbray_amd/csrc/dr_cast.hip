@@ -22,7 +22,7 @@ constexpr int kLeafMin = 4;
 // ... and fewer in a wave with few rays left, which would otherwise hold each leaf until its slowest ray
 __device__ __forceinline__ int leaf_min(int rays) { return min(kLeafMin, (5 * rays + 15) >> 4); }
 
-constexpr int kLongLeaf = 2048;       // records of a leaf from which small batches go out over more waves
+constexpr double kManyRecords = 2048; // records a ray meets from which small batches go out over more waves
 
 // One bounded step per loop iteration.  A lane that is traversing pops one child:
 // an interior child is expanded and pushed, a leaf child is held and the walk goes on to
@@ -239,11 +239,20 @@ static int launch_cast(dr_scene s, const float *rays, int n, unsigned flags, con
   // with 1 on four waves a SIMD, 81 us with 4 on one; 64 rays 46 -> 24 us; two or four waves a SIMD, with
   // as many lanes of each as the range holds: 4,096 bounce rays 112 and 177 us).  A larger one takes
   // whole ranges, with two of them staged.
-  // Where leaves hold thousands of records (the reference's build stops at some grids), a wave spends its
-  // time in their rounds, each a trip to memory that other waves of the SIMD hide: four waves a SIMD
-  // (524,288-triangle heightfield, leaves of up to 87,368 records: 4,096 rays 7.1 -> 3.0 ms,
-  // 40,000 rays 57 -> 22 ms).
-  const int waves = s->max_leaf >= kLongLeaf ? 16 : 4;
+  // Where a ray meets thousands of records (the reference's build stops at some grids), a wave spends its
+  // time in their rounds, each a trip to memory that other waves of the SIMD hide: four waves a SIMD.
+  // What counts is how many a ray can expect, not the longest leaf, which may be out of most rays' way.
+  // Rays over a sphere mesh with one leaf of many records, and over a heightfield of 524,288 triangles;
+  // one against four waves a SIMD:
+  //   records met, in the longest leaf     4,096 rays      16,384         65,536
+  //       8,    2,000                       68  /  166 us    66 /  182     101 /  208 us
+  //      24,    8,084                      139  /  227      208 /  323     316 /  427
+  //     147,   30,167                      639  /  739     1269 / 1383    1000 / 1123
+  //     267,    2,285                      152  /  252      227 /  333     377 /  405
+  //    2618,    9,237                      472  /  502      991 /  884    2407 / 1226
+  //   10228,   35,491                     2353  / 1941     3884 / 3069    9938 / 5589
+  //   63983,   87,368                     7366  / 2900    17736 / 9637   51498 / 26950
+  const int waves = s->ray_records >= kManyRecords ? 16 : 4;
   int chunk = 1;
   while (chunk < 64 && (long long)chunk * s->num_cu * waves < n) chunk *= 2;
   if ((long long)n > 2LL * 64 * kWavesPerBlock * s->num_cu * std::max(per_cu, 1)) chunk = kWaveChunk;

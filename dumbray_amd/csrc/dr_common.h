@@ -44,7 +44,7 @@ struct dr_scene_s {
   std::vector<float> faces_host;
   dr::DevTree tree;
   int max_depth = 0;                       // depth the octree reached: traversal stack levels
-  int max_leaf = 0;                        // most records of a leaf
+  double ray_records = 0.0;                // OctreeFlat::ray_records
   int ntris = 0;
   bool has_materials = false;
   int max_mat = -1;                        // largest material id in use

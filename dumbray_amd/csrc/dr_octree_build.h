@@ -64,7 +64,8 @@ struct OctreeFlat {
   int root_is_leaf = 0, root_start = 0, root_count = 0;
   int ngroups = 0, nrec = 0;
   int max_depth = 0;                       // depth of the deepest node (root: 0), not the build limit
-  int max_leaf = 0;                        // most records of a leaf
+  double ray_records = 0.0;                // records a random ray through the root box meets: the sum over
+                                           // leaves of their records times their box's share of its surface
   float reach = 0.0f;                      // largest magnitude of a box coordinate, inf if one is not finite
 };
 int flatten_octree(const OctreeHost &t, OctreeFlat &out);

@@ -557,6 +557,11 @@ int flatten_octree(const OctreeHost &t, OctreeFlat &out) {
     const Tri &tr = t.tris[id];
     return !(eq(tr.a, tr.b) || eq(tr.b, tr.c) || eq(tr.c, tr.a));    // degenerate never hits (Triangle.impl.h:292)
   };
+  auto surface = [&](int node) {
+    const Box &b = t.bounds[node];
+    const double x = (double)b.e.x - b.s.x, y = (double)b.e.y - b.s.y, z = (double)b.e.z - b.s.z;
+    return x * y + y * z + z * x;
+  };
   std::vector<int32_t> urec_of(t.tris.size(), -1);
   auto leaf_records = [&](int node, int32_t &start, int32_t &count) {
     start = (int32_t)(out.recs.size() / kRecWords);
@@ -572,7 +577,8 @@ int flatten_octree(const OctreeHost &t, OctreeFlat &out) {
       out.lref.push_back(urec_of[id]);
       count++;
     }
-    out.max_leaf = std::max(out.max_leaf, (int)count);
+    const double share = surface(node) / surface(0);
+    if (count > 0 && std::isfinite(share)) out.ray_records += share * count;
   };
   if (t.children[0] < 0) {
     out.root_is_leaf = 1;
