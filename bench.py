@@ -382,7 +382,7 @@ def bench_adjoint(D, S, stream, adam_steps):
 def bench_batch(D, S, stream):
     """64 renders in one persistent launch (hipGraph replay) over 8 seeded scenes of 3 displaced
     icospheres (levels 5-7: 61k-983k tris) + ground; resolution from {128^2..1024^2}, spp from
-    {1, 4, 16, 64}, depth from {2, 4, 8}; launch shape chosen by the library.  Compared with
+    {1, 4, 16, 64}, depth from {2, 4, 8}; launch shape chosen by the autotuner.  Compared with
     rendering the same requests one dr_render_blocks call at a time."""
     import torch
     specs, qs = S.batch_workload()

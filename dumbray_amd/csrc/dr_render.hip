@@ -15,6 +15,7 @@
 #include "dr_shade.h"
 
 #include <algorithm>
+#include <cmath>
 #include <new>
 #include <type_traits>
 #include <vector>
@@ -1604,6 +1605,7 @@ struct dr_batch_s {
     dr::DevBuf list;
   } items[2];
   std::vector<dr::DevRequest> host_reqs;
+  std::vector<char> streamed;        // per request: takes the streamed kernels
   std::vector<dr_scene> scenes;      // references held until dr_batch_destroy
   std::vector<dr_shading> shadings;
   hipStream_t cap_stream = nullptr;
@@ -1627,11 +1629,12 @@ static double pixel_cost(const dr_render_params &P) {
 
 // Queue of (request, first block, count) of the requests of plugin set `set` (0 =
 // benchmark, 1 = reference) that are not streamed, heaviest per-block cost first.
-static std::vector<int4> make_items(const std::vector<DevRequest> &R, int tile, int set) {
+static std::vector<int4> make_items(dr_batch b, int tile, int set) {
+  const std::vector<DevRequest> &R = b->host_reqs;
   std::vector<std::pair<double, int4>> v;
   for (int r = 0; r < (int)R.size(); r++) {
     const dr_render_params &P = R[r].A.P;
-    if ((P.plugins == DR_PLUGINS_REFERENCE) != (set == 1) || request_streams(P)) continue;
+    if ((P.plugins == DR_PLUGINS_REFERENCE) != (set == 1) || b->streamed[r]) continue;
     const int nb = block_count(&P);
     for (int b = 0; b < nb; b += tile)
       v.push_back({pixel_cost(P) * std::min(tile, nb - b), make_int4(r, b, std::min(tile, nb - b), 0)});
@@ -1653,7 +1656,7 @@ static int make_streams(dr_batch b, int set) {
   double total = 0.0;
   for (int r = 0; r < (int)b->host_reqs.size(); r++) {
     const dr_render_params &P = b->host_reqs[r].A.P;
-    if ((P.plugins == DR_PLUGINS_REFERENCE) != (set == 1) || !request_streams(P)) continue;
+    if ((P.plugins == DR_PLUGINS_REFERENCE) != (set == 1) || !b->streamed[r]) continue;
     ids.push_back(r);
     total += pixel_cost(P) * block_count(&P);
   }
@@ -1711,6 +1714,115 @@ static int launch_batch(dr_batch b, hipStream_t stream) {
   return DR_OK;
 }
 
+static void free_lists(dr_batch b) {
+  dev_free(b->reqs);
+  for (int set = 0; set < 2; set++) {
+    dev_free(b->items[set].list);
+    dev_free(b->streams[set].list);
+    dev_free(b->streams[set].first);
+  }
+  dev_free(b->counters);
+}
+
+// Uploads what a launch with b->tuning reads.
+static int upload_lists(dr_batch b) {
+  int rc = dev_upload(b->reqs, b->host_reqs.data(), b->host_reqs.size() * sizeof(DevRequest));
+  for (int set = 0; set < 2 && rc == DR_OK; set++) {
+    const std::vector<int4> items = make_items(b, b->tuning.tile_blocks, set);
+    b->items[set].n = (int)items.size();
+    rc = dev_upload(b->items[set].list, items.data(), items.size() * sizeof(int4));
+    if (rc == DR_OK) rc = make_streams(b, set);
+  }
+  const std::vector<int> zeros(b->streams[0].n + b->streams[1].n + 2, 0);
+  return rc == DR_OK ? dev_upload(b->counters, zeros.data(), zeros.size() * sizeof(int)) : rc;
+}
+
+// The shorter of two launches with the tuning t, in ms.
+static int time_tuning(dr_batch b, const dr_batch_tuning &t, hipStream_t stream, float &ms) {
+  b->tuning = t;
+  hipEvent_t e[3] = {nullptr, nullptr, nullptr};
+  int rc = upload_lists(b);
+  for (int k = 0; k < 3 && rc == DR_OK; k++)
+    if (hipEventCreate(&e[k]) != hipSuccess) rc = fail(DR_ERR_HIP, "dr_batch_create: event");
+  for (int k = 0; k < 3 && rc == DR_OK; k++) {
+    if (hipEventRecord(e[k], stream) != hipSuccess) rc = fail(DR_ERR_HIP, "dr_batch_create: event");
+    else if (k < 2) rc = launch_batch(b, stream);
+  }
+  if (hipStreamSynchronize(stream) != hipSuccess && rc == DR_OK) rc = fail(DR_ERR_HIP, "dr_batch_create: timing");
+  float a = 0.0f, c = 0.0f;
+  if (rc == DR_OK && (hipEventElapsedTime(&a, e[0], e[1]) != hipSuccess || hipEventElapsedTime(&c, e[1], e[2]) != hipSuccess))
+    rc = fail(DR_ERR_HIP, "dr_batch_create: timing");
+  ms = std::min(a, c);
+  for (hipEvent_t x : e)
+    if (x) (void)hipEventDestroy(x);
+  free_lists(b);
+  return rc;
+}
+
+// Chooses the launch shape of `b` by timed launches of a proxy: its requests into scratch frames, with fewer
+// samples a pixel (about kProxySamples in all, but one a pixel) where they have more.  From as many workgroups as the registers allow
+// and the streamed kernels' refill, one step at a time: workgroups a CU, idle lanes before a refill, and
+// the blocks of a queue item where there is a queue.  A change has to give kTuneGain on the proxy, which
+// cannot rank closer ones: 3 workgroups a CU are the best of 1, 2, 3, 4, 6 or within 2% of it on batches of
+// 24 requests (5.18 ms) to one 1024x1024 frame (0.48 ms), and 16 requests of 32 to 128 pixels take
+// 0.397 ms with 3, 0.378 ms with 2.
+constexpr double kProxySamples = 1e6, kTuneGain = 0.95;
+static int autotune(dr_batch b) {
+  dr_batch_s proxy;
+  proxy.num_cu = b->num_cu;
+  proxy.levels = b->levels;
+  proxy.host_reqs = b->host_reqs;
+  proxy.streamed = b->streamed;                 // each request in the kernel it takes uncut
+  double samples = 0.0;
+  for (const DevRequest &r : b->host_reqs) samples += (double)r.A.P.width * r.A.P.height * r.A.P.fsaa_x * r.A.P.fsaa_y;
+  const double cut = std::sqrt(std::min(1.0, kProxySamples / samples));
+  size_t bytes = 0;
+  for (DevRequest &r : proxy.host_reqs) {
+    dr_render_params &P = r.A.P;
+    P.fsaa_x = std::max(1, (int)(P.fsaa_x * cut));
+    P.fsaa_y = std::max(1, (int)(P.fsaa_y * cut));
+    P.iteration = 1;
+    r.A.K = frame_k(P);
+    bytes += (size_t)block_count(&P) * kBlockPixels * 16;
+  }
+  dr_batch_tuning best{1, kRenderWaves, BenchPath::kStreamRefillMin};
+  DevBuf frames;
+  if (hipMalloc(&frames.p, bytes) != hipSuccess) {   // no room to try others
+    (void)hipGetLastError();
+    b->tuning = best;
+    return DR_OK;
+  }
+  char *at = (char *)frames.p;
+  for (DevRequest &r : proxy.host_reqs) {
+    r.frame = (float *)at;
+    at += (size_t)block_count(&r.A.P) * kBlockPixels * 16;
+  }
+  // the proxy reads the requests' tables, which a stream of the caller may still be filling
+  if (hipDeviceSynchronize() != hipSuccess) {
+    dev_free(frames);
+    return fail(DR_ERR_HIP, "dr_batch_create: synchronize");
+  }
+  float best_ms = 0.0f;
+  int rc = time_tuning(&proxy, best, b->cap_stream, best_ms);
+  const struct { int32_t dr_batch_tuning::*field; int values[2]; } axes[] = {
+      {&dr_batch_tuning::groups_per_cu, {2, 4}}, {&dr_batch_tuning::refill_min, {1, 8}}, {&dr_batch_tuning::tile_blocks, {2, 4}}};
+  for (const auto &axis : axes) {
+    if (axis.field == &dr_batch_tuning::tile_blocks && std::count(b->streamed.begin(), b->streamed.end(), 0) == 0) continue;
+    const dr_batch_tuning base = best;
+    for (int v : axis.values) {
+      if (rc != DR_OK) break;
+      dr_batch_tuning t = base;
+      t.*axis.field = v;
+      float ms = 0.0f;
+      rc = time_tuning(&proxy, t, b->cap_stream, ms);
+      if (rc == DR_OK && ms < kTuneGain * best_ms) { best_ms = ms; best = t; }
+    }
+  }
+  dev_free(frames);
+  b->tuning = best;
+  return rc;
+}
+
 }  // namespace dr
 
 extern "C" int dr_batch_create(const dr_request *reqs, int n, const dr_batch_tuning *tuning, dr_batch *out) {
@@ -1733,6 +1845,7 @@ extern "C" int dr_batch_create(const dr_request *reqs, int n, const dr_batch_tun
     }
     d.frame = reqs[r].frame;
     b->host_reqs.push_back(d);
+    b->streamed.push_back(dr::request_streams(d.A.P));
     b->levels = std::max(b->levels, reqs[r].scene->max_depth);
   }
   if (rc == DR_OK) {
@@ -1742,22 +1855,12 @@ extern "C" int dr_batch_create(const dr_request *reqs, int n, const dr_batch_tun
     if (hipStreamCreate(&b->cap_stream) != hipSuccess) rc = dr::fail(DR_ERR_HIP, "dr_batch_create: stream");
   }
   if (rc == DR_OK) {
-    // by default as many workgroups as the registers allow and the streamed kernels' refill
-    b->tuning = tuning ? *tuning : dr_batch_tuning{1, dr::kRenderWaves, dr::BenchPath::kStreamRefillMin};
-    if (b->tuning.tile_blocks < 1 || b->tuning.groups_per_cu < 1 || b->tuning.refill_min < 1)
+    if (tuning) b->tuning = *tuning;
+    else rc = dr::autotune(b);
+    if (rc == DR_OK && (b->tuning.tile_blocks < 1 || b->tuning.groups_per_cu < 1 || b->tuning.refill_min < 1))
       rc = dr::fail(DR_ERR_ARG, "dr_batch_create: tuning values must be >= 1");
   }
-  if (rc == DR_OK) {
-    rc = dr::dev_upload(b->reqs, b->host_reqs.data(), b->host_reqs.size() * sizeof(dr::DevRequest));
-    for (int set = 0; set < 2 && rc == DR_OK; set++) {
-      const std::vector<int4> items = dr::make_items(b->host_reqs, b->tuning.tile_blocks, set);
-      b->items[set].n = (int)items.size();
-      rc = dr::dev_upload(b->items[set].list, items.data(), items.size() * sizeof(int4));
-      if (rc == DR_OK) rc = dr::make_streams(b, set);
-    }
-    const std::vector<int> zeros(b->streams[0].n + b->streams[1].n + 2, 0);
-    if (rc == DR_OK) rc = dr::dev_upload(b->counters, zeros.data(), zeros.size() * sizeof(int));
-  }
+  if (rc == DR_OK) rc = dr::upload_lists(b);
   if (rc == DR_OK) {
     hipError_t e = hipStreamBeginCapture(b->cap_stream, hipStreamCaptureModeThreadLocal);
     if (e == hipSuccess) {
@@ -1792,13 +1895,7 @@ extern "C" void dr_batch_destroy(dr_batch b) {
   if (b->exec) (void)hipGraphExecDestroy(b->exec);
   if (b->graph) (void)hipGraphDestroy(b->graph);
   if (b->cap_stream) (void)hipStreamDestroy(b->cap_stream);
-  dr::dev_free(b->reqs);
-  for (int set = 0; set < 2; set++) {
-    dr::dev_free(b->items[set].list);
-    dr::dev_free(b->streams[set].list);
-    dr::dev_free(b->streams[set].first);
-  }
-  dr::dev_free(b->counters);
+  dr::free_lists(b);
   for (dr_shading h : b->shadings) dr::shading_release(h);
   for (dr_scene sc : b->scenes) dr::scene_release(sc);
   delete b;

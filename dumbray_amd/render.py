@@ -368,8 +368,9 @@ class RenderBatch:
     """Many render requests in one persistent launch captured in a hipGraph (dr_batch_*).
 
     requests: list of (DumbRenderer, BlockBasedFrameBuffer, iteration, request_id).  The
-    renderers' parameters are read when the batch is created.  tuning: None takes the
-    library's own choice, else a dict with tile_blocks, groups_per_cu, refill_min."""
+    renderers' parameters are read when the batch is created.  tuning: None runs the
+    autotuner, else a dict with tile_blocks (blocks of a queue item; only requests of more than 256
+    samples a pixel are queued), groups_per_cu and refill_min."""
 
     def __init__(self, requests, tuning=None):
         self._keep = list(requests)

@@ -303,8 +303,9 @@ typedef struct dr_batch_s *dr_batch;
  * 355-379).  Persistent workgroups are spread over the requests by their cost; each runs one
  * request's tiles as a stream until they are gone and then joins the request with the most
  * work left (requests of more than 256 samples a pixel: a queue of blocks, longest first).
- * The launch (counter reset + kernels) is captured once in a hipGraph.  tuning == NULL takes
- * the library's own choice.
+ * The launch (counter reset + kernels) is captured once in a hipGraph.  tuning == NULL runs
+ * the autotuner (a few timed launches of a proxy of about 10^6 samples into scratch frames; request
+ * frames are not touched).
  * Requests of both plugin sets and every lens may be mixed: each plugin set has its own
  * persistent kernel, launched one after the other in the same graph.
  * Every request's frame equals what dr_render_blocks would produce for it. */

@@ -499,7 +499,7 @@ class RenderBatch {
     int iteration;
     uint32_t request;        // Philox counter word 3
   };
-  // tuning == nullptr takes the library's own choice
+  // tuning == nullptr runs the autotuner
   explicit RenderBatch(const std::vector<Request> &requests, const dr_batch_tuning *tuning = nullptr) {
     std::vector<dr_request> r(requests.size());
     for (size_t i = 0; i < requests.size(); i++) {

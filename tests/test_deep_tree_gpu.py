@@ -37,7 +37,8 @@ def test_batch_over_a_deep_tree(dev):
           for k, (spp, lens, l) in enumerate(shapes)]
     print(f"[case] batch of {len(rs)} requests over 18 levels", flush=True)
     frames = [D.BlockBasedFrameBuffer(9, 7) for _ in rs]
-    batch = D.RenderBatch([(r, f, 1, 0) for r, f in zip(rs, frames)])
+    batch = D.RenderBatch([(r, f, 1, 0) for r, f in zip(rs, frames)],
+                          dict(tile_blocks=1, groups_per_cu=3, refill_min=4))
     for _ in range(2):
         batch.run()
         torch.cuda.synchronize()

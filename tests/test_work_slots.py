@@ -9,7 +9,7 @@ import numpy as np
 import pytest
 
 HERE = os.path.dirname(os.path.abspath(__file__))
-CAPTURED = 1024                      # kCapturedSlots
+CAPTURED, EAGER = 1024, 16384        # kCapturedSlots, kEagerSlots
 
 
 def test_slots_of_captured_launches_are_their_own(tmp_path):
@@ -19,6 +19,27 @@ def test_slots_of_captured_launches_are_their_own(tmp_path):
     subprocess.run(["g++", "-std=c++17", "-O1", "-pthread", "-I" + os.path.join(HERE, "..", "dumbray_amd", "csrc"),
                     os.path.join(HERE, "cpp", "work_slots_probe.cpp"), "-o", exe], check=True)
     assert subprocess.run([exe], capture_output=True, text=True, timeout=60).stdout == "ok\n"
+
+
+@pytest.mark.gpu
+def test_eager_slots_are_used_again(dev):
+    """More eager casts than there are pairs in the ring: the last of them and a frame are the first's."""
+    import torch
+    import dumbray_amd as D
+    from dumbray_amd import scenes as S
+    sc = S.spheres_scene(4, seed=1)
+    tree = D.Octree(16, 12)
+    tree.push(sc.tris)
+    scene = tree.build().upload()
+    g = D.DumbRenderer(scene, sc.mat_id, sc.materials, sc.lights, sc.camera, 20, 18, (2, 2), 2)
+    rays = torch.from_numpy(S.primary_rays(sc.camera, 8, 8)).cuda()
+    frame, first = g.render().data, scene.cast(rays)["id"]
+    print(f"[case] {EAGER} eager casts", flush=True)
+    for k in range(EAGER + 8):
+        out = scene.cast(rays)
+        if k % 1024 == 0 or k >= EAGER - 8:
+            assert torch.equal(out["id"], first), k
+    assert torch.equal(g.render().data.view(torch.int32), frame.view(torch.int32))
 
 
 @pytest.mark.gpu
