@@ -13,8 +13,8 @@ namespace dr {
 constexpr int kCastBlock = 256;
 constexpr int kWavesPerBlock = kCastBlock / 64;
 constexpr int kWaveChunk = 128;       // most rays a wave takes from the global counter at a time
-// idle lanes that trigger a refill (incoherent batch: 12, 16, 20, 24, 28, 32 measured 2.16,
-// 2.11-2.12, 2.09, 2.07-2.08, 2.09, 2.11 ms)
+// idle lanes that trigger a refill (12, 16, 20, 24, 32: 4M incoherent rays 1225, 1222, 1217, 1217, 1217 us;
+// 1080p primary rays 736, 746, 751, 727, 728 us)
 constexpr int kRefillMin = 24;
 // lanes waiting at a leaf that trigger the (wave-shared) leaf tests (1080p primary rays 731, 721, 718,
 // 729 us with 4, 8, 10, 16; 4M incoherent rays 1215, 1227, 1231, 1238 us)

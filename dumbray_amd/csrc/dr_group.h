@@ -1,5 +1,7 @@
 // The conservative child-box test of the traversal, on the compact boxes of a child group
-// (dr_octree_build.h): which children a ray's walk may skip.  Host and device.
+// (dr_octree_build.h): which children a ray's walk may skip.  Host and device.  (Child boxes in the
+// cells of a grid per group are known from compressed wide BVHs, Ylitie, Karras and Laine 2017; the error
+// bound and the acceptance rule below are this tree's.)
 //
 // A leaf accepts a hit only at p = fl(o + fl(d * t)), t >= 0, inside its box, so a child may be
 // skipped if no real point o + d * t with t >= 0 lies within a rounding error of the boxes

@@ -29,8 +29,10 @@ constexpr int kBlockPixels = 128;      // BlockBasedFrameBuffer<8,16>
 constexpr int kLeafMin = 16;           // pending leaves that trigger the (wave-shared) leaf tests
 constexpr int kShadeMin = 32;          // finished casts of a busy wave that trigger the adjoint's path updates
 constexpr int kAdjointRefillMin = 4;   // idle lanes that pop the adjoint's queue
-// Waves per SIMD the render kernels are compiled for: the register cap this sets
-// (168 VGPRs) costs a few spills but beats 2 waves per SIMD clearly.
+// Waves per SIMD the render kernels are compiled for.  The register cap this sets (168 VGPRs) costs
+// k_render_stream<BenchPath> and k_backward no vector register, k_render_stream<RefPath> 12 B of scratch a
+// lane and k_batch_stream 12 and 28 B; 2 waves a SIMD were slower by a third (46.4 / 34.9 ms on an
+// earlier 1080p frame).
 constexpr int kRenderWaves = 3;
 
 // Per-lane path state.
@@ -940,8 +942,8 @@ __device__ __forceinline__ float wave_sum(float v) {
 
 // Lanes that must share a parameter before their terms are summed across the wave: a sum
 // costs six cross-lane steps per channel, a lane's own LDS atomic one contended add.
-// (1, 8, 24 and 65 measured 22.8 / 22.5 / 22.2 / 21.8 ms for the 512x512 16-spp adjoint of
-// 64 materials and 4 lights)
+// (512x512 16-spp adjoint of 64 materials and 4 lights: 6.21, 5.92, 5.87, 5.88 and 6.36 ms at 1, 8, 16,
+// 32 and 65, the last of which never sums)
 constexpr int kWaveSumMin = 16;
 
 // Adds v[0..2] of every lane with `has` to sum 3 * key + c (add(index, value)), one key at a time: the lanes
