@@ -918,6 +918,9 @@ __global__ __launch_bounds__(kRB, kRenderWaves) void k_render_stream(RenderArgs 
 //               limit) are added to the outputs.  (All terms added to the outputs, with FP64 atomics on
 //               few addresses: 80 ms against 15.6 ms, 12,620 materials.)
 constexpr int kVtxWords = 9;
+// Samples a pixel of one launch: the jobs of a block are counted in 31 bits.  A call with more takes several
+// launches.
+constexpr int kLaunchSamples = 1 << 23;
 enum : int { kSumsTight, kSumsFp32, kSumsFp64 };
 __device__ __forceinline__ int flush_paths(int spp) { return min(spp, 16) * (kBlockPixels / (kRB / 64)); }
 constexpr int kAdjointQueueWords = 64 * 11;   // direction, pixel, sample, loss gradient, origin
@@ -990,7 +993,8 @@ __global__ __launch_bounds__(kRB, kRenderWaves) void k_backward(DevTree T, const
                                                                  double *__restrict__ g_emission,
                                                                  float *__restrict__ vtx_all,
                                                                  int *__restrict__ next_unit, int nblocks, int chunk,
-                                                                 uint32_t unit_chunks, int levels, int maxv, int nlds) {
+                                                                 int unit_chunks, int levels, int maxv, int tight,
+                                                                 int s0) {
   extern __shared__ __align__(16) uint32_t lds[];
   __shared__ LeafLds leaf_all[kRB / 64];
   LeafLds &leaf = leaf_all[threadIdx.x >> 6];
@@ -1004,14 +1008,16 @@ __global__ __launch_bounds__(kRB, kRenderWaves) void k_backward(DevTree T, const
   if constexpr (kSums == kSumsTight) queues = vtx + (size_t)maxv * kVtxWords * kRB;
   else queues = (float *)beside;
   float *queue = queues + (threadIdx.x >> 6) * kAdjointQueueWords;   // [word][entry]
-  // sums of the last nlds parameters of nmat*3 albedo, then nlights*3 emission
+  // sums of nmat*3 albedo, then nlights*3 emission
   using Acc = std::conditional_t<kSums == kSumsFp64, double, float>;
   Acc *gacc = (Acc *)(kSums == kSumsTight ? beside : beside + kQueues);
-  const int first = 3 * (P.nmat + P.nlights) - nlds;
+  // (kSumsTight: of the last `tight` of them)
+  const int ngrad = 3 * (P.nmat + P.nlights), nlds = kSums == kSumsTight ? tight : ngrad, first = ngrad - nlds;
   const int spp = P.fsaa_x * P.fsaa_y;
   const uint32_t samp0 = (uint32_t)(P.iteration > 1 ? P.iteration - 1 : 0) * (uint32_t)spp;
   const float spw = uni(1.0f / (((float)P.fsaa_x) * ((float)P.fsaa_y)));
-  const UDiv Dspp = udiv_uniform((uint32_t)spp);
+  const int ns = min(spp - s0, kLaunchSamples);   // this launch's samples of a pixel, from s0 on
+  const UDiv Dns = udiv_uniform((uint32_t)ns);
   const bool clip = P.cull_backfaces != 0;
   const bool origins = P.lens == DR_SPHERICAL_SEGMENT_LENS;
   const int lane = (int)__lane_id();
@@ -1022,8 +1028,8 @@ __global__ __launch_bounds__(kRB, kRenderWaves) void k_backward(DevTree T, const
     if (kSums != kSumsTight || i >= first) atomicAdd(&gacc[kSums == kSumsTight ? i - first : i], (Acc)v);
     else atomicAdd(i < 3 * P.nmat ? &g_albedo[i] : &g_emission[i - 3 * P.nmat], (double)v);
   };
-  // units of unit_chunks chunks, numbered block by block (a block has up to 2^38 jobs, in fewer than 2^32 chunks)
-  const uint32_t nchunks = (uint32_t)spp * (uint32_t)(kBlockPixels / chunk), parts = (nchunks - 1) / unit_chunks + 1;
+  // units of unit_chunks chunks, numbered block by block
+  const int nchunks = kBlockPixels * ns / chunk, parts = (nchunks + unit_chunks - 1) / unit_chunks;
   auto V_ = [&](int k, int w) -> float & { return vtx[((size_t)k * kVtxWords + w) * kRB + threadIdx.x]; };
   // sums t, t + step, ... into the FP64 gradients
   auto flush = [&](int t0, int step) {
@@ -1047,9 +1053,8 @@ __global__ __launch_bounds__(kRB, kRenderWaves) void k_backward(DevTree T, const
   bool fin = false;               // the current path has ended; its albedo terms are pending
   float wdl[3] = {0, 0, 0};       // spw * dL/dI (* lens filter) of the current pixel
   // the wave's queue (wave-uniform): entries [qpos, qlen); the unit's next chunks [cnext, cend) of block `block`
-  int qpos = 0, qlen = 0, block = 0;
+  int qpos = 0, qlen = 0, block = 0, cnext = 0, cend = 0;
   int paths = 0;                  // ended since the wave last moved the FP32 sums out
-  uint32_t cnext = 0, cend = 0;
   bool ended = false;
   // the vertex's reflection factor and dA/dalbedo, then the next bounce (or the path's end)
   auto advance = [&]() {
@@ -1139,7 +1144,7 @@ __global__ __launch_bounds__(kRB, kRenderWaves) void k_backward(DevTree T, const
           wave_add3(add, has, m, av);
         }
         if (fin) { w.state = kWalkIdle; fin = false; }
-        if (kSums != kSumsFp64 && (paths += __popcll(fm)) >= flush_paths(spp)) {
+        if (kSums != kSumsFp64 && (paths += __popcll(fm)) >= flush_paths(ns)) {
           flush(lane, 64);
           paths = 0;
         }
@@ -1148,27 +1153,19 @@ __global__ __launch_bounds__(kRB, kRenderWaves) void k_backward(DevTree T, const
     // ---- the queue is empty: the next chunk of the unit, or the next unit
     if (qpos == qlen && !ended) {
       if (cnext == cend) {
-        uint32_t unit = 0;
-        if (lane == 0) unit = (uint32_t)atomicAdd(next_unit, 1);
+        int unit = 0;
+        if (lane == 0) unit = atomicAdd(next_unit, 1);
         unit = uni(unit);
-        block = (int)(unit / parts);
-        cnext = (unit - (uint32_t)block * parts) * unit_chunks;
-        cend = cnext + min(unit_chunks, nchunks - cnext);
+        block = unit / parts;
+        cnext = (unit - block * parts) * unit_chunks;
+        cend = min(cnext + unit_chunks, nchunks);
         ended = block >= nblocks;
       }
       if (!ended) {
         if (lane < chunk) {
-          int lp, s;
-          if (spp < (1 << 24)) {
-            const uint32_t q = cnext * (uint32_t)chunk + (uint32_t)lane;
-            lp = (int)udiv(q, Dspp);
-            s = (int)(q - (uint32_t)lp * (uint32_t)spp);
-          } else {                               // 128 pixels' jobs are 2^31 or more
-            const uint64_t q = (uint64_t)cnext * (uint32_t)chunk + (uint32_t)lane;
-            lp = (int)(q / (uint32_t)spp);
-            s = (int)(q - (uint64_t)lp * (uint32_t)spp);
-          }
-          const PathStart ps = path_start(P, FK, block, lp, s, samp0);
+          const int q = cnext * chunk + lane;
+          const int lp = (int)udiv((uint32_t)q, Dns);
+          const PathStart ps = path_start(P, FK, block, lp, s0 + (q - lp * ns), samp0);
           const float *g = dl + 4 * ((size_t)kBlockPixels * block + lp);
           queue[0 * 64 + lane] = ps.d.x;
           queue[1 * 64 + lane] = ps.d.y;
@@ -1465,8 +1462,7 @@ struct BackwardShape {
   int sums, nlds;         // kSums* of k_backward, and the sums it holds in LDS
   int levels, maxv;
   size_t lds, slice;      // LDS bytes, and bytes of one workgroup's slice of the scratch buffer
-  int nblocks, groups, chunk;
-  uint32_t unit_chunks;
+  int nblocks, groups, chunk, unit_chunks;
 };
 // Workgroups of the persistent grid: one per resident slot, at most one per 256 paths, and at
 // most as many as `vtx_bytes` of vertex records hold.
@@ -1495,7 +1491,7 @@ static int backward_shape(dr_scene s, const dr_render_params *p, size_t vtx_byte
   int per_cu = 0;
   DR_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, kRB, B.lds));
   const long long resident = (long long)s->num_cu * std::max(per_cu, 1);
-  const long long jobs = (long long)B.nblocks * kBlockPixels * p->fsaa_x * p->fsaa_y;
+  const long long jobs = (long long)B.nblocks * kBlockPixels * std::min(kLaunchSamples, p->fsaa_x * p->fsaa_y);
   B.groups = (int)std::min<long long>({(jobs + kRB - 1) / kRB, resident, (long long)(vtx_bytes / B.slice)});
   // jobs a wave takes at a time: 1/32 of its share, between 8 and 64
   const long long per_wave = jobs / ((long long)std::max(B.groups, 1) * (kRB / 64));
@@ -1522,9 +1518,13 @@ static void launch_backward(dr_scene s, const dr_render_params *p, const float *
                             void *scratch_mem, const BackwardShape &B, hipStream_t stream) {
   int *counter = (int *)scratch_mem;
   float *vtx = (float *)((char *)scratch_mem + kCounterBytes);
-  hipLaunchKernelGGL(k_zero, dim3(1), dim3(64), 0, stream, counter, 1);
-  hipLaunchKernelGGL(backward_kernel(B.sums), dim3(B.groups), dim3(kRB), B.lds, stream, s->tree, tables_of(s, p).shade,
-                     *p, frame_k(*p), dl, ga, ge, vtx, counter, B.nblocks, B.chunk, B.unit_chunks, B.levels, B.maxv, B.nlds);
+  const int spp = p->fsaa_x * p->fsaa_y;
+  for (int s0 = 0; s0 < spp; s0 += std::min(spp - s0, kLaunchSamples)) {
+    hipLaunchKernelGGL(k_zero, dim3(1), dim3(64), 0, stream, counter, 1);
+    hipLaunchKernelGGL(backward_kernel(B.sums), dim3(B.groups), dim3(kRB), B.lds, stream, s->tree, tables_of(s, p).shade,
+                       *p, frame_k(*p), dl, ga, ge, vtx, counter, B.nblocks, B.chunk, B.unit_chunks, B.levels, B.maxv,
+                       B.nlds, s0);
+  }
 }
 
 }  // namespace dr
