@@ -16,20 +16,22 @@ def _renderer(spp, size=(3, 2)):
 
 
 def test_adjoint_of_two_to_the_24_samples(dev):
-    """The gradients of 4096 x 4096 samples a pixel against those of 4095 x 4097, one sample fewer:
-    two estimates from 10^8 paths, a few 1e-4 apart at most; a lost part of the jobs would show whole."""
+    """The gradients of 4095 x 4097 and 4096 x 4096 samples a pixel, one sample more, against those of
+    2896 x 2896, the last square that one launch takes: estimates from 5 * 10^7 and 10^8 paths, a few 1e-4
+    apart at most; a lost part of the jobs would show whole."""
     import torch
     grads = []
-    for spp in ((4095, 4097), (4096, 4096)):
+    for spp in ((2896, 2896), (4095, 4097), (4096, 4096)):
         g = _renderer(spp)
         print(f"[case] adjoint of 3x2 pixels at {spp} samples", flush=True)
         dl = torch.rand((128, 4), generator=torch.Generator(device="cuda").manual_seed(3), device="cuda")
         ga, ge = g.backward(dl)
         torch.cuda.synchronize()
         grads.append((ga.cpu().numpy(), ge.cpu().numpy()))
-    for a, b in zip(*grads):
-        assert np.abs(a).max() > 0
-        assert np.abs(a - b).max() <= 0.01 * np.abs(a).max()
+    for other in grads[1:]:
+        for a, b in zip(grads[0], other):
+            assert np.abs(a).max() > 0
+            assert np.abs(a - b).max() <= 0.01 * np.abs(a).max()
 
 
 def test_sample_counts_beyond_31_bits_are_refused(dev):
